@@ -145,6 +145,21 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
   rp.dc_sq_max = sq_max(p->dc);
   rp.dm_sq_max = sq_max(p->dm);
   rp.seed_sq_max = sq_max(p->seed_dc);
+  // The flat kernel's test v <= t as clamp((t+ - v) * 2^k): 2^k t+ in [2^60, 2^61)
+  // (double: 2^120), so the unit in the last place of t+ is far above one and the
+  // products of values within the radius are finite.
+  {
+    const bool root = p->metric != CLUE_METRIC_MANHATTAN && p->metric != CLUE_METRIC_CHEBYSHEV &&
+                      p->metric != CLUE_METRIC_WEIGHTED_CHEBYSHEV;
+    const T next = std::nextafter(root ? rp.dc_sq_max : rp.dc, std::numeric_limits<T>::infinity());
+    const int top = sizeof(T) == 4 ? 61 : 121;
+    int ex = 0;
+    std::frexp(next, &ex);
+    if (std::isfinite(next) && ex >= -top && ex <= 2 * top - 2) {
+      rp.in_scale = std::ldexp(T(1), top - ex);
+      rp.in_limit = std::ldexp(next, top - ex);
+    }
+  }
   rp.kp0 = p->kparam[0];
   rp.kp1 = p->kparam[1];
   // 2 * sigma * sigma, evaluated left to right (ConvolutionalKernel.hpp:40).
@@ -165,12 +180,13 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
   }
   // Within the radius the kernel's exp argument is -lambda*d (exp) or -d*d/(2s^2)
   // (gauss), with 0 <= d <= dc; bound its magnitude with a 1% margin for rounding.
+  // Within 86 every value is a normal float, which the in-range exp relies on.
   {
     const double dc = p->dc;
     double mag = 0.0;
     if (p->kernel == CLUE_KERNEL_EXP) mag = static_cast<double>(p->kparam[0]) * dc;
     if (p->kernel == CLUE_KERNEL_GAUSS) mag = dc * dc / static_cast<double>(rp.gauss_den);
-    rp.exp_in_range = (std::isfinite(mag) && mag * 1.01 < 100.0) ? 1 : 0;
+    rp.exp_in_range = (std::isfinite(mag) && mag * 1.01 < 86.0) ? 1 : 0;
   }
   for (int d = 0; d < kMaxDim; ++d) {
     rp.wrapped[d] = d < p->ndim ? (p->wrapped[d] ? 1 : 0) : 0;
@@ -181,6 +197,17 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
     bool unit = true;
     for (int d = 0; d < p->ndim; ++d) unit = unit && p->mparam[d] == 1;
     if (unit) rp.metric = CLUE_METRIC_EUCLIDEAN;
+  }
+  // Periodic Euclidean: a period of zero makes min(a, 0 - a) = -a, whose square is
+  // a * a, the plain term. Dimensions before the last without a period (x, y beside
+  // phi) then take the plain term's two instructions instead of four.
+  if (rp.metric == CLUE_METRIC_PERIODIC_EUCLIDEAN) {
+    bool plain = true;
+    for (int d = 0; d + 1 < p->ndim; ++d) plain = plain && p->mparam[d] == 0;
+    if (plain && p->mparam[p->ndim - 1] == 0)
+      rp.metric = CLUE_METRIC_EUCLIDEAN;
+    else if (plain && p->ndim >= 2)
+      rp.metric = kMetricPeriodicLast;
   }
   return rp;
 }

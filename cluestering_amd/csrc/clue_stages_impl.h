@@ -42,7 +42,7 @@ constexpr int kWaves = kBlock / kWave;
 constexpr int kMaxNeighbourBlock = 1024;
 
 enum { M_EUCLID = 0, M_WEUCLID = 1, M_PERIODIC = 2, M_MANHATTAN = 3, M_CHEBYSHEV = 4,
-       M_WCHEBYSHEV = 5, M_MAHALANOBIS = 6 };
+       M_WCHEBYSHEV = 5, M_MAHALANOBIS = 6, M_PERIODIC_LAST = kMetricPeriodicLast };
 enum { K_FLAT = 0, K_EXP = 1, K_GAUSS = 2 };
 
 // Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
@@ -100,7 +100,8 @@ struct MetricTraits {
   // Metrics ending in a square root are compared through the squared sum against
   // the largest float whose correctly rounded square root is within the radius.
   static constexpr bool kSqrt =
-      (M == M_EUCLID || M == M_WEUCLID || M == M_PERIODIC || M == M_MAHALANOBIS);
+      (M == M_EUCLID || M == M_WEUCLID || M == M_PERIODIC || M == M_PERIODIC_LAST ||
+       M == M_MAHALANOBIS);
 };
 
 // ---------------------------------------------------------------------------
@@ -555,6 +556,11 @@ static __global__ __launch_bounds__(kBlock) void k_items_one_block(
   }
 }
 
+__device__ __forceinline__ float fmin_t(float a, float b) { return __builtin_fminf(a, b); }
+__device__ __forceinline__ double fmin_t(double a, double b) { return __builtin_fmin(a, b); }
+__device__ __forceinline__ float fmax_t(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ __forceinline__ double fmax_t(double a, double b) { return __builtin_fmax(a, b); }
+
 // ---------------------------------------------------------------------------
 // Distances (DistanceMetrics.hpp), right fold over dimensions
 // (internal/meta/accumulate.hpp): t0 + (t1 + (... + (t_{D-1} + 0))).
@@ -579,13 +585,17 @@ __device__ __forceinline__ T metric_pair(const T (&xi)[D], const T (&si)[D], con
       s = rp.mparam[d] * dx * dx + s;
     }
     return s;
-  } else if constexpr (M == M_PERIODIC) {
+  } else if constexpr (M == M_PERIODIC || M == M_PERIODIC_LAST) {
     T s;
 #pragma unroll
     for (int d = D - 1; d >= 0; --d) {
-      const T a = __builtin_fabs(xi[d] - xj[d]);
-      const T pa = rp.mparam[d] - a;
-      const T m = (pa < a) ? pa : a;  // std::min(a, P - a)
+      T m = xi[d] - xj[d];
+      if (M == M_PERIODIC || d == D - 1) {
+        // std::min(a, P - a) by one instruction: NaN in a is NaN in P - a too, a NaN
+        // period leaves a on both, and the sign of a zero is lost in the square.
+        const T a = __builtin_fabs(m);
+        m = fmin_t(a, rp.mparam[d] - a);
+      }
       s = (d == D - 1) ? m * m : m * m + s;
     }
     return s;
@@ -833,11 +843,6 @@ __device__ __forceinline__ void wave_counting_sort(int b, int e, const int32_t* 
     }
   }
 }
-
-__device__ __forceinline__ float fmin_t(float a, float b) { return __builtin_fminf(a, b); }
-__device__ __forceinline__ double fmin_t(double a, double b) { return __builtin_fmin(a, b); }
-__device__ __forceinline__ float fmax_t(float a, float b) { return __builtin_fmaxf(a, b); }
-__device__ __forceinline__ double fmax_t(double a, double b) { return __builtin_fmax(a, b); }
 
 // Minimum and maximum over each group of N = 8 or 16 lanes (a half row or a row),
 // in every lane of the group (float through DPP lane moves: pair swap, quad swap,
@@ -1110,7 +1115,7 @@ enum { K_GAUSS2 = 3, K_EXP_UNIT = 4, K_GAUSS2_UNIT = 5 };
 // handling; both forms give the same value there.
 template <bool InRange>
 __device__ __forceinline__ float kernel_exp(float x, const RunParamsT<float>&) {
-  return InRange ? expf_cw_core(x) : expf_cw(x);
+  return InRange ? expf_cw_core<true>(x) : expf_cw(x);
 }
 template <bool InRange>
 __device__ __forceinline__ double kernel_exp(double x, const RunParamsT<double>&) {
@@ -1132,7 +1137,7 @@ __device__ __forceinline__ T kernel_value(T v, const RunParamsT<T>& rp, T c0) {
     // exp((-dd*dd) * 2^-s) with 2^-s = 1 / gauss_den folded into rp.es.
     const T dd = finish_distance<M, Normal>(v);
     const T y = -dd * dd;
-    const T e = InRange ? expf_cw_core_scaled(y, rp.es, c0) : expf_cw_scaled(y, rp.es, c0);
+    const T e = InRange ? expf_cw_core_scaled<true>(y, rp.es, c0) : expf_cw_scaled(y, rp.es, c0);
     return K == K_GAUSS2_UNIT ? e : rp.kp1 * e;
   } else {
     const T dd = finish_distance<M, Normal>(v);
@@ -1184,13 +1189,17 @@ __device__ __forceinline__ T metric_lb(const T (&qlo)[D], const T (&qhi)[D], con
 #pragma unroll
     for (int d = D - 1; d >= 0; --d) s = rp.mparam[d] * g[d] * g[d] + s;
     return s;
-  } else if constexpr (M == M_PERIODIC) {
+  } else if constexpr (M == M_PERIODIC || M == M_PERIODIC_LAST) {
     // a = |dx| lies in [g, G]. With period P > 0, min(a, P - a) >= min(g, P - G)
     // when P - G >= 0 (else 0 bounds its square). With P <= 0 (an unwrapped
     // dimension), min(a, P - a) = P - a and |P - a| >= a >= g.
     T s;
 #pragma unroll
     for (int d = D - 1; d >= 0; --d) {
+      if (M == M_PERIODIC_LAST && d < D - 1) {
+        s = g[d] * g[d] + s;
+        continue;
+      }
       const T P = rp.mparam[d];
       const T G = fmax_t(qhi[d] - bl[d], bh[d] - qlo[d]);
       const T pg = P - G;
@@ -1219,8 +1228,26 @@ __device__ __forceinline__ T metric_lb(const T (&qlo)[D], const T (&qhi)[D], con
   }
 }
 
+// 1 where v * scale <= limit by at least one, 0 where it is not less (and for a NaN
+// v): the fma's output clamped to [0, 1]. With limit = scale * t, t the next value
+// above a threshold and scale a power of two that makes t's unit in the last place
+// at least one, it is 1 exactly where v is within the threshold.
+__device__ __forceinline__ float within(float v, float limit, float scale) {
+  float in;
+  asm("v_fma_f32 %0, -%1, %2, %3 clamp" : "=v"(in) : "v"(v), "s"(scale), "v"(limit));
+  return in;
+}
+__device__ __forceinline__ double within(double v, double limit, double scale) {
+  double in;
+  asm("v_fma_f64 %0, -%1, %2, %3 clamp" : "=v"(in) : "v"(v), "s"(scale), "v"(limit));
+  return in;
+}
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // Compile-time loop modes of the density stage: kernel exp arguments known to be
-// in range, and square roots known to need no tiny-input branch.
+// in range, and square roots known to need no tiny-input branch (flat kernel: the
+// sums by within()).
 template <bool InRange, bool Normal>
 struct ModeC {
   static constexpr bool kInRange = InRange;
@@ -1297,10 +1324,18 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
       constexpr bool inr = decltype(mode_c)::kInRange;
       constexpr bool nrm = decltype(mode_c)::kNormal;
       if constexpr (K == K_FLAT) {
-        // rho + 0 == rho here (rho is never -0), so selecting the unchanged sum is
-        // the reference's addition of a zero term.
-        const T next = rho + ((own && j == s) ? wself : wj);
-        rho = (v <= thr) ? next : rho;
+        const T wt = (own && j == s) ? wself : wj;
+        if constexpr (nrm) {
+          // rho + 1 * w rounds as rho + w does, and rho + 0 * w is rho for a finite
+          // w: two instructions where a compare, a select (both at half rate) and an
+          // addition take three.
+          rho = fma_t(within(v, thr, rp.in_scale), wt, rho);
+        } else {
+          // rho + 0 == rho here (rho is never -0), so selecting the unchanged sum is
+          // the reference's addition of a zero term.
+          const T next = rho + wt;
+          rho = (v <= thr) ? next : rho;
+        }
       } else if constexpr (K == K_EXP_UNIT || K == K_GAUSS2_UNIT) {
         // Amplitude 1: the diagonal's distance is 0 and exp(-0) is exactly 1, the
         // reference's K(i, i), so the diagonal needs no case of its own.
@@ -1312,6 +1347,8 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
         }
       }
     };
+    // The diagonal needs a case of its own (not with amplitude 1, see add).
+    constexpr bool kDiagonal = K != K_EXP_UNIT && K != K_GAUSS2_UNIT;
     auto walk = [&](int j0, int j1, T thr, auto own_c, auto mode_c) {
       int j = j0;
       for (; j + U <= j1; j += U) {
@@ -1319,8 +1356,15 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
   #pragma unroll
         for (int k = 0; k < U; ++k) v[k] = metric_value<D, M>(xi, si, sx, cs, j + k, ssig, rp);
         load_block<U>(wcol + j, w);
+        // In the own tile only the blocks that hold a lane's point test for it.
+        if (kDiagonal && decltype(own_c)::value &&
+            ballot(static_cast<unsigned>(s - j) < static_cast<unsigned>(U)) != 0ull) {
   #pragma unroll
-        for (int k = 0; k < U; ++k) add(v[k], j + k, w[k], thr, own_c, mode_c);
+          for (int k = 0; k < U; ++k) add(v[k], j + k, w[k], thr, std::true_type{}, mode_c);
+        } else {
+  #pragma unroll
+          for (int k = 0; k < U; ++k) add(v[k], j + k, w[k], thr, std::false_type{}, mode_c);
+        }
       }
       for (; j < j1; ++j)
         add(metric_value<D, M>(xi, si, sx, cs, j, ssig, rp), j, wcol[j], thr, own_c, mode_c);
@@ -1330,7 +1374,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
     // lane's threshold) holds only candidates beyond every lane's radius, whose
     // terms the reference adds as +0, so it is skipped without changing the sums.
     // (The own tile is the dense one: there nearly every box is reached.)
-    auto walk_boxes = [&](int j0, int j1, T thr, auto mode_c) {
+    auto walk_boxes = [&](int j0, int j1, T thr_box, T thr, auto mode_c) {
       if constexpr (M != M_MAHALANOBIS) {
         for (int j = j0; j < j1;) {
           const int qb = j / kSortedBox;
@@ -1341,7 +1385,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
             bl[d] = sbox[static_cast<int64_t>(qb) * 2 * D + d];
             bh[d] = sbox[static_cast<int64_t>(qb) * 2 * D + D + d];
           }
-          if (ballot(metric_lb<D, M>(xi, xi, bl, bh, rp) <= thr) != 0ull)
+          if (ballot(metric_lb<D, M>(xi, xi, bl, bh, rp) <= thr_box) != 0ull)
             walk(j, je, thr, std::false_type{}, mode_c);
           j = je;
         }
@@ -1353,11 +1397,13 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
       walk_tiles<D>(lo, hi, ev.nper, rp.wrapped, ev.t_base, [&](int t, bool in) {
         const int j0 = toff[t];
         const int j1 = toff[t + 1];
-        const T thr = in ? thr_in : T(-1);
+        const T thr_box = in ? thr_in : T(-1);
+        const T thr = (K == K_FLAT && decltype(mode_c)::kNormal) ? (in ? rp.in_limit : -rp.in_limit)
+                                                                 : thr_box;
         if (t == it.tile)
           walk(j0, j1, thr, std::true_type{}, mode_c);
         else if (sbox)
-          walk_boxes(j0, j1, thr, mode_c);
+          walk_boxes(j0, j1, thr_box, thr, mode_c);
         else
           walk(j0, j1, thr, std::false_type{}, mode_c);
       });
@@ -1369,8 +1415,20 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
     //    (floats of magnitude >= 2^-24 are multiples of 2^-47, and the largest float
     //    below 2^-24 is 2^-24 - 2^-48), so v >= 2^-96 and the square root needs no
     //    tiny-input branch.
+    // The flat kernel has one decision of another kind: sums through within(), taken
+    // again with selects where a weight was not finite (0 * inf is NaN; finite
+    // weights get here only when their sum overflows). 2^20 points in 2-D: 986 us
+    // with selects, 801 us.
     if constexpr (K == K_FLAT) {
-      run(ModeC<true, false>{});
+      bool again = true;
+      if (rp.in_scale != T(0)) {
+        run(ModeC<true, true>{});
+        again = ballot(!(__builtin_fabs(rho) <= std::numeric_limits<T>::max())) != 0ull;
+      }
+      if (again) {
+        rho = T(0);
+        run(ModeC<true, false>{});
+      }
     } else {
       bool tiny = false;
   #pragma unroll
@@ -2244,6 +2302,9 @@ static void launch_nh_blocks_d(const NeighbourLaunch<T>& L) {
     case M_EUCLID: launch_nh_blocks_dm<D, M_EUCLID>(L); break;
     case M_WEUCLID: launch_nh_blocks_dm<D, M_WEUCLID>(L); break;
     case M_PERIODIC: launch_nh_blocks_dm<D, M_PERIODIC>(L); break;
+    case M_PERIODIC_LAST:
+      if constexpr (D >= 2) launch_nh_blocks_dm<D, M_PERIODIC_LAST>(L);
+      break;
     case M_MANHATTAN: launch_nh_blocks_dm<D, M_MANHATTAN>(L); break;
     case M_CHEBYSHEV: launch_nh_blocks_dm<D, M_CHEBYSHEV>(L); break;
     default: launch_nh_blocks_dm<D, M_WCHEBYSHEV>(L); break;
@@ -2269,6 +2330,14 @@ void launch_neighbour_d(const NeighbourLaunch<T>& L, bool density) {
     CLUE_METRIC_CASE(M_EUCLID)
     CLUE_METRIC_CASE(M_WEUCLID)
     CLUE_METRIC_CASE(M_PERIODIC)
+    case M_PERIODIC_LAST:
+      if constexpr (D >= 2) {
+        if (density)
+          launch_density_dm<D, M_PERIODIC_LAST>(L);
+        else
+          launch_nh_dm<D, M_PERIODIC_LAST>(L);
+      }
+      break;
     CLUE_METRIC_CASE(M_MANHATTAN)
     CLUE_METRIC_CASE(M_CHEBYSHEV)
     CLUE_METRIC_CASE(M_WCHEBYSHEV)

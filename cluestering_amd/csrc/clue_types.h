@@ -14,6 +14,10 @@ constexpr int kNhBlock = 16;
 // skips a box that no lane can reach).
 constexpr int kSortedBox = 16;
 
+// Metric id of a periodic Euclidean metric whose only non-zero period is the last
+// dimension's (a detector's phi): chosen by the host for the device stages alone.
+constexpr int kMetricPeriodicLast = 7;
+
 // Largest tile count of an event that the fused per-event tile build takes (its
 // per-wave tile counters live in LDS); batches with a larger event take the
 // radix-sort path.
@@ -103,6 +107,8 @@ struct RunParamsT {
   T dc_sq_max;           // largest t with sqrt_rn(t) <= dc (sqrt metrics)
   T dm_sq_max;           // same for dm
   T seed_sq_max;         // same for seed_dc
+  T in_scale;            // 2^k and 2^k times the value after the density radius' threshold, for
+  T in_limit;            // the flat kernel's sums (0: not representable)
   T kp0, kp1;            // kernel parameters (flat f | exp lambda, A | gauss sigma, A)
   T gauss_den;           // (2 * sigma) * sigma, as the reference evaluates it
   T gauss_inv_den;       // 1 / gauss_den when gauss_den is a power of two

@@ -366,3 +366,26 @@ def test_large_tiles(gpu_ctx, oracle_mod, plain):
                     name=f"large-tiles plain={plain}"), gpu_ctx, oracle_mod)
     finally:
         gpu_ctx.set_tuning()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [40, 3000])
+def test_flat_sums_with_infinite_and_nan_weights(gpu_ctx, n, dtype):
+    """Flat kernel, unit weights but for one infinite and one NaN: their neighbours'
+    sums are infinite or NaN, every other point's sum is exact and untouched."""
+    from cluestering_amd.device import Clusterer, PointsDevice
+    print(f"[case] non-finite weights n={n} {np.dtype(dtype)}", flush=True)
+    rng = np.random.default_rng(77)
+    xy = rng.uniform(0, np.sqrt(n) * 0.7, size=(2, n)).astype(dtype)
+    xy[:, :4] = np.array([[-9.0, -8.5, 90.0, 90.5], [0.0, 0.0, 0.0, 0.0]], dtype)
+    w = np.ones(n, dtype)
+    w[1], w[3] = np.inf, np.nan
+    p = PointsDevice.from_host(gpu_ctx, xy, w, dtype=dtype)
+    Clusterer(gpu_ctx, 1.0, 2.0).make_clusters(p, None, K.FlatKernel(0.5))
+    rho = p.rho.to_host()
+    x, y = xy
+    near = np.sqrt((x[:, None] - x[None]) ** 2 + (y[:, None] - y[None]) ** 2) <= 1
+    want = 0.5 * near.sum(1) + 0.5   # the point itself counts 1
+    assert rho[0] == np.inf and rho[1] == np.inf
+    assert np.isnan(rho[2]) and np.isnan(rho[3])
+    np.testing.assert_array_equal(rho[4:], want[4:].astype(dtype))
