@@ -184,7 +184,7 @@ struct WorkspaceShape {
   bool own_rho = false;            // results the caller does not provide live in the workspace
   bool own_nh = false;
   bool own_is_seed = false;
-  bool sorted_boxes = false;       // density culls candidate blocks by their bounding boxes
+  bool sorted_boxes = false;       // density leaves out tiles by their bounding boxes
   bool density_morton = false;     // density takes the Morton order (no class order for dc)
 };
 
@@ -224,7 +224,7 @@ inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) 
   bytes[S_HIDX] = sizeof(int32_t) * h_slots;
   bytes[S_HBOX] = T * h_blocks * 2 * D;
   bytes[S_HBKEY] = sizeof(uint64_t) * h_blocks;
-  bytes[S_SBOX] = w.sorted_boxes ? T * ((n + clue_dev::kSortedBox - 1) / clue_dev::kSortedBox) * 2 * D : 0;
+  bytes[S_SBOX] = w.sorted_boxes ? T * NT * 2 * D : 0;  // one box per tile
   bytes[S_SRHO] = T * n;
   bytes[S_SKEY] = w.nh_blocks ? 0 : sizeof(uint64_t) * n;  // the block scan's keys: S_HKEY
   bytes[S_SFW] = w.flat_kernel ? T * n : 0;

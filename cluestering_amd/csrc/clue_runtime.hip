@@ -79,30 +79,29 @@ clue_status validate(const P* p) {
   return CLUE_OK;
 }
 
-// Whether the nearest-higher stage runs over the Morton-ordered block layout:
-// it needs the Morton order of the query grouping, candidates visited in any
-// order (unique tags: the default ones), and a metric with a lower bound over a
-// bounding box (not Mahalanobis; weighted metrics with weights >= 0).
-// Bounding boxes of each kSortedBox tile-sorted positions, for the density stage's
-// block culling: every metric with a lower bound over a box (not Mahalanobis),
-// weighted metrics with weights >= 0.
+// A metric with monotone terms: weights, where there are any, are not below 0.
 template <class P>
-bool sorted_boxes_enabled(const P* p) {
-  if (p->metric == CLUE_METRIC_MAHALANOBIS) return false;
+bool weights_not_negative(const P* p) {
   if (p->metric == CLUE_METRIC_WEIGHTED_EUCLIDEAN || p->metric == CLUE_METRIC_WEIGHTED_CHEBYSHEV)
     for (int d = 0; d < p->ndim; ++d)
       if (!(p->mparam[d] >= 0)) return false;
   return true;
 }
 
+// A metric with a lower bound over a bounding box (not Mahalanobis).
+template <class P>
+bool sorted_boxes_enabled(const P* p) {
+  return p->metric != CLUE_METRIC_MAHALANOBIS && weights_not_negative(p);
+}
+
+// Whether the nearest-higher stage runs over the Morton-ordered block layout:
+// it needs the Morton order of the query grouping, candidates visited in any
+// order (unique tags: the default ones), and a metric with a lower bound over a
+// bounding box.
 template <class P, class Pts>
 bool nh_blocks_enabled(const P* p, const Pts* pts, const BatchPlan& bp) {
   if (bp.tuning.nh_plain_scan || !bp.tuning.group_queries || pts->tags != nullptr) return false;
-  if (p->metric == CLUE_METRIC_MAHALANOBIS) return false;
-  if (p->metric == CLUE_METRIC_WEIGHTED_EUCLIDEAN || p->metric == CLUE_METRIC_WEIGHTED_CHEBYSHEV)
-    for (int d = 0; d < p->ndim; ++d)
-      if (!(p->mparam[d] >= 0)) return false;
-  return true;
+  return sorted_boxes_enabled(p);
 }
 
 // Density's queries in Morton order: with candidate boxes the class order buys
@@ -130,6 +129,7 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
   rp.block_waves = bp.tuning.block_waves > 0 ? bp.tuning.block_waves : 4;
   rp.persistent = bp.tuning.persistent > 0 ? bp.tuning.persistent : 0;
   rp.nh_blocks = nh_blocks_enabled(p, pts, bp) ? 1 : 0;
+  rp.cull = weights_not_negative(p) ? 1 : 0;
   rp.D = p->ndim;
   rp.kernel = p->kernel;
   rp.metric = p->metric;
@@ -333,7 +333,7 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   b.hbox = nhb ? at<T>(slot, S_HBOX) : nullptr;
   b.hbkey = nhb ? at<uint64_t>(slot, S_HBKEY) : nullptr;
   b.h_stride = h_slots;
-  b.sbox = sorted_boxes_enabled(p) ? at<T>(slot, S_SBOX) : nullptr;
+  b.tbox = sorted_boxes_enabled(p) ? at<T>(slot, S_SBOX) : nullptr;
   for (int d = 0; d < kMaxDim; ++d) {
     b.sorted.x[d] = d < D ? at<T>(slot, S_SX) + stride * d : nullptr;
     b.sorted.sigma[d] = (has_sigma && d < D) ? at<T>(slot, S_SSIG) + stride * d : nullptr;

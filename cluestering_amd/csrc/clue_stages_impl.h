@@ -834,6 +834,19 @@ __device__ __forceinline__ void wave_counting_sort(int b, int e, const int32_t* 
   }
 }
 
+// Wave-wide minimum and maximum of floating-point values.
+template <class T>
+__device__ __forceinline__ T wave_min_f(T v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = fmin_t(v, __shfl_xor(v, off, 64));
+  return v;
+}
+template <class T>
+__device__ __forceinline__ T wave_max_f(T v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = fmax_t(v, __shfl_xor(v, off, 64));
+  return v;
+}
 // Minimum and maximum over each group of N = 8 or 16 lanes (a half row or a row),
 // in every lane of the group (float through DPP lane moves: pair swap, quad swap,
 // half-row mirror, then for 16 the row mirror; lanes a move does not write take
@@ -949,65 +962,39 @@ __device__ __forceinline__ void write_nh_layout(int t, int b, int cnt, const int
   }
 }
 
-// Bounding box of each kSortedBox consecutive tile-sorted positions (positions
-// past n hold nothing). A box may cover the end of one tile and the start of the
-// next, or of two events: it then bounds more points than a walk takes from it,
-// which only makes it skipped less often. Float: a thread takes four positions
-// with one 16-byte load per column (the columns start 64-aligned) and four lanes
-// make a box; double: sixteen lanes, one position each.
-template <class F>
-__device__ __forceinline__ float quad_reduce_dpp(float v, float id, F op) {
-  const int i = __float_as_int(id);
-  int x = __float_as_int(v);
-  x = __float_as_int(op(__int_as_float(x), __int_as_float(__builtin_amdgcn_update_dpp(i, x, 0xB1, 0xF, 0xF, false))));
-  x = __float_as_int(op(__int_as_float(x), __int_as_float(__builtin_amdgcn_update_dpp(i, x, 0x4E, 0xF, 0xF, false))));
-  return __int_as_float(x);
-}
-
+// Bounding box of every tile's points, one wave per tile: the density stage leaves
+// out the tiles none of a wave's queries can reach.
 template <int D, class T>
-__global__ __launch_bounds__(kBlock) void k_sorted_boxes(const T* __restrict__ sx, int64_t cs,
-                                                         int n, T* __restrict__ sbox) {
-  static_assert(kSortedBox == 16, "a box is four lanes of four floats, or one row of 16 lanes");
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if constexpr (sizeof(T) == 4) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    const int64_t p = 4 * t;  // first of the thread's four positions
+__global__ __launch_bounds__(kBlock) void k_tile_boxes(const int32_t* __restrict__ toff, int n_tiles,
+                                                       const T* __restrict__ sx, int64_t cs,
+                                                       T* __restrict__ tbox) {
+  const int t = blockIdx.x * kWaves + threadIdx.x / kWave;
+  if (t >= n_tiles) return;
+  const int e = toff[t + 1];
+  T lo[D], hi[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    lo[d] = std::numeric_limits<T>::infinity();
+    hi[d] = -std::numeric_limits<T>::infinity();
+  }
+#pragma unroll 4
+  for (int s = toff[t] + lane_id(); s < e; s += kWave)
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      float lo = __builtin_inff(), hi = -__builtin_inff();
-      if (p + 3 < n) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(sx + d * cs + p);
-        lo = __builtin_fminf(__builtin_fminf(v.x, v.y), __builtin_fminf(v.z, v.w));
-        hi = __builtin_fmaxf(__builtin_fmaxf(v.x, v.y), __builtin_fmaxf(v.z, v.w));
-      } else {
-        for (int k = 0; k < 4; ++k)
-          if (p + k < n) {
-            const float x = sx[d * cs + p + k];
-            lo = __builtin_fminf(lo, x);
-            hi = __builtin_fmaxf(hi, x);
-          }
-      }
-      lo = quad_reduce_dpp(lo, __builtin_inff(), [](float a, float b) { return __builtin_fminf(a, b); });
-      hi = quad_reduce_dpp(hi, -__builtin_inff(), [](float a, float b) { return __builtin_fmaxf(a, b); });
-      if (p < n && (t % 4) == 0) {
-        const int64_t q = p / kSortedBox;
-        sbox[q * 2 * D + d] = lo;
-        sbox[q * 2 * D + D + d] = hi;
-      }
+      const T x = sx[d * cs + s];
+      lo[d] = fmin_t(lo[d], x);
+      hi[d] = fmax_t(hi[d], x);
     }
-  } else {
-    const int64_t p = t;
-    const bool real = p < n;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    lo[d] = wave_min_f(lo[d]);
+    hi[d] = wave_max_f(hi[d]);
+  }
+  if (lane_id() == 0) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      const T x = real ? sx[d * cs + p] : T(0);
-      const T lo = row_min(real ? x : std::numeric_limits<T>::infinity());
-      const T hi = row_max(real ? x : -std::numeric_limits<T>::infinity());
-      if (real && (p % kSortedBox) == 0) {
-        const int64_t q = p / kSortedBox;
-        sbox[q * 2 * D + d] = lo;
-        sbox[q * 2 * D + D + d] = hi;
-      }
+      tbox[static_cast<int64_t>(t) * 2 * D + d] = lo[d];
+      tbox[static_cast<int64_t>(t) * 2 * D + D + d] = hi[d];
     }
   }
 }
@@ -1276,6 +1263,123 @@ __device__ __forceinline__ double within(double v, double limit, double scale) {
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
+// Lane i's value in every lane (i wave-uniform).
+__device__ __forceinline__ float read_lane(float v, int i) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
+}
+__device__ __forceinline__ double read_lane(double v, int i) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane(static_cast<int>(b), i);
+  const int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), i);
+  return __longlong_as_double((static_cast<long long>(hi) << 32) |
+                              static_cast<long long>(static_cast<uint32_t>(lo)));
+}
+__device__ __forceinline__ uint64_t read_lane(uint64_t v, int i) {
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), i));
+  const uint32_t hi =
+      static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), i));
+  return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// ---------------------------------------------------------------------------
+// The candidates a wave of queries has to look at: the tiles of the union of the
+// lanes' search boxes in the reference's order (dimension 0 outermost), listed 64
+// at a time, one per lane, so that their offsets and boxes arrive together.
+// ---------------------------------------------------------------------------
+template <int D>
+struct BoxUnion {
+  int lo[D], ext[D];
+  int tiles;  // 0: no active lane
+};
+template <int D>
+__device__ __forceinline__ BoxUnion<D> box_union(const int (&lo)[D], const int (&hi)[D]) {
+  BoxUnion<D> u;
+  u.tiles = 1;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    u.lo[d] = wave_min_uniform(lo[d]);
+    const int h = wave_max_uniform(hi[d]);
+    u.ext[d] = h - u.lo[d] + 1;
+    u.tiles = u.lo[d] > h ? 0 : u.tiles * u.ext[d];
+  }
+  return u;
+}
+
+template <int D>
+struct TileGroup {
+  int t, j0, j1;  // this lane's tile and its candidates
+  int b[D];       // its bins (past nper on a wrapped dimension)
+};
+template <int D>
+__device__ __forceinline__ void list_tiles(const BoxUnion<D>& u, int base, int nper,
+                                           const int32_t* wrapped, int t_base,
+                                           const int32_t* __restrict__ toff, TileGroup<D>* g) {
+  const int idx = base + lane_id();
+  int q = idx, t = 0, scale = 1;
+#pragma unroll
+  for (int d = D - 1; d >= 0; --d) {
+    const int r = d == 0 ? q : q % u.ext[d];
+    q = d == 0 ? 0 : q / u.ext[d];
+    g->b[d] = u.lo[d] + r;
+    t += scale * (wrapped[d] ? g->b[d] % nper : g->b[d]);
+    scale *= nper;
+  }
+  g->t = t_base + t;
+  g->j0 = g->j1 = 0;
+  if (idx < u.tiles) {
+    g->j0 = toff[g->t];
+    g->j1 = toff[g->t + 1];
+  }
+}
+// Does each lane's own box hold the tile of lane i?
+template <int D>
+__device__ __forceinline__ bool box_holds(const TileGroup<D>& g, int i, const int (&lo)[D],
+                                          const int (&hi)[D]) {
+  bool in = true;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const int b = __builtin_amdgcn_readlane(g.b[d], i);
+    in = in && lo[d] <= b && b <= hi[d];
+  }
+  return in;
+}
+
+// Box of a wave's query points, and their largest sigmas (wave-uniform, in scalar
+// registers).
+template <int D, class T>
+struct QueryBox {
+  T lo[D], hi[D], s[D];
+};
+template <int D, int M, class T>
+__device__ __forceinline__ QueryBox<D, T> query_box(const T (&x)[D], const T (&s)[D], bool active) {
+  QueryBox<D, T> q;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    q.lo[d] = read_lane(wave_min_f(active ? x[d] : std::numeric_limits<T>::infinity()), 0);
+    q.hi[d] = read_lane(wave_max_f(active ? x[d] : -std::numeric_limits<T>::infinity()), 0);
+    q.s[d] = M == M_MAHALANOBIS ? read_lane(wave_max_f(active ? __builtin_fabs(s[d]) : T(0)), 0) : T(0);
+  }
+  return q;
+}
+// A lower bound of the metric between any query of the box and a candidate at x (with
+// sigma sx, Mahalanobis): the metric's own operations on the gaps and, Mahalanobis, on
+// the largest sigma, each monotone after rounding. A NaN excludes nothing.
+template <int D, int M, class T>
+__device__ __forceinline__ bool out_of_reach(const QueryBox<D, T>& q, const T (&x)[D],
+                                             const T (&sx)[D], const RunParamsT<T>& rp, T thr) {
+  if constexpr (M == M_MAHALANOBIS) {
+    T s = T(0);
+#pragma unroll
+    for (int d = D - 1; d >= 0; --d) {
+      const T g = fmax_t(fmax_t(x[d] - q.hi[d], q.lo[d] - x[d]), T(0));
+      s = g * g / (q.s[d] * q.s[d] + sx[d] * sx[d]) + s;
+    }
+    return s > thr;
+  } else {
+    return metric_lb<D, M>(q.lo, q.hi, x, x, rp) > thr;
+  }
+}
+
 // Compile-time loop modes of the density stage: kernel exp arguments known to be
 // in range, and square roots known to need no tiny-input branch (flat kernel: the
 // sums by within()).
@@ -1286,12 +1390,10 @@ struct ModeC {
 };
 
 // Candidates are walked in blocks of U so that their wave-uniform data arrives
-// in a few wide scalar loads (measured on MI355X: 8 for density, 16 for
-// nearest-higher, whose blocks carry less work per candidate).
+// in a few wide scalar loads (measured on MI355X).
 template <int D>
 struct Unroll {
   static constexpr int U = D <= 3 ? 8 : 4;
-  static constexpr int U_NH = D <= 3 ? 16 : 4;
 };
 
 // ---------------------------------------------------------------------------
@@ -1306,7 +1408,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
     int32_t* __restrict__ n_items, const T* __restrict__ sx, int64_t cs,
     const T* __restrict__ sw, const T* __restrict__ sfw, const T* __restrict__ ssig,
     const uint32_t* __restrict__ stag, const int32_t* __restrict__ qperm,
-    T* __restrict__ srho, uint64_t* __restrict__ skey, const T* __restrict__ sbox,
+    T* __restrict__ srho, uint64_t* __restrict__ skey, const T* __restrict__ tbox,
     uint64_t* __restrict__ hkey, uint64_t* __restrict__ hbkey) {
   constexpr int U = Unroll<D>::U;
   auto process = [&](const int item) {
@@ -1387,8 +1489,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
   #pragma unroll
         for (int k = 0; k < U; ++k) v[k] = metric_value<D, M>(xi, si, sx, cs, j + k, ssig, rp);
         load_block<U>(wcol + j, w);
-        // In the own tile only the blocks that hold a lane's point test for it.
-        if (kDiagonal && decltype(own_c)::value &&
+        if (decltype(own_c)::value &&
             ballot(static_cast<unsigned>(s - j) < static_cast<unsigned>(U)) != 0ull) {
   #pragma unroll
           for (int k = 0; k < U; ++k) add(v[k], j + k, w[k], thr, std::true_type{}, mode_c);
@@ -1400,44 +1501,95 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
       for (; j < j1; ++j)
         add(metric_value<D, M>(xi, si, sx, cs, j, ssig, rp), j, wcol[j], thr, own_c, mode_c);
     };
-    // A neighbour tile's candidates go by boxes of kSortedBox sorted positions: a
-    // box that no lane can reach (a lower bound of the metric over it above every
-    // lane's threshold) holds only candidates beyond every lane's radius, whose
-    // terms the reference adds as +0, so it is skipped without changing the sums.
-    // (The own tile is the dense one: there nearly every box is reached.)
-    auto walk_boxes = [&](int j0, int j1, T thr_box, T thr, auto mode_c) {
-      if constexpr (M != M_MAHALANOBIS) {
-        for (int j = j0; j < j1;) {
-          const int qb = j / kSortedBox;
-          const int je = min(j1, (qb + 1) * kSortedBox);
+    // A tile's candidates, 64 at a time, one per lane: those that no query of the wave
+    // can reach (a lower bound of the metric above the radius: the reference adds
+    // their terms as +0) are left out by one ballot. Where few are left, their
+    // coordinates come from the lanes; where many are, the block is walked whole,
+    // through the scalar cache, which costs a candidate four instructions less. The
+    // line between them, measured at 1/8 to 13/16: the 4096-event batch is flat from
+    // 1/4 to 1/2 (22.5-22.7 ms; 23.5 at 2/3), 2^20 points in 2-D and 3-D best from 3/8
+    // to 1/2 (742, 733 us; 482, 473 us).
+    const bool cull = rp.cull != 0;
+    const QueryBox<D, T> qb = query_box<D, M>(xi, si, active);
+    auto walk_tile = [&](int j0, int j1, T thr, auto mode_c) {
+      T nx[D], ns[D];
+      auto fetch = [&](int j) {
+        const int c = j + lane_id();
+  #pragma unroll
+        for (int d = 0; d < D; ++d) {
+          nx[d] = c < j1 ? sx[d * cs + c] : T(0);
+          ns[d] = (M == M_MAHALANOBIS && c < j1) ? ssig[d * cs + c] : T(0);
+        }
+      };
+      fetch(j0);
+      for (int j = j0; j < j1; j += kWave) {
+        T cx[D], cg[D];
+  #pragma unroll
+        for (int d = 0; d < D; ++d) {
+          cx[d] = nx[d];
+          cg[d] = ns[d];
+        }
+        if (j + kWave < j1) fetch(j + kWave);
+        const int cnt = min(kWave, j1 - j);
+        uint64_t left = ballot(lane_id() < cnt &&
+                               !(cull && out_of_reach<D, M>(qb, cx, cg, rp, thr_in)));
+        const int n = __popcll(left);
+        if (n == 0) continue;
+        const T cw = lane_id() < cnt ? wcol[j + lane_id()] : T(0);
+        auto each = [&](auto self_c) {
+          if (8 * n >= 3 * cnt) {
+            walk(j, j + cnt, thr, self_c, mode_c);
+            return;
+          }
+          while (left) {
+            const int i = __builtin_ctzll(left);
+            left &= left - 1ull;
+            T xj[D], sj[D];
+  #pragma unroll
+            for (int d = 0; d < D; ++d) {
+              xj[d] = read_lane(cx[d], i);
+              sj[d] = M == M_MAHALANOBIS ? read_lane(cg[d], i) : T(0);
+            }
+            add(metric_pair<D, M>(xi, si, xj, sj, rp), j + i, read_lane(cw, i), thr, self_c,
+                mode_c);
+          }
+        };
+        // Only the blocks that hold a lane's own point test for it.
+        if (kDiagonal && ballot(static_cast<unsigned>(s - j) < static_cast<unsigned>(cnt)) != 0ull)
+          each(std::true_type{});
+        else
+          each(std::false_type{});
+      }
+    };
+    const BoxUnion<D> u = box_union(lo, hi);
+    auto run = [&](auto mode_c) {
+      for (int base = 0; base < u.tiles; base += kWave) {
+        TileGroup<D> g;
+        list_tiles(u, base, ev.nper, rp.wrapped, ev.t_base, toff, &g);
+        bool reach = g.j0 < g.j1;
+        if (M != M_MAHALANOBIS && cull && reach) {
           T bl[D], bh[D];
   #pragma unroll
           for (int d = 0; d < D; ++d) {
-            bl[d] = sbox[static_cast<int64_t>(qb) * 2 * D + d];
-            bh[d] = sbox[static_cast<int64_t>(qb) * 2 * D + D + d];
+            bl[d] = tbox[static_cast<int64_t>(g.t) * 2 * D + d];
+            bh[d] = tbox[static_cast<int64_t>(g.t) * 2 * D + D + d];
           }
-          if (ballot(metric_lb<D, M>(xi, xi, bl, bh, rp) <= thr_box) != 0ull)
-            walk(j, je, thr, std::false_type{}, mode_c);
-          j = je;
+          if constexpr (M != M_MAHALANOBIS)
+            reach = !(metric_lb<D, M>(qb.lo, qb.hi, bl, bh, rp) > thr_in);
         }
-      } else {
-        walk(j0, j1, thr, std::false_type{}, mode_c);
+        uint64_t held = ballot(reach);
+        while (held) {
+          const int i = __builtin_ctzll(held);
+          held &= held - 1ull;
+          const bool in = box_holds(g, i, lo, hi);
+          if (ballot(in) == 0ull) continue;
+          const int j0 = __builtin_amdgcn_readlane(g.j0, i), j1 = __builtin_amdgcn_readlane(g.j1, i);
+          const T thr = (K == K_FLAT && decltype(mode_c)::kNormal)
+                            ? (in ? rp.in_limit : -rp.in_limit)
+                            : (in ? thr_in : T(-1));
+          walk_tile(j0, j1, thr, mode_c);
+        }
       }
-    };
-    auto run = [&](auto mode_c) {
-      walk_tiles<D>(lo, hi, ev.nper, rp.wrapped, ev.t_base, [&](int t, bool in) {
-        const int j0 = toff[t];
-        const int j1 = toff[t + 1];
-        const T thr_box = in ? thr_in : T(-1);
-        const T thr = (K == K_FLAT && decltype(mode_c)::kNormal) ? (in ? rp.in_limit : -rp.in_limit)
-                                                                 : thr_box;
-        if (t == it.tile)
-          walk(j0, j1, thr, std::true_type{}, mode_c);
-        else if (sbox)
-          walk_boxes(j0, j1, thr_box, thr, mode_c);
-        else
-          walk(j0, j1, thr, std::false_type{}, mode_c);
-      });
     };
     // Both decisions are made once, outside the candidate loop:
     //  - in range: launch-wide, every exp argument within the radius is in range;
@@ -1555,6 +1707,36 @@ __device__ __forceinline__ uint64_t query_key(double rho, uint32_t) {
   return rho_key_f64(rho, true);
 }
 
+// A lower bound of the wave's smallest ordering key. (LDS permutes here and in
+// wave_min_f: the DPP form costs more vector instructions, and this scan is short of
+// them; measured on MI355X.)
+// The smallest high word with a zero low word: never above the smallest key, so
+// "a block key above it" keeps every block that could hold a higher candidate.
+__device__ __forceinline__ uint64_t wave_min_key_bound(uint64_t v) {
+  uint32_t h = static_cast<uint32_t>(v >> 32);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(h), off, 64));
+    h = o < h ? o : h;
+  }
+  return static_cast<uint64_t>(h) << 32;
+}
+
+// May a block whose largest key is bk hold a candidate higher than the query?
+// Float keys decide it exactly; double keys leave equal densities to the tags.
+__device__ __forceinline__ bool block_may_be_higher(uint64_t bk, uint64_t ki, float) {
+  return bk > ki;
+}
+__device__ __forceinline__ bool block_may_be_higher(uint64_t bk, uint64_t ki, double) {
+  return bk >= ki;
+}
+__device__ __forceinline__ bool key_maybe_higher(uint64_t kj, uint64_t ki, float) {
+  return kj > ki;
+}
+__device__ __forceinline__ bool key_maybe_higher(uint64_t kj, uint64_t ki, double) {
+  return (kj > ki) | ((kj == ki) & (kj > 0x8000000000000000ull));
+}
+
 template <int D, int M, class T>
 __global__ __launch_bounds__(kMaxNeighbourBlock) void k_nearest_higher(
     const RunParamsT<T> rp, const EventDesc* __restrict__ events, const T* __restrict__ geo,
@@ -1565,7 +1747,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_nearest_higher(
     const uint64_t* __restrict__ skey, const int32_t* __restrict__ qperm,
     int32_t* __restrict__ snh, T* __restrict__ sdelta) {
   constexpr bool kF64 = sizeof(T) == 8;
-  constexpr int U = Unroll<D>::U_NH;
+  constexpr int U = Unroll<D>::U;
   const int item = xcd_block(blockIdx.x, gridDim.x, rp.xcd_chunk_log2) * (blockDim.x / kWave) +
                    threadIdx.x / kWave;
   if (item >= *n_items) return;
@@ -1622,45 +1804,88 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_nearest_higher(
     }
   };
 
-  walk_tiles<D>(lo, hi, ev.nper, rp.wrapped, ev.t_base, [&](int t, bool in) {
-    const int j0 = toff[t];
-    const int j1 = toff[t + 1];
-    if (!in) return;  // lanes whose box does not hold this tile idle through it
-    int j = j0;
-    for (; j + U <= j1; j += U) {
-      // m: the smallest distance among the block's higher candidates (vector
-      // selects and minima instead of per-candidate scalar mask logic).
-      T v[U];
-      uint32_t tj[U];
-      T m = std::numeric_limits<T>::infinity();
+  // A candidate's density and tag, loaded where its key does not hold them.
+  auto accept = [&](T v, uint64_t kj, uint64_t key_in, int j) {
+    if (!(key_maybe_higher(kj, key_in, T(0)) && v <= bound)) return;
+    if constexpr (kF64) {
+      const uint32_t tj = stag[j];
+      if (key_higher(kj, tj, key_in, tag_i, T(0))) consider(v, srho[j], tj, j);
+    } else {
+      const float rj = key_rho(kj);
+      consider(v, rj, rj > 0.0f ? static_cast<uint32_t>(kj) : stag[j], j);
+    }
+  };
+
+  // As in the density stage, a tile's candidates 64 at a time, one per lane: those
+  // out of every lane's reach (its bound, here) or not above the wave's smallest key
+  // are left out by one ballot; then from the lanes, or through the scalar cache.
+  const bool cull = rp.cull != 0;
+  const QueryBox<D, T> qb = query_box<D, M>(xi, si, active);
+  const uint64_t kmin = wave_min_key_bound(key_i);
+  const BoxUnion<D> u = box_union(lo, hi);
+  for (int base = 0; base < u.tiles; base += kWave) {
+    TileGroup<D> g;
+    list_tiles(u, base, ev.nper, rp.wrapped, ev.t_base, toff, &g);
+    uint64_t held = ballot(g.j0 < g.j1);
+    while (held) {
+      const int t = __builtin_ctzll(held);
+      held &= held - 1ull;
+      const bool in = box_holds(g, t, lo, hi);
+      if (ballot(in) == 0ull) continue;
+      const int j0 = __builtin_amdgcn_readlane(g.j0, t), j1 = __builtin_amdgcn_readlane(g.j1, t);
+      const uint64_t key_in = in ? key_i : ~0ull;
+      for (int j = j0; j < j1; j += kWave) {
+        const int cnt = min(kWave, j1 - j);
+        const bool valid = lane_id() < cnt;
+        T cx[D], cg[D];
 #pragma unroll
-      for (int k = 0; k < U; ++k) tj[k] = kF64 ? stag[j + k] : 0u;
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        v[k] = metric_value<D, M>(xi, si, sx, cs, j + k, ssig, rp);
-        const bool h = key_higher(skey[j + k], tj[k], key_i, tag_i, T(0));
-        m = fmin_t(m, h ? v[k] : std::numeric_limits<T>::infinity());
-      }
-      // Most blocks hold no candidate for any lane: one wave-wide test skips them.
-      if (ballot(m <= bound) != 0ull) {
-        T rj[U];
-#pragma unroll
-        for (int k = 0; k < U; ++k) {
-          rj[k] = srho[j + k];
-          if (!kF64) tj[k] = stag[j + k];
+        for (int d = 0; d < D; ++d) {
+          cx[d] = valid ? sx[d * cs + j + lane_id()] : T(0);
+          cg[d] = (M == M_MAHALANOBIS && valid) ? ssig[d * cs + j + lane_id()] : T(0);
         }
+        const uint64_t ck = valid ? skey[j + lane_id()] : 0ull;
+        const T bmax = wave_max_f(in ? bound : -std::numeric_limits<T>::infinity());
+        uint64_t left = ballot(valid && block_may_be_higher(ck, kmin, T(0)) &&
+                               !(cull && out_of_reach<D, M>(qb, cx, cg, rp, bmax)));
+        if (left == 0ull) continue;
+        if (8 * __popcll(left) < 3 * cnt) {
+          while (left) {
+            const int i = __builtin_ctzll(left);
+            left &= left - 1ull;
+            T xj[D], sj[D];
 #pragma unroll
-        for (int k = 0; k < U; ++k)
-          if (key_higher(skey[j + k], tj[k], key_i, tag_i, T(0)) && v[k] <= bound)
-            consider(v[k], rj[k], tj[k], j + k);
+            for (int d = 0; d < D; ++d) {
+              xj[d] = read_lane(cx[d], i);
+              sj[d] = M == M_MAHALANOBIS ? read_lane(cg[d], i) : T(0);
+            }
+            accept(metric_pair<D, M>(xi, si, xj, sj, rp), read_lane(ck, i), key_in, j + i);
+          }
+          continue;
+        }
+        int k = j;
+        const int ke = j + cnt;
+        for (; k + U <= ke; k += U) {
+          // m: the smallest distance among the block's higher candidates (vector
+          // selects and minima instead of per-candidate scalar mask logic).
+          T v[U];
+          T m = std::numeric_limits<T>::infinity();
+#pragma unroll
+          for (int c = 0; c < U; ++c) {
+            v[c] = metric_value<D, M>(xi, si, sx, cs, k + c, ssig, rp);
+            const bool h = key_maybe_higher(skey[k + c], key_in, T(0));
+            m = fmin_t(m, h ? v[c] : std::numeric_limits<T>::infinity());
+          }
+          // Most blocks hold no candidate for any lane: one wave-wide test skips them.
+          if (ballot(m <= bound) != 0ull) {
+#pragma unroll
+            for (int c = 0; c < U; ++c) accept(v[c], skey[k + c], key_in, k + c);
+          }
+        }
+        for (; k < ke; ++k)
+          accept(metric_value<D, M>(xi, si, sx, cs, k, ssig, rp), skey[k], key_in, k);
       }
     }
-    for (; j < j1; ++j) {
-      const T v = metric_value<D, M>(xi, si, sx, cs, j, ssig, rp);
-      if (key_higher(skey[j], stag[j], key_i, tag_i, T(0)) & (v <= bound))
-        consider(v, srho[j], stag[j], j);
-    }
-  });
+  }
   if (active) {
     snh[s] = nh;
     sdelta[s] = delta;
@@ -1681,70 +1906,10 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_nearest_higher(
 // monotone), so the results are those of the plain scan.
 // ---------------------------------------------------------------------------
 
-// Wave-wide minimum and maximum of floating-point values, and a lower bound of
-// the wave's smallest ordering key. (LDS permutes here: the DPP form costs more
-// vector instructions, and this scan is short of them; measured on MI355X.)
-template <class T>
-__device__ __forceinline__ T wave_min_f(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmin_t(v, __shfl_xor(v, off, 64));
-  return v;
-}
-template <class T>
-__device__ __forceinline__ T wave_max_f(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax_t(v, __shfl_xor(v, off, 64));
-  return v;
-}
-// The smallest high word with a zero low word: never above the smallest key, so
-// "a block key above it" keeps every block that could hold a higher candidate.
-__device__ __forceinline__ uint64_t wave_min_key_bound(uint64_t v) {
-  uint32_t h = static_cast<uint32_t>(v >> 32);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const uint32_t o = static_cast<uint32_t>(__shfl_xor(static_cast<int>(h), off, 64));
-    h = o < h ? o : h;
-  }
-  return static_cast<uint64_t>(h) << 32;
-}
-
-// Lane i's value in every lane (i wave-uniform).
-__device__ __forceinline__ float read_lane(float v, int i) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i));
-}
-__device__ __forceinline__ double read_lane(double v, int i) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane(static_cast<int>(b), i);
-  const int hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), i);
-  return __longlong_as_double((static_cast<long long>(hi) << 32) |
-                              static_cast<long long>(static_cast<uint32_t>(lo)));
-}
-__device__ __forceinline__ uint64_t read_lane(uint64_t v, int i) {
-  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), i));
-  const uint32_t hi =
-      static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), i));
-  return (static_cast<uint64_t>(hi) << 32) | lo;
-}
-
 // Candidates per register block of the layout scan (a divisor of kNhBlock).
 template <int D>
 constexpr int nh_sub_block() {
   return D <= 3 ? 8 : 4;
-}
-
-// May a block whose largest key is bk hold a candidate higher than the query?
-// Float keys decide it exactly; double keys leave equal densities to the tags.
-__device__ __forceinline__ bool block_may_be_higher(uint64_t bk, uint64_t ki, float) {
-  return bk > ki;
-}
-__device__ __forceinline__ bool block_may_be_higher(uint64_t bk, uint64_t ki, double) {
-  return bk >= ki;
-}
-__device__ __forceinline__ bool key_maybe_higher(uint64_t kj, uint64_t ki, float) {
-  return kj > ki;
-}
-__device__ __forceinline__ bool key_maybe_higher(uint64_t kj, uint64_t ki, double) {
-  return (kj > ki) | ((kj == ki) & (kj > 0x8000000000000000ull));
 }
 
 // Eight waves per SIMD in 1-D and 2-D: the scan waits on chains of scalar loads,
@@ -2261,7 +2426,7 @@ static void launch_density_dmk(const NeighbourLaunch<T>& L) {
   auto go = [&](auto kern, unsigned grid) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(L.block), 0, L.s, *L.rp, b.events, b.geo, b.toff,
                        b.items, b.n_items, b.sorted.x[0], L.cs, b.sorted.w, b.sorted.fw,
-                       b.sorted.sigma[0], b.sorted.tag, b.qperm, b.srho, b.skey, b.sbox,
+                       b.sorted.sigma[0], b.sorted.tag, b.qperm, b.srho, b.skey, b.tbox,
                        b.hkey, b.hbkey);
   };
   if constexpr (kPersistentBuilt<D>) {
@@ -2407,29 +2572,26 @@ static void launch_query_order_d(const NeighbourLaunch<T>& L) {
 }
 
 template <int D, class T>
-static void launch_sorted_boxes_d(const NeighbourLaunch<T>& L) {
+static void launch_tile_boxes_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
-  // Float: four positions per thread; double: one.
-  const int64_t per = sizeof(T) == 4 ? 4 : 1;
-  const int64_t n16 = (static_cast<int64_t>(b.n_total) + kSortedBox - 1) / kSortedBox * kSortedBox;
-  const int64_t threads = n16 / per;
-  hipLaunchKernelGGL((k_sorted_boxes<D, T>), dim3(static_cast<unsigned>((threads + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, L.s, b.sorted.x[0], L.cs, b.n_total, b.sbox);
+  const unsigned grid = static_cast<unsigned>((b.n_tiles_total + kWaves - 1) / kWaves);
+  hipLaunchKernelGGL((k_tile_boxes<D, T>), dim3(grid), dim3(kBlock), 0, L.s, b.toff,
+                     b.n_tiles_total, b.sorted.x[0], L.cs, b.tbox);
 }
 
 template <class T>
-static void launch_sorted_boxes(const NeighbourLaunch<T>& L) {
+static void launch_tile_boxes(const NeighbourLaunch<T>& L) {
   switch (L.rp->D) {
-    case 1: launch_sorted_boxes_d<1>(L); break;
-    case 2: launch_sorted_boxes_d<2>(L); break;
-    case 3: launch_sorted_boxes_d<3>(L); break;
-    case 4: launch_sorted_boxes_d<4>(L); break;
-    case 5: launch_sorted_boxes_d<5>(L); break;
-    case 6: launch_sorted_boxes_d<6>(L); break;
-    case 7: launch_sorted_boxes_d<7>(L); break;
-    case 8: launch_sorted_boxes_d<8>(L); break;
-    case 9: launch_sorted_boxes_d<9>(L); break;
-    default: launch_sorted_boxes_d<10>(L); break;
+    case 1: launch_tile_boxes_d<1>(L); break;
+    case 2: launch_tile_boxes_d<2>(L); break;
+    case 3: launch_tile_boxes_d<3>(L); break;
+    case 4: launch_tile_boxes_d<4>(L); break;
+    case 5: launch_tile_boxes_d<5>(L); break;
+    case 6: launch_tile_boxes_d<6>(L); break;
+    case 7: launch_tile_boxes_d<7>(L); break;
+    case 8: launch_tile_boxes_d<8>(L); break;
+    case 9: launch_tile_boxes_d<9>(L); break;
+    default: launch_tile_boxes_d<10>(L); break;
   }
 }
 
@@ -2535,7 +2697,7 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
       blocks, (static_cast<int64_t>(device_cus()) * std::max(rp.persistent, 0) + waves - 1) / waves);
   L.grid_persistent = static_cast<unsigned>((pblocks + kXcds - 1) / kXcds * kXcds);
   L.s = s;
-  if (bb.sbox) launch_sorted_boxes(L);  // candidate boxes of the density stage
+  if (bb.tbox) launch_tile_boxes(L);    // bounds of the density stage's candidates
   if (bb.qperm) launch_query_order(L);  // query orders of the two neighbour stages
 
   // (b), (c)

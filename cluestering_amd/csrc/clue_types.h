@@ -10,10 +10,6 @@ constexpr int kMaxDim = 10;
 // one largest key per block).
 constexpr int kNhBlock = 16;
 
-// Candidates per bounding box of the tile-sorted columns (the density stage
-// skips a box that no lane can reach).
-constexpr int kSortedBox = 16;
-
 // Metric id of a periodic Euclidean metric whose only non-zero period is the last
 // dimension's (a detector's phi): chosen by the host for the device stages alone.
 constexpr int kMetricPeriodicLast = 7;
@@ -121,6 +117,7 @@ struct RunParamsT {
   int32_t xcd_chunk_log2;  // neighbour stages: 2^k consecutive blocks per XCD turn; < 0: none
   int32_t block_waves;     // neighbour stages: waves per workgroup (1, 2, 4, 8 or 16)
   int32_t nh_blocks;       // nearest-higher over the Morton-ordered block layout
+  int32_t cull;            // density: candidates bounded by the metric's lower bound (no weight below 0)
   int32_t persistent;      // neighbour stages: persistent waves per CU pulling items (0: none)
 };
 using RunParams = RunParamsT<float>;
