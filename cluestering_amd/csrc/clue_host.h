@@ -26,6 +26,15 @@ using clue_dev::scan_temp_elems;
 constexpr int kChunk = 2048;  // points per chunk of the per-point grids
 constexpr int kEvtSoloMaxPoints = 8192;  // largest lone event for the fused per-event stages
 constexpr int kDefaultPointsPerTile = 128;
+// Launches up to this many points have their neighbour stages run by teams of waves
+// (clue_team.h). Lone events on MI355X, one wave per item against a team of eight,
+// whole calls: 16,000 points 258 -> 179 us (2-D) and 476 -> 301 us (3-D), 100,000
+// points 662 -> 551 and 521 -> 449 us, 131,072 points 803 -> 678 and 533 -> 631 us.
+// Batches of small events have short walks and fill the chip sooner: 36,558 points in
+// 16 events 243 -> 192 us, 70,850 in 128 events 171 -> 185 us.
+constexpr int kTeamMaxPoints = 110000;
+constexpr int kTeamMaxPointsSmall = 49152;  // events of fewer than kTeamSmallEvent points
+constexpr int kTeamSmallEvent = 4096;
 
 // Constants of exp(y * 2^-s) (clue_dev::ExpScaled): each constant of the float
 // exp scaled by a power of two, exact for |s| <= 8.
@@ -52,7 +61,7 @@ enum Slot {
   S_EVENTS, S_CHUNKS, S_EXT, S_GEO, S_K0, S_V0, S_K1, S_V1, S_HIST, S_SCAN, S_TOFF, S_ICOUNT,
   S_NITEMS, S_ITEMS, S_SRHO, S_SKEY, S_SNH, S_SDELTA, S_FLAG, S_RANK, S_NSEEDS, S_SEEDS, S_SX,
   S_SW, S_SSIG, S_SU, S_STAG, S_SFW, S_PERM, S_RHO, S_NH, S_ISSEED, S_DELTA, S_HIN, S_HCL,
-  S_QPERM, S_QPERM_NH, S_QFINE, S_QKEY, S_HX, S_HKEY, S_HIDX, S_HBOX, S_HBKEY, S_EORDER, S_ESEEDS, S_EOFF, S_IPERM, S_SBOX, S_NUM
+  S_QPERM, S_QPERM_NH, S_QFINE, S_HX, S_HKEY, S_HIDX, S_HBOX, S_HBKEY, S_EORDER, S_ESEEDS, S_EOFF, S_IPERM, S_SBOX, S_NUM
 };
 
 // Host-side description of one batch (all derived from the event sizes).
@@ -64,6 +73,7 @@ struct BatchPlan {
   int64_t n_tiles_total = 0;
   int64_t max_items = 0;
   int key_bits = 0;
+  bool team = false;  // neighbour stages by teams of waves
   clue_tuning tuning{};
 };
 
@@ -157,6 +167,11 @@ inline clue_status plan_batch(int D, int points_per_tile, const uint32_t* sizes,
                        [&](int32_t a, int32_t b) { return bp->events[a].n > bp->events[b].n; });
   }
   bp->tuning = fixed ? *fixed : table_tuning(D, off, static_cast<int64_t>(bp->events.size()));
+  // A fixed tuning keeps one wave per item.
+  const int64_t mean = bp->events.empty() ? 0 : off / static_cast<int64_t>(bp->events.size());
+  bp->team = !fixed && off <= (mean < kTeamSmallEvent && bp->events.size() > 1 ? kTeamMaxPointsSmall
+                                                                                : kTeamMaxPoints);
+  if (bp->team) bp->tuning.group_queries = 1;  // small boxes around each team's points
   bp->max_items = (off + 63) / 64 + tiles;
   int bits = 0;
   while ((int64_t(1) << bits) < tiles) ++bits;
@@ -218,7 +233,6 @@ inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) 
   bytes[S_QPERM] = (w.group_queries && !w.density_morton) ? sizeof(int32_t) * n : 0;
   bytes[S_QPERM_NH] = (w.group_queries && w.separate_dm_order) ? sizeof(int32_t) * n : 0;
   bytes[S_QFINE] = w.group_queries ? sizeof(int32_t) * n : 0;
-  bytes[S_QKEY] = w.group_queries ? sizeof(uint32_t) * n : 0;
   bytes[S_HX] = T * h_slots * D;
   bytes[S_HKEY] = sizeof(uint64_t) * h_slots;
   bytes[S_HIDX] = sizeof(int32_t) * h_slots;

@@ -100,23 +100,8 @@ bool sorted_boxes_enabled(const P* p) {
 // bounding box.
 template <class P, class Pts>
 bool nh_blocks_enabled(const P* p, const Pts* pts, const BatchPlan& bp) {
-  if (bp.tuning.nh_plain_scan || !bp.tuning.group_queries || pts->tags != nullptr) return false;
+  if (bp.team || bp.tuning.nh_plain_scan || !bp.tuning.group_queries || pts->tags != nullptr) return false;
   return sorted_boxes_enabled(p);
-}
-
-// Density's queries in Morton order: with candidate boxes the class order buys
-// nothing (measured on MI355X on the 4096-event 2-D batch: 24.9 ms either way), and
-// the block scan's layout then receives the keys from the density stage itself.
-template <class P>
-bool density_morton(const P* p, const BatchPlan& bp) {
-  return bp.tuning.group_queries && sorted_boxes_enabled(p);
-}
-
-// The plain nearest-higher scan's own (class, Morton) order for dm, when the
-// density stage's order is not that order.
-template <class P>
-bool separate_dm_order(const P* p, const BatchPlan& bp, bool nhb) {
-  return bp.tuning.group_queries && !nhb && (p->dm != p->dc || density_morton(p, bp));
 }
 
 template <class P, class Pts>
@@ -128,6 +113,7 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
   rp.xcd_chunk_log2 = bp.tuning.xcd_chunk_log2;
   rp.block_waves = bp.tuning.block_waves > 0 ? bp.tuning.block_waves : 4;
   rp.persistent = bp.tuning.persistent > 0 ? bp.tuning.persistent : 0;
+  rp.team = bp.team ? 1 : 0;
   rp.nh_blocks = nh_blocks_enabled(p, pts, bp) ? 1 : 0;
   rp.cull = weights_not_negative(p) ? 1 : 0;
   rp.D = p->ndim;
@@ -173,7 +159,8 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
     rp.gauss_inv_den = rp.gauss_pow2 ? std::ldexp(T(1), 1 - ex) : T(0);
     // Float: fold gauss_den = 2^s into the exp's constants when |s| <= 8.
     rp.gauss_fold = 0;
-    if (sizeof(T) == 4 && rp.gauss_pow2 && ex - 1 >= -8 && ex - 1 <= 8) {
+    rp.es = exp_scaled(0);
+    if (sizeof(T) == 4 && p->kernel == CLUE_KERNEL_GAUSS && rp.gauss_pow2 && ex - 1 >= -8 && ex - 1 <= 8) {
       rp.gauss_fold = 1;
       rp.es = exp_scaled(ex - 1);
     }
@@ -245,7 +232,6 @@ WorkspaceShape workspace_shape(const BatchPlan& bp, const P* p, const Pts* pts, 
   w.event_tiles = !bp.event_order.empty();
   w.group_queries = bp.tuning.group_queries != 0;
   w.nh_blocks = nh_blocks_enabled(p, pts, bp);
-  w.separate_dm_order = separate_dm_order(p, bp, w.nh_blocks);
   w.flat_kernel = p->kernel == CLUE_KERNEL_FLAT;
   w.has_sigma = pts->sigma[0] != nullptr;
   w.has_u = pts->density_uncertainty != nullptr;
@@ -253,7 +239,7 @@ WorkspaceShape workspace_shape(const BatchPlan& bp, const P* p, const Pts* pts, 
   w.own_nh = res->nearest_higher == nullptr;
   w.own_is_seed = res->is_seed == nullptr;
   w.sorted_boxes = sorted_boxes_enabled(p);
-  w.density_morton = density_morton(p, bp);
+  w.density_morton = w.group_queries;
   return w;
 }
 
@@ -309,12 +295,6 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   b.n_items = at<int32_t>(slot, S_NITEMS);
   b.items = at<Item>(slot, S_ITEMS);
   b.qfine = bp.tuning.group_queries ? at<int32_t>(slot, S_QFINE) : nullptr;
-  b.qperm = !bp.tuning.group_queries ? nullptr
-            : density_morton(p, bp)  ? b.qfine
-                                     : at<int32_t>(slot, S_QPERM);
-  // The block scan orders its queries by qfine: no separate order for dm.
-  b.qperm_nh = separate_dm_order(p, bp, nhb) ? at<int32_t>(slot, S_QPERM_NH) : b.qperm;
-  b.qkey = bp.tuning.group_queries ? at<uint32_t>(slot, S_QKEY) : nullptr;
   b.srho = at<T>(slot, S_SRHO);
   b.skey = nhb ? nullptr : at<uint64_t>(slot, S_SKEY);
   b.snh = at<int32_t>(slot, S_SNH);
@@ -350,9 +330,6 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   ra->delta = res->delta;
   ra->event_of_cluster = nullptr;
   ra->local_ids = 0;
-  // The density stage fills the block layout's keys only from the Morton order
-  // (the block scan implies it: no Mahalanobis, weights >= 0, query grouping).
-  if (nhb && b.qperm != b.qfine) return CLUE_ERR_RUNTIME;
   return CLUE_OK;
 }
 

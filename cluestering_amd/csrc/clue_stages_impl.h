@@ -728,30 +728,15 @@ __device__ __forceinline__ void walk_tiles(const int (&lo)[D], const int (&hi)[D
 }
 
 // ---------------------------------------------------------------------------
-// Query order within a tile. A wave walks the union of its lanes' search boxes
-// and runs a candidate's kernel when any lane has it within the radius, so waves
-// of lanes with alike boxes and nearby points waste fewer slots. The points of
-// every tile with more than one wave's worth are ordered by
-//   (box class, Morton index of the point's sub-cell of the tile),
-// where the class says, per dimension (first three), whether the search box
-// reaches below and above the tile's bin; items then take 64 consecutive entries
-// of that order. Results do not depend on the order: a point's traversal is its
-// own, whichever lane runs it. k_query_order builds both stages' orders, one
-// wave per tile (below).
+// Query order within a tile. A wave pays for the candidates that any of its lanes can
+// reach, so the points of every tile with more than one wave's worth are ordered by
+// the Morton index of their sub-cell of the tile; items then take 64 consecutive
+// entries. Results do not depend on the order: a point's traversal is its own,
+// whichever lane runs it. (An order by which neighbouring tiles a point's search box
+// reaches, kept within the Morton order, measured no faster once candidates were
+// culled by the wave's box.)
 // ---------------------------------------------------------------------------
 constexpr int kQueryDims = 3;  // dimensions that enter the keys
-
-template <int D, class T>
-__device__ __forceinline__ uint32_t query_class(const GeoT<T>& g, const T (&xi)[D],
-                                                const T (&si)[D], T R, const int (&tb)[D]) {
-  int lo[D], hi[D];
-  search_box<D>(g, xi, si, R, lo, hi);
-  uint32_t c = 0;
-#pragma unroll
-  for (int d = 0; d < (D < kQueryDims ? D : kQueryDims); ++d)
-    c |= ((lo[d] < tb[d] ? 2u : 0u) | (hi[d] > tb[d] ? 1u : 0u)) << (2 * d);
-  return c;
-}
 
 // Morton index of the point's sub-cell: 8 bits over the first (up to) three
 // dimensions of the tile, bits interleaved from the most significant.
@@ -774,64 +759,6 @@ __device__ __forceinline__ uint32_t query_fine(const GeoT<T>& g, const T (&xi)[D
 #pragma unroll
     for (int d = 0; d < kD; ++d) key = (key << 1) | ((q[d] >> b) & 1u);
   return key;
-}
-
-// Stable counting sort of the points at positions [b, e) of `order` (identity
-// when NULL) by a Bits-bit key, into out[b, e). One wave; cnt is its LDS
-// counter array of 2^Bits entries. The counts need no order (one LDS atomic per
-// point); the placement visits rounds and lanes in position order and ranks equal
-// keys by ballot, so equal keys keep their input order. Placement takes four
-// rounds' positions and keys with their loads in flight together, then ranks
-// the rounds one after the other.
-template <int Bits, class KeyOf>
-__device__ __forceinline__ void wave_counting_sort(int b, int e, const int32_t* order,
-                                                   int32_t* cnt, KeyOf key_of, int32_t* out) {
-  constexpr int kKeys = 1 << Bits;
-  constexpr int kRounds = 4;
-  const int lane = lane_id();
-  for (int c = lane; c < kKeys; c += kWave) cnt[c] = 0;
-  __builtin_amdgcn_wave_barrier();
-  for (int i = b + lane; i < e; i += kWave) atomicAdd(&cnt[key_of(order ? order[i] : i)], 1);
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  int carry = b;
-  for (int c0 = 0; c0 < kKeys; c0 += kWave) {
-    const int c = c0 + lane;
-    const int v = c < kKeys ? cnt[c] : 0;
-    int x = v;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const int y = __shfl_up(x, off, 64);
-      if (lane >= off) x += y;
-    }
-    if (c < kKeys) cnt[c] = carry + x - v;
-    carry += __shfl(x, kWave - 1, 64);
-  }
-  __builtin_amdgcn_wave_barrier();
-  for (int i0 = b; i0 < e; i0 += kRounds * kWave) {
-    int sr[kRounds];
-    uint32_t kr[kRounds];
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      const int i = i0 + r * kWave + lane;
-      sr[r] = i < e ? (order ? order[i] : i) : 0;
-    }
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) kr[r] = (i0 + r * kWave + lane < e) ? key_of(sr[r]) : 0u;
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-      if (i0 + r * kWave >= e) break;  // wave-uniform
-      const bool valid = i0 + r * kWave + lane < e;
-      const uint32_t k = kr[r];
-      const uint64_t peers = match_peers(k, Bits, valid);
-      int pos = 0;
-      if (valid) pos = cnt[k] + __popcll(peers & lanemask_lt());
-      __builtin_amdgcn_wave_barrier();
-      if (valid && (peers & lanemask_lt()) == 0) cnt[k] += __popcll(peers);
-      __builtin_amdgcn_wave_barrier();
-      if (valid) out[pos] = sr[r];
-    }
-  }
 }
 
 // Wave-wide minimum and maximum of floating-point values.
@@ -999,46 +926,33 @@ __global__ __launch_bounds__(kBlock) void k_tile_boxes(const int32_t* __restrict
   }
 }
 
-// The query orders of kWaves tiles per workgroup. A tile of at most one wave's
+// The query order of kWaves tiles per workgroup. A tile of at most one wave's
 // points keeps its order (one wave each). The others are taken one after the other
 // by the whole workgroup, a counting sort in LDS by the Morton index: the dense
 // tiles, thousands of points where most tiles hold a few dozen, are what one wave
 // per tile waited for (4096-event batch: 1043 -> 789 us; one event of 2^20 points
 // in 2-D: 248 -> 89 us; of 100,000: 87 -> 28 us). Points of equal index are placed by LDS atomics, in no
 // order among themselves: no result depends on the query order or on the order
-// within the nearest-higher layout. The orders by (class, Morton) for dc (qperm)
-// and for dm (qperm_nh), where they are no aliases, then follow from stable
-// counting sorts of the Morton order, one wave each, by the classes packed into
-// qkey (dc in bits 8-13, dm in 14-19).
+// within the nearest-higher layout.
 template <int D, class T>
 __global__ __launch_bounds__(kBlock) void k_query_order(
     const RunParamsT<T> rp, const EventDesc* __restrict__ events, const Item* __restrict__ items,
     const int32_t* __restrict__ ioff, const T* __restrict__ geo, const int32_t* __restrict__ toff,
-    int n_tiles, const T* __restrict__ sx, int64_t cs, const T* __restrict__ ssig,
-    uint32_t* __restrict__ qkey, int32_t* __restrict__ qfine, int32_t* __restrict__ qperm,
-    int32_t* __restrict__ qperm_nh, T* __restrict__ hx, int64_t hs, int32_t* __restrict__ hidx,
-    T* __restrict__ hbox) {
+    int n_tiles, const T* __restrict__ sx, int64_t cs, int32_t* __restrict__ qfine,
+    T* __restrict__ hx, int64_t hs, int32_t* __restrict__ hidx, T* __restrict__ hbox) {
   constexpr int kD = D < kQueryDims ? D : kQueryDims;
   constexpr int kFineBits = (8 / kD) * kD;
-  constexpr int kClassBits = 2 * kD;
   constexpr int kFine = 1 << kFineBits;
   constexpr int kHeld = 4;  // rounds whose Morton indices stay in registers
   static_assert(kFine <= kBlock, "one counter per thread in the scan");
   __shared__ int32_t cnt[kFine];
-  __shared__ int32_t class_cnt[2][1 << kClassBits];
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
-  const bool class_dc = qperm != qfine;
-  const bool class_dm = qperm_nh != qperm && qperm_nh != qfine;
   {
     const int t = blockIdx.x * kWaves + w;
     const int b = t < n_tiles ? toff[t] : 0, e = t < n_tiles ? toff[t + 1] : 0;
     if (t < n_tiles && e - b <= kWave) {  // one item: the query order is irrelevant
-      if (b + lane < e) {
-        qfine[b + lane] = b + lane;
-        if (class_dc) qperm[b + lane] = b + lane;
-        if (class_dm) qperm_nh[b + lane] = b + lane;
-      }
+      if (b + lane < e) qfine[b + lane] = b + lane;
       if (hx) write_nh_layout<D>(t, b, e - b, nullptr, 0, 1, sx, cs, hx, hs, hidx, hbox);
     }
   }
@@ -1067,8 +981,7 @@ __global__ __launch_bounds__(kBlock) void k_query_order(
       T xi[D];
 #pragma unroll
       for (int d = 0; d < D; ++d) xi[d] = sx[d * cs + s];
-      const uint32_t fine = query_fine<D>(g, xi, tb);
-      return fine;
+      return query_fine<D>(g, xi, tb);
     };
     uint32_t held[kHeld];
 #pragma unroll
@@ -1079,19 +992,6 @@ __global__ __launch_bounds__(kBlock) void k_query_order(
     }
     for (int s = b + kHeld * kBlock + static_cast<int>(threadIdx.x); s < e; s += kBlock)
       atomicAdd(&cnt[key_of(s)], 1);
-    if (class_dc || class_dm) {
-      for (int s = b + static_cast<int>(threadIdx.x); s < e; s += kBlock) {
-        T xi[D], si[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-          xi[d] = sx[d * cs + s];
-          si[d] = rp.has_sigma ? ssig[d * cs + s] : T(0);
-        }
-        const uint32_t c_dc = class_dc ? query_class<D>(g, xi, si, rp.dc, tb) : 0u;
-        const uint32_t c_dm = class_dm ? query_class<D>(g, xi, si, rp.dm, tb) : 0u;
-        qkey[s] = (c_dc << 8) | (c_dm << 14);
-      }
-    }
     __syncthreads();
     int total;
     const int c = threadIdx.x < kFine ? cnt[threadIdx.x] : 0;
@@ -1105,14 +1005,8 @@ __global__ __launch_bounds__(kBlock) void k_query_order(
     }
     for (int s = b + kHeld * kBlock + static_cast<int>(threadIdx.x); s < e; s += kBlock)
       qfine[atomicAdd(&cnt[key_of(s)], 1)] = s;
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // qfine and qkey of the tile
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // qfine of the tile
     __syncthreads();
-    if (class_dc && w == 0)
-      wave_counting_sort<kClassBits>(b, e, qfine, class_cnt[0],
-                                     [&](int s) { return (qkey[s] >> 8) & 63u; }, qperm);
-    if (class_dm && w == 1)
-      wave_counting_sort<kClassBits>(b, e, qfine, class_cnt[1],
-                                     [&](int s) { return (qkey[s] >> 14) & 63u; }, qperm_nh);
     if (hx) write_nh_layout<D>(t, b, e - b, qfine, w, kWaves, sx, cs, hx, hs, hidx, hbox);
   }
 }
@@ -1307,7 +1201,8 @@ __device__ __forceinline__ BoxUnion<D> box_union(const int (&lo)[D], const int (
 
 template <int D>
 struct TileGroup {
-  int t, j0, j1;  // this lane's tile and its candidates
+  bool listed;    // this lane has a tile
+  int t, j0, j1;  // the tile and its candidates
   int b[D];       // its bins (past nper on a wrapped dimension)
 };
 template <int D>
@@ -1326,7 +1221,8 @@ __device__ __forceinline__ void list_tiles(const BoxUnion<D>& u, int base, int n
   }
   g->t = t_base + t;
   g->j0 = g->j1 = 0;
-  if (idx < u.tiles) {
+  g->listed = idx < u.tiles;
+  if (g->listed) {
     g->j0 = toff[g->t];
     g->j1 = toff[g->t + 1];
   }
@@ -1378,6 +1274,26 @@ __device__ __forceinline__ bool out_of_reach(const QueryBox<D, T>& q, const T (&
   } else {
     return metric_lb<D, M>(q.lo, q.hi, x, x, rp) > thr;
   }
+}
+
+// Does the lane's tile hold candidates, and can a query of the box reach its box?
+template <int D, int M, class T>
+__device__ __forceinline__ bool tile_in_reach(const TileGroup<D>& g, const QueryBox<D, T>& q,
+                                              const T* __restrict__ tbox, const RunParamsT<T>& rp,
+                                              T thr) {
+  bool reach = g.j0 < g.j1;
+  if constexpr (M != M_MAHALANOBIS) {
+    if (tbox && g.listed) {  // beside the offsets, not after them
+      T bl[D], bh[D];
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        bl[d] = tbox[static_cast<int64_t>(g.t) * 2 * D + d];
+        bh[d] = tbox[static_cast<int64_t>(g.t) * 2 * D + D + d];
+      }
+      reach = reach && !(metric_lb<D, M>(q.lo, q.hi, bl, bh, rp) > thr);
+    }
+  }
+  return reach;
 }
 
 // Compile-time loop modes of the density stage: kernel exp arguments known to be
@@ -1566,18 +1482,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
       for (int base = 0; base < u.tiles; base += kWave) {
         TileGroup<D> g;
         list_tiles(u, base, ev.nper, rp.wrapped, ev.t_base, toff, &g);
-        bool reach = g.j0 < g.j1;
-        if (M != M_MAHALANOBIS && cull && reach) {
-          T bl[D], bh[D];
-  #pragma unroll
-          for (int d = 0; d < D; ++d) {
-            bl[d] = tbox[static_cast<int64_t>(g.t) * 2 * D + d];
-            bh[d] = tbox[static_cast<int64_t>(g.t) * 2 * D + D + d];
-          }
-          if constexpr (M != M_MAHALANOBIS)
-            reach = !(metric_lb<D, M>(qb.lo, qb.hi, bl, bh, rp) > thr_in);
-        }
-        uint64_t held = ballot(reach);
+        uint64_t held = ballot(tile_in_reach<D, M>(g, qb, tbox, rp, thr_in));
         while (held) {
           const int i = __builtin_ctzll(held);
           held &= held - 1ull;
@@ -1626,7 +1531,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
     }
     if (hkey) {
       // The nearest-higher block layout takes the keys here: the lanes are the
-      // tile's points in Morton order (qperm is qfine) from a multiple of 64, so
+      // tile's points in Morton order (qfine) from a multiple of 64, so
       // lane k's point fills layout slot k of the tile and each row of 16 lanes
       // is one block, whose largest key a row reduction gives. Lanes past the
       // tile's points write the padding's key 0 up to the last block.
@@ -2386,6 +2291,12 @@ static __global__ __launch_bounds__(kBlock) void k_labels(const Chunk* __restric
   }
 }
 
+}  // namespace clue_dev
+
+#include "clue_team.h"
+
+namespace clue_dev {
+
 // ---------------------------------------------------------------------------
 // Dispatch over (D, metric, kernel).
 // ---------------------------------------------------------------------------
@@ -2412,6 +2323,7 @@ struct NeighbourLaunch {
   unsigned grid;             // one wave per work item (the grid form)
   unsigned grid_persistent;  // rp.persistent waves per CU (kernels with persistent variants)
   unsigned block;  // threads per workgroup of the neighbour stages
+  unsigned grid_team;  // one workgroup per work item (rp.team, clue_team.h)
   hipStream_t s;
 };
 
@@ -2426,7 +2338,7 @@ static void launch_density_dmk(const NeighbourLaunch<T>& L) {
   auto go = [&](auto kern, unsigned grid) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(L.block), 0, L.s, *L.rp, b.events, b.geo, b.toff,
                        b.items, b.n_items, b.sorted.x[0], L.cs, b.sorted.w, b.sorted.fw,
-                       b.sorted.sigma[0], b.sorted.tag, b.qperm, b.srho, b.skey, b.tbox,
+                       b.sorted.sigma[0], b.sorted.tag, b.qfine, b.srho, b.skey, b.tbox,
                        b.hkey, b.hbkey);
   };
   if constexpr (kPersistentBuilt<D>) {
@@ -2440,6 +2352,14 @@ static void launch_density_dmk(const NeighbourLaunch<T>& L) {
 
 template <int D, int M, class T>
 static void launch_density_dm(const NeighbourLaunch<T>& L) {
+  if (L.rp->team) {
+    const BatchBuffersT<T>& b = *L.bb;
+    hipLaunchKernelGGL((k_density_team<D, M, T>), dim3(L.grid_team), dim3(kTeam * kWave), 0, L.s,
+                       *L.rp, b.events, b.geo, b.toff, b.items, b.n_items, b.sorted.x[0], L.cs,
+                       b.sorted.w, b.sorted.fw, b.sorted.sigma[0], b.sorted.tag, b.qfine, b.tbox,
+                       b.srho, b.skey);
+    return;
+  }
   switch (L.rp->kernel) {
     case K_FLAT: launch_density_dmk<D, M, K_FLAT>(L); break;
     case K_EXP:
@@ -2465,9 +2385,16 @@ static void launch_density_dm(const NeighbourLaunch<T>& L) {
 template <int D, int M, class T>
 static void launch_nh_dm(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
+  if (L.rp->team) {
+    hipLaunchKernelGGL((k_nearest_higher_team<D, M, T>), dim3(L.grid_team), dim3(kTeam * kWave), 0,
+                       L.s, *L.rp, b.events, b.geo, b.toff, b.items, b.n_items, b.sorted.x[0], L.cs,
+                       b.sorted.sigma[0], b.sorted.u, b.sorted.tag, b.srho, b.skey, b.qfine,
+                       b.tbox, b.snh, b.sdelta);
+    return;
+  }
   hipLaunchKernelGGL((k_nearest_higher<D, M, T>), dim3(L.grid), dim3(L.block), 0, L.s, *L.rp,
                      b.events, b.geo, b.toff, b.items, b.n_items, b.sorted.x[0], L.cs,
-                     b.sorted.sigma[0], b.sorted.u, b.sorted.tag, b.srho, b.skey, b.qperm_nh,
+                     b.sorted.sigma[0], b.sorted.u, b.sorted.tag, b.srho, b.skey, b.qfine,
                      b.snh, b.sdelta);
 }
 
@@ -2567,8 +2494,7 @@ static void launch_query_order_d(const NeighbourLaunch<T>& L) {
   const unsigned grid = static_cast<unsigned>((b.n_tiles_total + kWaves - 1) / kWaves);
   hipLaunchKernelGGL((k_query_order<D, T>), dim3(grid), dim3(kBlock), 0, L.s, *L.rp, b.events,
                      b.items, b.icount, b.geo, b.toff, b.n_tiles_total, b.sorted.x[0], L.cs,
-                     b.sorted.sigma[0], b.qkey, b.qfine, b.qperm, b.qperm_nh, b.hx, b.h_stride,
-                     b.hidx, b.hbox);
+                     b.qfine, b.hx, b.h_stride, b.hidx, b.hbox);
 }
 
 template <int D, class T>
@@ -2595,7 +2521,7 @@ static void launch_tile_boxes(const NeighbourLaunch<T>& L) {
   }
 }
 
-// The query orders of both neighbour stages (qperm for dc, qperm_nh for dm).
+// The query order of both neighbour stages.
 template <class T>
 static void launch_query_order(const NeighbourLaunch<T>& L) {
   switch (L.rp->D) {
@@ -2696,9 +2622,11 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
   const int64_t pblocks = std::min<int64_t>(
       blocks, (static_cast<int64_t>(device_cus()) * std::max(rp.persistent, 0) + waves - 1) / waves);
   L.grid_persistent = static_cast<unsigned>((pblocks + kXcds - 1) / kXcds * kXcds);
+  L.grid_team =
+      static_cast<unsigned>((static_cast<int64_t>(bb.max_items) + kXcds - 1) / kXcds * kXcds);
   L.s = s;
   if (bb.tbox) launch_tile_boxes(L);    // bounds of the density stage's candidates
-  if (bb.qperm) launch_query_order(L);  // query orders of the two neighbour stages
+  if (bb.qfine) launch_query_order(L);  // query order of the two neighbour stages
 
   // (b), (c)
   mark(kStageDensity);

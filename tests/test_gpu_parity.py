@@ -389,3 +389,58 @@ def test_flat_sums_with_infinite_and_nan_weights(gpu_ctx, n, dtype):
     assert rho[0] == np.inf and rho[1] == np.inf
     assert np.isnan(rho[2]) and np.isnan(rho[3])
     np.testing.assert_array_equal(rho[4:], want[4:].astype(dtype))
+
+
+@pytest.mark.parametrize("kernel", [K.FlatKernel(0.5), K.ExponentialKernel(0.7, 1.2),
+                                    K.GaussianKernel(1.0, 1.0), K.GaussianKernel(0.8, 1.3)])
+@pytest.mark.parametrize("metric", [None, K.EuclideanMetric([1.0, 0.0]), K.ManhattanMetric(),
+                                    K.ChebyshevMetric([1.0, 2.0]), K.MahalanobisMetric(),
+                                    K.PeriodicEuclideanMetric([0.0, 40.0]),
+                                    K.PeriodicEuclideanMetric([50.0, 40.0])])
+def test_one_wave_per_item(gpu_ctx, oracle_mod, kernel, metric):
+    """A fixed tuning keeps the kernels of large launches (one wave per item) at sizes
+    that teams of waves would take."""
+    c, w = read_points("data_4096.csv")
+    rng = np.random.default_rng(5)
+    w = rng.uniform(0.5, 1.5, w.size).astype(np.float32)
+    sigma = rng.uniform(0.3, 1.0, size=c.shape).astype(np.float32) \
+        if metric is not None and metric.tag == "mahalanobis" else None
+    gpu_ctx.set_tuning(group_queries=True, xcd_chunk_log2=4, block_waves=1)
+    try:
+        _check(Case(c, w, 1.5, 10.0, 1.7, kernel=kernel, metric=metric, sigma=sigma,
+                    name=f"{kernel}-{metric}"), gpu_ctx, oracle_mod)
+    finally:
+        gpu_ctx.set_tuning()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 63, 65, 255, 256, 257, 512, 1024, 1279, 1281, 4097])
+def test_team_list_sizes(gpu_ctx, oracle_mod, n, dtype):
+    """One tile whose points all reach each other: the teams' lists fill, empty and
+    end at every boundary (8, 16, 64, 256 and 1,024 candidates and what is left)."""
+    rng = np.random.default_rng(n)
+    x = rng.normal(0, 0.4, size=(2, n)).astype(dtype)
+    w = rng.uniform(0.5, 1.5, n).astype(dtype)
+    for kernel in (K.FlatKernel(0.5), K.GaussianKernel(0.9, 1.0)):
+        case = Case(x, w, 1.0, 3.0, 1.5, kernel=kernel, points_per_tile=100000, dtype=dtype,
+                    name=f"list {n} {kernel}")
+        print(f"[case] {case.name} {np.dtype(dtype)}", flush=True)
+        assert_same(case.run_gpu(gpu_ctx), case.run_oracle(oracle_mod), case.name)
+
+
+@pytest.mark.parametrize("fixed", [False, True])
+def test_equal_tags_keep_the_first_candidate(gpu_ctx, oracle_mod, fixed):
+    """Equal user tags, coordinates on a coarse grid and unit weights: many candidates
+    agree in distance, density and tag, and the first in the reference's order wins."""
+    rng = np.random.default_rng(9)
+    n = 6000
+    x = rng.integers(0, 40, size=(2, n)).astype(np.float32)
+    w = np.ones(n, np.float32)
+    tags = rng.integers(0, 3, n).astype(np.uint32)
+    if fixed:
+        gpu_ctx.set_tuning(group_queries=True, xcd_chunk_log2=4, block_waves=1)
+    try:
+        _check(Case(x, w, 2.5, 10.0, 4.5, tags=tags, name=f"equal tags fixed={fixed}"), gpu_ctx,
+               oracle_mod)
+    finally:
+        gpu_ctx.set_tuning()
