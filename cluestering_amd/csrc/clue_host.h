@@ -23,7 +23,7 @@ using clue_dev::Item;
 using clue_dev::radix_hist_elems;
 using clue_dev::scan_temp_elems;
 
-constexpr int kChunk = 2048;  // points per chunk of the per-point grids
+constexpr int kChunk = clue_dev::kPointChunk;
 constexpr int kEvtSoloMaxPoints = 8192;  // largest lone event for the fused per-event stages
 constexpr int kDefaultPointsPerTile = 128;
 // Launches up to this many points have their neighbour stages run by teams of waves
@@ -244,7 +244,7 @@ inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) 
   bytes[S_SFW] = w.flat_kernel ? T * n : 0;
   bytes[S_SNH] = sizeof(int32_t) * n;
   bytes[S_SDELTA] = T * n;
-  bytes[S_FLAG] = w.event_tiles ? 0 : sizeof(int32_t) * n;
+  bytes[S_FLAG] = w.event_tiles ? 0 : sizeof(uint32_t) * ((n + 31) / 32);
   bytes[S_RANK] = sizeof(int32_t) * n;
   bytes[S_NSEEDS] = sizeof(int32_t) * 4;
   bytes[S_SEEDS] = sizeof(int32_t) * n;

@@ -86,11 +86,11 @@ struct BatchBuffersT {
                        // (the plain nearest-higher scan; NULL with the block layout)
   int32_t* snh;
   T* sdelta;
-  int32_t* flag;       // [n_total]
+  int32_t* flag;       // one bit per point, in input order: its seed flag (radix path)
   int32_t* event_seeds;    // [n_events] seeds per event (fused per-event seed stage)
   int32_t* event_offsets;  // [n_events] exclusive scan of event_seeds
   int32_t* iperm;          // [n_total] sorted position of every input point (fused per-event path)
-  int32_t* rank;       // [n_total]
+  int32_t* rank;       // [n_total] ranks of seeds (radix path: seeds before each word of flag)
   int32_t* n_seeds;    // [1]
   int32_t* seeds;      // [n_total]
   SortedArraysT<T> sorted;

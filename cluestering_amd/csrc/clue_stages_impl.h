@@ -237,9 +237,11 @@ template <class T>
 __global__ __launch_bounds__(kBlock) void k_gather(const GatherArgs<T> a, const RunParamsT<T> rp,
                                                    const uint32_t* __restrict__ keys,
                                                    const int32_t* __restrict__ perm, int n,
-                                                   int n_tiles_total, int32_t* __restrict__ toff) {
+                                                   int n_tiles_total, int32_t* __restrict__ toff,
+                                                   uint32_t* __restrict__ bits) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
+  if (s < (n + 31) / 32) bits[s] = 0u;  // no seeds yet (k_results)
   const int i = perm[s];
   for (int d = 0; d < rp.D; ++d) a.out.x[d][s] = a.in.x[d][i];
   const T wi = a.in.w[i];
@@ -2020,17 +2022,21 @@ __attribute__((amdgpu_waves_per_eu(D <= 2 ? 8 : 1))) void k_nh_blocks(
 }
 
 // ---------------------------------------------------------------------------
-// (d) Seed flags (ClusteringKernels.hpp:300-316) and the results in input order.
-// snh is rewritten in place as the follower link of the label stage:
-// -2 for a seed, -1 for a point without nearest-higher, else the sorted
-// position of its nearest-higher.
+// (d) Seed flags (ClusteringKernels.hpp:300-316) and the results in input order,
+// one thread per sorted point. A seed sets its bit of bits[], in input order.
+// snh is rewritten in place as the follower link of the label stage: -2 for a
+// seed, -1 for a point without nearest-higher, else the sorted position of a point
+// further up its chain. The thread follows up to kResultHops links for that; those
+// it meets may be old or already rewritten, and all lie on its own chain, so the
+// label stage's chase ends at the same point whatever order the threads run in.
 // ---------------------------------------------------------------------------
+constexpr int kResultHops = 3;
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_unpermute(
+__global__ __launch_bounds__(kBlock) void k_results(
     const RunParamsT<T> rp, int n, const int32_t* __restrict__ perm, const T* __restrict__ srho,
-    int32_t* __restrict__ snh, const T* __restrict__ sdelta, const T* __restrict__ su,
-    T* __restrict__ rho, int32_t* __restrict__ nh, T* __restrict__ delta,
-    int32_t* __restrict__ is_seed, int32_t* __restrict__ flag) {
+    int32_t* snh, const T* __restrict__ sdelta, const T* __restrict__ su, T* __restrict__ rho,
+    int32_t* __restrict__ nh, T* __restrict__ delta, int32_t* __restrict__ is_seed,
+    uint32_t* __restrict__ bits) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= n) return;
   const int i = perm[s];
@@ -2042,16 +2048,82 @@ __global__ __launch_bounds__(kBlock) void k_unpermute(
   nh[i] = h >= 0 ? perm[h] : -1;
   if (delta) delta[i] = sdelta[s];
   is_seed[i] = seed;
-  flag[i] = seed;
-  snh[s] = seed ? -2 : h;
+  if (seed) {
+    atomicOr(&bits[i >> 5], 1u << (i & 31));
+    snh[s] = -2;
+    return;
+  }
+  if (h < 0) return;
+  int l = h;
+  for (int k = 0; k < kResultHops; ++k) {
+    const int next = snh[l];
+    if (next < 0) break;
+    l = next;
+  }
+  if (l != h) snh[s] = l;
+}
+
+// Seeds before every word of bits[] (an exclusive scan of the words' bit counts) and
+// their total: up to kRankWords words by one workgroup, four consecutive words per
+// thread and row, the rows' loads all in flight together; more by k_seed_counts and
+// the general scan.
+constexpr int kRankBlock = 1024;
+constexpr int kRankRows = 8;
+constexpr int kRankWords = 4 * kRankBlock * kRankRows;
+static __global__ __launch_bounds__(kRankBlock) void k_seed_ranks(const uint32_t* __restrict__ bits,
+                                                                  int words,
+                                                                  int32_t* __restrict__ before,
+                                                                  int32_t* __restrict__ total) {
+  constexpr int kW = kRankBlock / kWave;
+  static_assert(kRankRows * kW == 2 * kWave, "two row totals per lane of the scanning wave");
+  __shared__ int32_t part[kRankRows * kW];
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  int c[kRankRows][4], incl[kRankRows];
+#pragma unroll
+  for (int r = 0; r < kRankRows; ++r)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int w = (r * kRankBlock + static_cast<int>(threadIdx.x)) * 4 + k;
+      c[r][k] = w < words ? __popc(bits[w]) : 0;
+    }
+#pragma unroll
+  for (int r = 0; r < kRankRows; ++r) {
+    incl[r] = wave_incl_scan(c[r][0] + c[r][1] + c[r][2] + c[r][3]);
+    if (lane == kWave - 1) part[r * kW + wave] = incl[r];
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int p0 = part[2 * lane], p1 = part[2 * lane + 1];
+    const int upto = wave_incl_scan(p0 + p1);
+    part[2 * lane] = upto - p0 - p1;
+    part[2 * lane + 1] = upto - p1;
+    if (lane == kWave - 1) *total = upto;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kRankRows; ++r) {
+    int run = part[r * kW + wave] + incl[r] - (c[r][0] + c[r][1] + c[r][2] + c[r][3]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int w = (r * kRankBlock + static_cast<int>(threadIdx.x)) * 4 + k;
+      if (w < words) before[w] = run;
+      run += c[r][k];
+    }
+  }
+}
+static __global__ __launch_bounds__(kBlock) void k_seed_counts(const uint32_t* __restrict__ bits,
+                                                               int words,
+                                                               int32_t* __restrict__ count) {
+  const int w = blockIdx.x * kBlock + threadIdx.x;
+  if (w < words) count[w] = __popc(bits[w]);
 }
 
 // ---------------------------------------------------------------------------
 // (d fused) With the per-event tile build, one workgroup per event does the seed
-// stage of k_unpermute, numbers the event's seeds in input order through a bit
+// stage of k_results, numbers the event's seeds in input order through a bit
 // per point in LDS (one popcount scan over the bits: the rank of a seed among
 // the event's seeds, stored in rank[i]), counts them (event_seeds[e]) and
-// shortens the follower links with the pointer-jumping passes of k_link_jump.
+// shortens the follower links by pointer jumping.
 // The seeds of earlier events are added by the label stage from an exclusive
 // scan of event_seeds. The seed flags and links are settled in sorted order;
 // the results are then written in input order, each point's sorted values
@@ -2174,8 +2246,9 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
       *lone_total = total;
     }
   }
-  // Pointer jumping on the event's links (as k_link_jump; any interleaving of the
-  // updates leaves every link on its own chain).
+  // Pointer jumping on the event's links: a pass replaces a link by its target's link
+  // when that target is itself a follower, which halves every chain (at least); any
+  // interleaving of the updates leaves every link on its own chain.
   if (in_lds) {
     // A link is a position, a seed's code or -1 (the end of an outlier chain), and
     // every point shares the label of what its link names; replacing a position
@@ -2220,46 +2293,24 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
 // where a chain stays among neighbouring tiles of one event. An event occupies
 // the same range of positions in input and sorted order.
 // ---------------------------------------------------------------------------
-// Pointer jumping on the follower links before the chase: each pass replaces a
-// link by its target's link when that target is itself a follower, so a pass
-// halves every chain (at least) and the chase's dependent loads shrink with it.
-// Every link still points to an ancestor on the same chain, whatever order the
-// threads run in, so the chase ends at the same seed or outlier.
-static __global__ __launch_bounds__(kBlock) void k_link_jump(int32_t* __restrict__ link, int n) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  const int l = link[s];
-  if (l < 0) return;
-  const int l2 = link[l];
-  if (l2 >= 0) link[s] = l2;
-}
-
-// rank[i] of a seed i is its global rank (seeds of the whole batch before it in
-// input order), or, with event_offsets, its rank within its event, to which the
-// seeds of the earlier events (event_offsets[e]) are added here. Chains are
-// chased from sorted positions, so their first links are read in order and the
+// After the fused seed stage, rank[i] of a seed i is its rank within its event, to
+// which the seeds of the earlier events (event_offsets[e]) are added here. Chains
+// are chased from sorted positions, so their first links are read in order and the
 // label stores scatter within each event (chasing from input order instead
 // stores in order but reads twice the bytes, for the same time on MI355X).
 // An event the fused seed stage resolved in LDS (at most kEvtLdsLinks points)
 // has its labels within the event in cluster[] already and its seed list in
 // rank[p_off, p_off + event_seeds[e]): only the offset is added.
-static __global__ __launch_bounds__(kBlock) void k_labels(const Chunk* __restrict__ chunks,
-                                                   const EventDesc* __restrict__ events,
-                                                   const int32_t* __restrict__ perm,
-                                                   const int32_t* __restrict__ link,
-                                                   const int32_t* __restrict__ rank,
-                                                   const int32_t* __restrict__ event_offsets,
-                                                   const int32_t* __restrict__ event_seeds,
-                                                   int32_t* __restrict__ cluster,
-                                                   int32_t* __restrict__ seeds,
-                                                   int32_t* __restrict__ event_of_cluster,
-                                                   int local_ids) {
+static __global__ __launch_bounds__(kBlock) void k_event_labels(
+    const Chunk* __restrict__ chunks, const EventDesc* __restrict__ events,
+    const int32_t* __restrict__ perm, const int32_t* __restrict__ link,
+    const int32_t* __restrict__ rank, const int32_t* __restrict__ event_offsets,
+    const int32_t* __restrict__ event_seeds, int32_t* __restrict__ cluster,
+    int32_t* __restrict__ seeds, int32_t* __restrict__ event_of_cluster, int local_ids) {
   const Chunk ch = chunks[blockIdx.x];
   const EventDesc ev = events[ch.event];
-  // Seeds of the earlier events: added to local ranks, subtracted from global
-  // ranks with per-event numbering.
-  const int first = event_offsets ? event_offsets[ch.event] : rank[ev.p_off];
-  if (event_offsets && ev.n <= kEvtLdsLinks) {
+  const int first = event_offsets[ch.event];
+  if (ev.n <= kEvtLdsLinks) {
     const int count = event_seeds[ch.event];
     for (int p = ch.begin + threadIdx.x; p < ch.end; p += kBlock) {
       const int c = cluster[p];
@@ -2272,7 +2323,6 @@ static __global__ __launch_bounds__(kBlock) void k_labels(const Chunk* __restric
     }
     return;
   }
-  const int add = event_offsets ? first : 0;
   const int sub = local_ids ? first : 0;
   for (int s = ch.begin + threadIdx.x; s < ch.end; s += kBlock) {
     int cur = s;
@@ -2282,12 +2332,42 @@ static __global__ __launch_bounds__(kBlock) void k_labels(const Chunk* __restric
       nx = link[cur];
     }
     const int i = perm[s];
-    const int c = (nx == -2) ? rank[perm[cur]] + add : -1;
+    const int c = (nx == -2) ? rank[perm[cur]] + first : -1;
     cluster[i] = c >= 0 ? c - sub : -1;
     if (cur == s && nx == -2) {
       seeds[c] = i;
       if (event_of_cluster) event_of_cluster[c] = ev.index;
     }
+  }
+}
+
+// The same after k_results: a seed's rank over the whole batch is the number of seed
+// bits before its own.
+static __global__ __launch_bounds__(kBlock) void k_labels(
+    const Chunk* __restrict__ chunks, const EventDesc* __restrict__ events,
+    const int32_t* __restrict__ perm, const int32_t* __restrict__ link,
+    const uint32_t* __restrict__ bits, const int32_t* __restrict__ before,
+    int32_t* __restrict__ cluster, int32_t* __restrict__ seeds,
+    int32_t* __restrict__ event_of_cluster, int local_ids) {
+  auto rank = [&](int i) {
+    return before[i >> 5] + __popc(bits[i >> 5] & ((1u << (i & 31)) - 1u));
+  };
+  const Chunk ch = chunks[blockIdx.x / (kPointChunk / kBlock)];
+  const int s = ch.begin + (blockIdx.x % (kPointChunk / kBlock)) * kBlock + threadIdx.x;
+  if (s >= ch.end) return;
+  const EventDesc ev = events[ch.event];
+  int cur = s;
+  int nx = link[cur];
+  while (nx >= 0) {
+    cur = nx;
+    nx = link[cur];
+  }
+  const int i = perm[s];
+  const int c = (nx == -2) ? rank(perm[cur]) : -1;
+  cluster[i] = c >= 0 ? c - (local_ids ? rank(ev.p_off) : 0) : -1;
+  if (cur == s && nx == -2) {
+    seeds[c] = i;
+    if (event_of_cluster) event_of_cluster[c] = ev.index;
   }
 }
 
@@ -2593,7 +2673,8 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
   ga.out = bb.sorted;
   ga.cs = 0;
   hipLaunchKernelGGL(k_gather<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, ga, rp, skeys,
-                     sperm, n, bb.n_tiles_total, bb.toff);
+                     sperm, n, bb.n_tiles_total, bb.toff,
+                     reinterpret_cast<uint32_t*>(bb.flag));
   }
   if (bb.n_tiles_total <= kItemsOneBlockTiles) {
     hipLaunchKernelGGL(k_items_one_block, dim3(1), dim3(kBlock), 0, s, bb.toff, bb.n_tiles_total,
@@ -2645,19 +2726,28 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
                        out.cluster);
     if (!lone) scan_exclusive(bb.event_seeds, bb.event_offsets, bb.n_events, bb.scan_tmp, bb.n_seeds, s);
     mark(kStageLabels);
+    hipLaunchKernelGGL(k_event_labels, dim3(bb.n_chunks), dim3(kBlock), 0, s, bb.chunks, bb.events,
+                       bb.sorted.perm, bb.snh, bb.rank, bb.event_offsets, bb.event_seeds,
+                       out.cluster, bb.seeds, out.event_of_cluster, out.local_ids);
   } else {
-    hipLaunchKernelGGL(k_unpermute<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, n,
+    const int words = (n + 31) / 32;
+    uint32_t* bits = reinterpret_cast<uint32_t*>(bb.flag);
+    hipLaunchKernelGGL(k_results<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, n,
                        bb.sorted.perm, bb.srho, bb.snh, bb.sdelta, bb.sorted.u, out.rho, out.nh,
-                       out.delta, out.is_seed, bb.flag);
-    scan_exclusive(bb.flag, bb.rank, n, bb.scan_tmp, bb.n_seeds, s);
+                       out.delta, out.is_seed, bits);
+    if (words <= kRankWords) {
+      hipLaunchKernelGGL(k_seed_ranks, dim3(1), dim3(kRankBlock), 0, s, bits, words, bb.rank,
+                         bb.n_seeds);
+    } else {
+      hipLaunchKernelGGL(k_seed_counts, dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
+                         bits, words, bb.rank);
+      scan_exclusive(bb.rank, bb.rank, words, bb.scan_tmp, bb.n_seeds, s);
+    }
     mark(kStageLabels);
-    for (int pass = 0; pass < kLinkJumpPasses; ++pass)
-      hipLaunchKernelGGL(k_link_jump, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, bb.snh, n);
+    hipLaunchKernelGGL(k_labels, dim3(bb.n_chunks * (kPointChunk / kBlock)), dim3(kBlock), 0, s,
+                       bb.chunks, bb.events, bb.sorted.perm, bb.snh, bits, bb.rank, out.cluster,
+                       bb.seeds, out.event_of_cluster, out.local_ids);
   }
-  hipLaunchKernelGGL(k_labels, dim3(bb.n_chunks), dim3(kBlock), 0, s, bb.chunks, bb.events,
-                     bb.sorted.perm, bb.snh, bb.rank,
-                     bb.event_order ? bb.event_offsets : nullptr, bb.event_seeds,
-                     out.cluster, bb.seeds, out.event_of_cluster, out.local_ids);
   mark(kNumStages);
 }
 

@@ -21,6 +21,8 @@ constexpr int kEvtMaxTiles = 1024;
 // Largest event the fused per-event stages take (one bit per point in LDS).
 constexpr int kEvtMaxPoints = 1 << 17;
 
+constexpr int kPointChunk = 2048;  // points per chunk of the per-point grids
+
 // Workspace sizes of the scan and radix-sort primitives (clue_primitives.hip),
 // here so that host-only code sizes workspaces exactly as the device path does.
 constexpr int kScanTileElems = 4096;  // elements per block of the exclusive scan
