@@ -86,9 +86,8 @@ __global__ __launch_bounds__(kBlock) void k_assoc_offsets(const uint32_t* __rest
 }  // namespace
 
 void assoc_scratch_elems(int64_t n, int64_t* hist_elems, int64_t* scan_elems) {
-  const int64_t hist = radix_hist_elems(n);
-  *hist_elems = hist;
-  *scan_elems = std::max(scan_temp_elems(n), scan_temp_elems(hist)) + 16;
+  *hist_elems = radix_hist_elems((n + kRsTileKeys - 1) / kRsTileKeys);
+  *scan_elems = scan_temp_elems(n) + 16;
 }
 
 hipError_t assoc_stats(const int32_t* keys, int n, int32_t* stats_dev, hipStream_t s) {
@@ -107,7 +106,7 @@ hipError_t assoc_build(const int32_t* keys, int n, int bins, const AssocScratch&
     int bits = 0;
     while ((int64_t(1) << bits) <= bins) ++bits;  // keys lie in [0, bins]
     bool in_first = true;
-    radix_sort_pairs(w.k0, w.v0, w.k1, w.v1, n, bits, w.hist, w.scan, &in_first, s);
+    radix_sort_pairs(w.k0, w.v0, w.k1, w.v1, n, bits, w.hist, nullptr, 0, &in_first, s);
     const uint32_t* sk = in_first ? w.k0 : w.k1;
     const int32_t* sv = in_first ? w.v0 : w.v1;
     hipLaunchKernelGGL(k_assoc_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0,

@@ -74,6 +74,7 @@ struct BatchPlan {
   int64_t max_items = 0;
   int key_bits = 0;
   bool team = false;  // neighbour stages by teams of waves
+  int ext_group = 1;  // chunks per result of the extremes stage
   clue_tuning tuning{};
 };
 
@@ -167,6 +168,10 @@ inline clue_status plan_batch(int D, int points_per_tile, const uint32_t* sizes,
                        [&](int32_t a, int32_t b) { return bp->events[a].n > bp->events[b].n; });
   }
   bp->tuning = fixed ? *fixed : table_tuning(D, off, static_cast<int64_t>(bp->events.size()));
+  // At most 512 results per event: every workgroup of the key stage reads them all.
+  int64_t largest = 0;
+  for (const EventDesc& ev : bp->events) largest = std::max<int64_t>(largest, ev.n);
+  bp->ext_group = static_cast<int>(std::max<int64_t>(1, (largest + 512 * kChunk - 1) / (512 * kChunk)));
   // A fixed tuning keeps one wave per item.
   const int64_t mean = bp->events.empty() ? 0 : off / static_cast<int64_t>(bp->events.size());
   bp->team = !fixed && off <= (mean < kTeamSmallEvent && bp->events.size() > 1 ? kTeamMaxPointsSmall
@@ -189,6 +194,7 @@ struct WorkspaceShape {
   int64_t chunks = 0;
   int64_t tiles = 0;        // sum of nper^D
   int64_t max_items = 0;
+  bool team = false;               // neighbour stages by teams of waves
   bool event_tiles = false;        // the fused per-event tile build (no radix-sort buffers)
   bool group_queries = false;
   bool separate_dm_order = false;  // dm != dc and the plain nearest-higher scan
@@ -207,9 +213,9 @@ struct WorkspaceShape {
 inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) {
   std::memset(bytes, 0, sizeof(bytes));
   const int64_t n = w.n, NT = w.tiles;
-  const int64_t hist = radix_hist_elems(n);
+  const int64_t hist = radix_hist_elems(w.chunks);
   const int64_t scan_elems =
-      std::max({scan_temp_elems(n), scan_temp_elems(hist), scan_temp_elems(NT)}) + 16;
+      std::max({scan_temp_elems(n), scan_temp_elems(w.events), scan_temp_elems(NT)}) + 16;
   const int64_t stride = (n + 63) / 64 * 64;
   const int64_t h_blocks = w.nh_blocks ? (n + clue_dev::kNhBlock - 1) / clue_dev::kNhBlock + NT + 1 : 0;
   const int64_t h_slots = h_blocks * clue_dev::kNhBlock;
@@ -217,7 +223,7 @@ inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) 
   const size_t D = static_cast<size_t>(w.D);
   bytes[S_EVENTS] = sizeof(EventDesc) * w.events;
   bytes[S_CHUNKS] = sizeof(Chunk) * w.chunks;
-  bytes[S_EXT] = w.event_tiles ? 0 : static_cast<size_t>(w.key_bytes) * w.events * D * 2;
+  bytes[S_EXT] = w.event_tiles ? 0 : static_cast<size_t>(w.key_bytes) * w.chunks * D * 2;
   bytes[S_GEO] = T * w.events * 3 * D;
   bytes[S_K0] = bytes[S_K1] = w.event_tiles ? 0 : sizeof(uint32_t) * n;
   bytes[S_V0] = bytes[S_V1] = w.event_tiles ? 0 : sizeof(int32_t) * n;
@@ -227,7 +233,7 @@ inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) 
   bytes[S_IPERM] = w.event_tiles ? sizeof(int32_t) * n : 0;
   bytes[S_SCAN] = sizeof(int32_t) * scan_elems;
   bytes[S_TOFF] = sizeof(int32_t) * (NT + 1);
-  bytes[S_ICOUNT] = sizeof(int32_t) * NT;
+  bytes[S_ICOUNT] = w.team ? 0 : sizeof(int32_t) * NT;
   bytes[S_NITEMS] = sizeof(int32_t) * 32;  // item count, then the work-item queue counters
   bytes[S_ITEMS] = sizeof(Item) * w.max_items;
   bytes[S_QPERM] = (w.group_queries && !w.density_morton) ? sizeof(int32_t) * n : 0;

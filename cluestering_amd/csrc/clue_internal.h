@@ -13,8 +13,20 @@ namespace clue_dev {
 // total (device, may be NULL) receives the sum.
 void scan_exclusive(const int32_t* in, int32_t* out, int64_t n, int32_t* temp, int32_t* total,
                     hipStream_t s);
+// Stable radix sort of (key, value) by the low key_bits bits, in passes of
+// radix_plan(key_bits).bits. Blocks take the chunks given (contiguous ranges in order
+// that cover [0, n)), or kRsTileKeys keys each (chunks NULL). With chunks the caller
+// has counted the first pass's digits into hist ([digit][chunk]) and the values are the
+// keys' places; without, the values are v0 and the sort counts for itself. hist:
+// radix_hist_elems(n_blocks) ints. The result is in (k0, v0) or (k1, v1).
+struct RadixPlan {
+  int bits;    // of a digit
+  int passes;
+};
+RadixPlan radix_plan(int key_bits);
 void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int64_t n, int key_bits,
-                      int32_t* hist, int32_t* scan_temp, bool* in_first, hipStream_t s);
+                      int32_t* hist, const Chunk* chunks, int n_chunks, bool* in_first,
+                      hipStream_t s);
 
 // ---- stages (clue_stages_impl.h, instantiated in clue_stages_f32.hip / _f64.hip) ----
 
@@ -67,7 +79,8 @@ struct BatchBuffersT {
   const EventDesc* events;
   const int32_t* event_order;  // events largest first for the fused tile build; NULL: radix path
   const Chunk* chunks;
-  typename FloatBits<T>::Int* ext;  // [E][D][2] ordered-integer extremes
+  typename FloatBits<T>::Int* ext;  // [n_chunks][D][2] ordered-integer extremes
+  int32_t ext_group;                // chunks per result of the extremes
   T* geo;                           // [E][3][D] mn, mx, side
   uint32_t* keys0;
   int32_t* vals0;
@@ -76,8 +89,8 @@ struct BatchBuffersT {
   int32_t* rs_hist;
   int32_t* scan_tmp;
   int32_t* toff;       // [n_tiles_total + 1]
-  int32_t* icount;     // [n_tiles_total]
-  int32_t* n_items;    // [1]
+  int32_t* icount;     // [n_tiles_total] first item of every tile; NULL: from the offsets (teams)
+  int32_t* n_items;    // number of items (with icount), then the work-item queue counters
   Item* items;         // [max_items]
   int32_t* qfine;      // [n_total] query order of both neighbour stages, the Morton order
                        // within tiles; NULL = sorted order

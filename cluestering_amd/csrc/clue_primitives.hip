@@ -2,6 +2,8 @@
 // LSD radix sort of (key, value) pairs. No rocPRIM/rocThrust.
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 #include "clue_device.h"
 #include "clue_internal.h"
 
@@ -125,109 +127,176 @@ void scan_exclusive(const int32_t* in, int32_t* out, int64_t n, int32_t* temp, i
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort of (uint32 key, int32 value), 8-bit digits.
+// Stable LSD radix sort of (uint32 key, int32 value), digits of up to 10 bits.
 //
-// Each block owns a contiguous range of kRsTile keys; each of its four waves owns a
-// contiguous quarter, walked in rounds of 64. Within a round, lanes with the same
-// digit are found with one ballot per digit bit and ranked by lane order; per-wave
-// digit counters live in LDS. Ranges, rounds and lanes are all visited in index
-// order, so the pass is stable.
+// Each block owns a contiguous range of at most kRsTile keys; each of its sixteen
+// waves owns a contiguous sixteenth, walked in rounds of 64 (two: a wave alone takes
+// 23 us for the sixteen rounds of a 256-thread block). Within a round, lanes with the
+// same digit are found with one ballot per digit bit and ranked by lane order;
+// per-wave digit counters live in LDS. Ranges, rounds and lanes are all visited in
+// index order, so the pass is stable. Between the counts and the placement one
+// workgroup per digit scans the digit's counts over the blocks; the digits' totals
+// are scanned by every placing block for itself.
 // ---------------------------------------------------------------------------
-constexpr int kRsBits = 8;
-constexpr int kRsBins = 1 << kRsBits;
-constexpr int kRsRounds = 16;
-constexpr int kRsWaveKeys = kWave * kRsRounds;
-constexpr int kRsTile = kRsWaveKeys * kWavesPerBlock;  // 4096
-static_assert(kRsTile == kRsTileKeys && kRsBins == kRsDigitBins, "radix workspace sizing");
+constexpr int kRsWaves = 16;
+constexpr int kRsBlock = kRsWaves * kWave;
+constexpr int kRsTile = kRsTileKeys;
+constexpr int kRsRounds = kRsTile / kRsBlock;
+static_assert(kRsMaxBins <= kRsBlock, "one digit per thread in the scan of the totals");
 
-__global__ __launch_bounds__(kBlock) void k_rs_hist(const uint32_t* __restrict__ keys, int64_t n,
-                                                    int shift, int64_t nblocks,
-                                                    int32_t* __restrict__ hist) {
-  __shared__ int cnt[kRsBins];
-  for (int k = threadIdx.x; k < kRsBins; k += kBlock) cnt[k] = 0;
-  __syncthreads();
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kRsTile;
-  for (int k = threadIdx.x; k < kRsTile; k += kBlock) {
-    const int64_t i = base + k;
-    if (i < n) atomicAdd(&cnt[(keys[i] >> shift) & (kRsBins - 1)], 1);
+__device__ __forceinline__ void rs_range(const Chunk* chunks, int64_t n, int64_t* begin,
+                                         int64_t* end) {
+  if (chunks) {
+    *begin = chunks[blockIdx.x].begin;
+    *end = chunks[blockIdx.x].end;
+  } else {
+    *begin = static_cast<int64_t>(blockIdx.x) * kRsTile;
+    *end = *begin + kRsTile < n ? *begin + kRsTile : n;
   }
-  __syncthreads();
-  for (int d = threadIdx.x; d < kRsBins; d += kBlock) hist[d * nblocks + blockIdx.x] = cnt[d];
 }
 
-__global__ __launch_bounds__(kBlock) void k_rs_scatter(const uint32_t* __restrict__ kin,
-                                                       const int32_t* __restrict__ vin,
-                                                       uint32_t* __restrict__ kout,
-                                                       int32_t* __restrict__ vout, int64_t n,
-                                                       int shift, int digit_bits, int64_t nblocks,
-                                                       const int32_t* __restrict__ scanned) {
-  __shared__ int cnt[kWavesPerBlock][kRsBins];
+// hist[digit][block]
+__global__ __launch_bounds__(kBlock) void k_rs_hist(const uint32_t* __restrict__ keys, int64_t n,
+                                                    const Chunk* __restrict__ chunks, int shift,
+                                                    int bits, int32_t* __restrict__ hist) {
+  __shared__ int cnt[kRsMaxBins];
+  const int bins = 1 << bits;
+  for (int k = threadIdx.x; k < bins; k += kBlock) cnt[k] = 0;
+  __syncthreads();
+  int64_t b, e;
+  rs_range(chunks, n, &b, &e);
+  for (int64_t i = b + threadIdx.x; i < e; i += kBlock)
+    atomicAdd(&cnt[(keys[i] >> shift) & (bins - 1)], 1);
+  __syncthreads();
+  for (int d = threadIdx.x; d < bins; d += kBlock)
+    hist[static_cast<int64_t>(d) * gridDim.x + blockIdx.x] = cnt[d];
+}
+
+// One workgroup per digit: its counts become an exclusive scan over the blocks, and
+// total[digit] their sum.
+__global__ __launch_bounds__(kBlock) void k_rs_rows(int32_t* __restrict__ hist, int64_t nblocks,
+                                                    int32_t* __restrict__ total) {
+  int32_t* row = hist + static_cast<int64_t>(blockIdx.x) * nblocks;
+  int carry = 0;
+  for (int64_t base = 0; base < nblocks; base += kBlock * 4) {
+    int v[4], sum = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t i = base + threadIdx.x * 4 + k;
+      v[k] = i < nblocks ? row[i] : 0;
+      sum += v[k];
+    }
+    int tot;
+    int run = carry + block_excl_scan(sum, &tot);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t i = base + threadIdx.x * 4 + k;
+      if (i < nblocks) row[i] = run;
+      run += v[k];
+    }
+    carry += tot;
+  }
+  if (threadIdx.x == 0) total[blockIdx.x] = carry;
+}
+
+// MaxBits: room for the counters (16 KB of LDS at 8 bits, 64 KB at 10).
+template <int MaxBits>
+__global__ __launch_bounds__(kRsBlock) void k_rs_scatter(
+    const uint32_t* __restrict__ kin, const int32_t* __restrict__ vin, uint32_t* __restrict__ kout,
+    int32_t* __restrict__ vout, int64_t n, const Chunk* __restrict__ chunks, int shift, int bits,
+    const int32_t* __restrict__ rows, const int32_t* __restrict__ total) {
+  __shared__ int cnt[kRsWaves << MaxBits];  // [kRsWaves][bins]
+  const int bins = 1 << bits;
   const int w = threadIdx.x / kWave;
   const int l = lane_id();
-  for (int k = threadIdx.x; k < kWavesPerBlock * kRsBins; k += kBlock) (&cnt[0][0])[k] = 0;
-  __syncthreads();
-  const int64_t wbase = static_cast<int64_t>(blockIdx.x) * kRsTile + w * kRsWaveKeys;
-  const uint64_t lt = lanemask_lt();
-  // Phase A: per-wave digit counts.
+  int64_t b, e;
+  rs_range(chunks, n, &b, &e);
+  const int64_t wb = b + static_cast<int64_t>(w) * (kRsTile / kRsWaves);
+  uint32_t key[kRsRounds];
+  uint64_t peers[kRsRounds];
+#pragma unroll
   for (int r = 0; r < kRsRounds; ++r) {
-    const int64_t i = wbase + r * kWave + l;
-    const bool valid = i < n;
-    const uint32_t dgt = valid ? (kin[i] >> shift) & (kRsBins - 1) : 0u;
-    const uint64_t peers = match_peers(dgt, digit_bits, valid);
-    if (valid && (peers & lt) == 0) cnt[w][dgt] += __popcll(peers);
+    const int64_t i = wb + r * kWave + l;
+    key[r] = i < e ? kin[i] : 0u;
+  }
+  const int d0 = static_cast<int>(threadIdx.x);
+  const int mine = d0 < bins ? total[d0] : 0;
+  const int row = d0 < bins ? rows[static_cast<int64_t>(d0) * gridDim.x + blockIdx.x] : 0;
+  for (int k = threadIdx.x; k < kRsWaves * bins; k += kRsBlock) cnt[k] = 0;
+  int all;
+  const int before = block_excl_scan<kRsBlock>(mine, &all);  // keys of smaller digits
+  const uint64_t lt = lanemask_lt();
+  int* my = cnt + w * bins;
+  // Per-wave digit counts.
+#pragma unroll
+  for (int r = 0; r < kRsRounds; ++r) {
+    const bool valid = wb + r * kWave + l < e;
+    const uint32_t dgt = (key[r] >> shift) & (bins - 1);
+    peers[r] = match_peers(dgt, bits, valid);
+    if (valid && (peers[r] & lt) == 0) my[dgt] += __popcll(peers[r]);
+    __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
   // Per digit: global offset of this block, then the waves in order.
-  for (int d = threadIdx.x; d < kRsBins; d += kBlock) {
-    int run = scanned[d * nblocks + blockIdx.x];
+  if (d0 < bins) {
+    int run = before + row;
 #pragma unroll
-    for (int k = 0; k < kWavesPerBlock; ++k) {
-      const int c = cnt[k][d];
-      cnt[k][d] = run;
+    for (int k = 0; k < kRsWaves; ++k) {
+      const int c = cnt[k * bins + d0];
+      cnt[k * bins + d0] = run;
       run += c;
     }
   }
   __syncthreads();
-  // Phase B: place keys.
+  // Place keys.
+#pragma unroll
   for (int r = 0; r < kRsRounds; ++r) {
-    const int64_t i = wbase + r * kWave + l;
-    const bool valid = i < n;
-    const uint32_t key = valid ? kin[i] : 0u;
-    const uint32_t dgt = (key >> shift) & (kRsBins - 1);
-    const uint64_t peers = match_peers(dgt, digit_bits, valid);
+    const int64_t i = wb + r * kWave + l;
+    const bool valid = i < e;
+    const uint32_t dgt = (key[r] >> shift) & (bins - 1);
     int pos = 0;
-    if (valid) pos = cnt[w][dgt] + __popcll(peers & lt);
+    if (valid) pos = my[dgt] + __popcll(peers[r] & lt);
     __builtin_amdgcn_wave_barrier();
-    if (valid && (peers & lt) == 0) cnt[w][dgt] += __popcll(peers);
+    if (valid && (peers[r] & lt) == 0) my[dgt] += __popcll(peers[r]);
+    __builtin_amdgcn_wave_barrier();
     if (valid) {
-      kout[pos] = key;
-      vout[pos] = vin[i];
+      kout[pos] = key[r];
+      vout[pos] = vin ? vin[i] : static_cast<int32_t>(i);
     }
   }
 }
 
-// Sorts (keys, vals) by the low `key_bits` bits of the keys. The result ends in
-// (k0, v0) or (k1, v1); *in_first receives true when it is (k0, v0).
+RadixPlan radix_plan(int key_bits) {
+  RadixPlan p;
+  p.passes = key_bits <= 0 ? 1 : (key_bits + kRsMaxBits - 1) / kRsMaxBits;
+  p.bits = key_bits <= 0 ? 1 : (key_bits + p.passes - 1) / p.passes;
+  return p;
+}
+
 void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int64_t n, int key_bits,
-                      int32_t* hist, int32_t* scan_temp, bool* in_first, hipStream_t s) {
+                      int32_t* hist, const Chunk* chunks, int n_chunks, bool* in_first,
+                      hipStream_t s) {
   *in_first = true;
   if (n <= 0) return;
-  const int64_t nblocks = (n + kRsTile - 1) / kRsTile;
+  const RadixPlan plan = radix_plan(key_bits);
+  const unsigned nblocks =
+      chunks ? static_cast<unsigned>(n_chunks) : static_cast<unsigned>((n + kRsTile - 1) / kRsTile);
+  const int bins = 1 << plan.bits;
+  int32_t* total = hist + static_cast<int64_t>(bins) * nblocks;
   uint32_t *ka = k0, *kb = k1;
   int32_t *va = v0, *vb = v1;
-  for (int shift = 0; shift < key_bits; shift += kRsBits) {
-    const int bits = key_bits - shift < kRsBits ? key_bits - shift : kRsBits;
-    hipLaunchKernelGGL(k_rs_hist, dim3(static_cast<unsigned>(nblocks)), dim3(kBlock), 0, s, ka, n,
-                       shift, nblocks, hist);
-    scan_exclusive(hist, hist, kRsBins * nblocks, scan_temp, nullptr, s);
-    hipLaunchKernelGGL(k_rs_scatter, dim3(static_cast<unsigned>(nblocks)), dim3(kBlock), 0, s, ka,
-                       va, kb, vb, n, shift, bits, nblocks, hist);
-    uint32_t* tk = ka;
-    ka = kb;
-    kb = tk;
-    int32_t* tv = va;
-    va = vb;
-    vb = tv;
+  for (int pass = 0; pass < plan.passes; ++pass) {
+    const int shift = pass * plan.bits;
+    if (!chunks || pass > 0)
+      hipLaunchKernelGGL(k_rs_hist, dim3(nblocks), dim3(kBlock), 0, s, ka, n, chunks, shift,
+                         plan.bits, hist);
+    hipLaunchKernelGGL(k_rs_rows, dim3(static_cast<unsigned>(bins)), dim3(kBlock), 0, s, hist,
+                       static_cast<int64_t>(nblocks), total);
+    hipLaunchKernelGGL(plan.bits <= 8 ? k_rs_scatter<8> : k_rs_scatter<kRsMaxBits>, dim3(nblocks),
+                       dim3(kRsBlock), 0, s, ka, (chunks && pass == 0) ? nullptr : va, kb, vb, n,
+                       chunks, shift, plan.bits, hist, total);
+    std::swap(ka, kb);
+    std::swap(va, vb);
     *in_first = !*in_first;
   }
 }

@@ -114,6 +114,7 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
   rp.block_waves = bp.tuning.block_waves > 0 ? bp.tuning.block_waves : 4;
   rp.persistent = bp.tuning.persistent > 0 ? bp.tuning.persistent : 0;
   rp.team = bp.team ? 1 : 0;
+  rp.max_items = static_cast<int32_t>(bp.max_items);
   rp.nh_blocks = nh_blocks_enabled(p, pts, bp) ? 1 : 0;
   rp.cull = weights_not_negative(p) ? 1 : 0;
   rp.D = p->ndim;
@@ -229,6 +230,7 @@ WorkspaceShape workspace_shape(const BatchPlan& bp, const P* p, const Pts* pts, 
   w.chunks = static_cast<int64_t>(bp.chunks.size());
   w.tiles = bp.n_tiles_total;
   w.max_items = bp.max_items;
+  w.team = bp.team;
   w.event_tiles = !bp.event_order.empty();
   w.group_queries = bp.tuning.group_queries != 0;
   w.nh_blocks = nh_blocks_enabled(p, pts, bp);
@@ -283,6 +285,7 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   b.event_order = bp.event_order.empty() ? nullptr : at<int32_t>(slot, S_EORDER);
   b.chunks = at<Chunk>(slot, S_CHUNKS);
   b.ext = at<I>(slot, S_EXT);
+  b.ext_group = bp.ext_group;
   b.geo = at<T>(slot, S_GEO);
   b.keys0 = at<uint32_t>(slot, S_K0);
   b.vals0 = at<int32_t>(slot, S_V0);
@@ -291,7 +294,7 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   b.rs_hist = at<int32_t>(slot, S_HIST);
   b.scan_tmp = at<int32_t>(slot, S_SCAN);
   b.toff = at<int32_t>(slot, S_TOFF);
-  b.icount = at<int32_t>(slot, S_ICOUNT);
+  b.icount = bp.team ? nullptr : at<int32_t>(slot, S_ICOUNT);
   b.n_items = at<int32_t>(slot, S_NITEMS);
   b.items = at<Item>(slot, S_ITEMS);
   b.qfine = bp.tuning.group_queries ? at<int32_t>(slot, S_QFINE) : nullptr;

@@ -65,12 +65,12 @@ __device__ __forceinline__ int xcd_block(int b, int nb, int log2_chunk) {
 // workgroup mapped by xcd_block). In the persistent form (rp.persistent waves per
 // CU) waves pull items from device queues: the item space is dealt to the XCDs in
 // chunks of 2^k items, as xcd_block deals workgroups, each XCD counts off its own
-// chunks (ctl[x], zeroed by k_item_fill), and a wave whose XCD has no items left
+// chunks (ctl[x], zeroed by k_tile_setup), and a wave whose XCD has no items left
 // takes them from the next XCDs in turn. A queue's items come in increasing order,
 // so a wave stops once every one of the eight counters has passed the last item.
 constexpr int kQueueDensity = 8;  // counters in the n_items block: density
 constexpr int kQueueNh = 16;      // nearest-higher
-constexpr int kQueueWords = 24;   // words of the block k_item_fill zeroes
+constexpr int kQueueWords = 24;   // words of the block k_tile_setup zeroes
 struct ItemCursor {
   int32_t* ctl;
   int n;
@@ -116,23 +116,34 @@ struct CoordPtrs {
   const T* x[kMaxDim];
 };
 
+// One workgroup per chunk, or per `group` consecutive chunks of an event (at the first
+// of them), each with its own result: a common one took as many atomic updates of one
+// address as there are workgroups (18 us for 2^20 points, 9 us this way).
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_extremes(CoordPtrs<T> c, int D,
                                                      const Chunk* __restrict__ chunks,
+                                                     const EventDesc* __restrict__ events, int group,
                                                      typename FloatBits<T>::Int* __restrict__ ext) {
   using I = typename FloatBits<T>::Int;
   constexpr I kHi = std::numeric_limits<I>::max(), kLo = std::numeric_limits<I>::min();
   const Chunk ch = chunks[blockIdx.x];
+  int end = ch.end;
+  if (group > 1) {
+    const EventDesc ev = events[ch.event];
+    if ((ch.begin - ev.p_off) / kPointChunk % group != 0) return;
+    end = min(ev.p_off + ev.n, ch.begin + group * kPointChunk);
+  }
   __shared__ I smin[kWaves][kMaxDim], smax[kWaves][kMaxDim];
   const int w = threadIdx.x / kWave;
   for (int d = 0; d < D; ++d) {
     I lo = kHi, hi = kLo;
-    for (int i = ch.begin + threadIdx.x; i < ch.end; i += kBlock) {
+#pragma unroll 8
+    for (int i = ch.begin + threadIdx.x; i < end; i += kBlock) {
       const T v = c.x[d][i];
-      if (v != v) continue;
       const I o = float_to_ordered(v);
-      lo = o < lo ? o : lo;
-      hi = o > hi ? o : hi;
+      const bool ok = v == v;
+      lo = (ok && o < lo) ? o : lo;
+      hi = (ok && o > hi) ? o : hi;
     }
     lo = wave_min_i(lo);
     hi = wave_max_i(hi);
@@ -149,41 +160,8 @@ __global__ __launch_bounds__(kBlock) void k_extremes(CoordPtrs<T> c, int D,
       lo = smin[k][d] < lo ? smin[k][d] : lo;
       hi = smax[k][d] > hi ? smax[k][d] : hi;
     }
-    if (lo != kHi) atomicMin(&ext[(ch.event * D + d) * 2 + 0], lo);
-    if (hi != kLo) atomicMax(&ext[(ch.event * D + d) * 2 + 1], hi);
-  }
-}
-
-// Extremes start from the identities of min and max.
-template <class I>
-__global__ void k_init_extremes(I* __restrict__ ext, int64_t pairs) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k < pairs) {
-    ext[2 * k] = std::numeric_limits<I>::max();
-    ext[2 * k + 1] = std::numeric_limits<I>::min();
-  }
-}
-
-// geo[e] = {mn[D], mx[D], side[D]}, side = (max - min) / nper (ComputeTiles.hpp:33-34).
-template <class T>
-__global__ void k_geometry(const typename FloatBits<T>::Int* __restrict__ ext,
-                           const EventDesc* __restrict__ events, int n_events, int D,
-                           T* __restrict__ geo) {
-  using I = typename FloatBits<T>::Int;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n_events) return;
-  const int nper = events[e].nper;
-  for (int d = 0; d < D; ++d) {
-    const I lo = ext[(e * D + d) * 2 + 0];
-    const I hi = ext[(e * D + d) * 2 + 1];
-    const T mn = lo == std::numeric_limits<I>::max() ? std::numeric_limits<T>::max()
-                                                     : ordered_to_float(lo);
-    const T mx = hi == std::numeric_limits<I>::min() ? std::numeric_limits<T>::lowest()
-                                                     : ordered_to_float(hi);
-    T* g = geo + static_cast<int64_t>(e) * 3 * D;
-    g[d] = mn;
-    g[D + d] = mx;
-    g[2 * D + d] = (mx - mn) / static_cast<T>(nper);
+    ext[(static_cast<int64_t>(blockIdx.x) * D + d) * 2 + 0] = lo;
+    ext[(static_cast<int64_t>(blockIdx.x) * D + d) * 2 + 1] = hi;
   }
 }
 
@@ -202,24 +180,84 @@ __device__ __forceinline__ GeoT<T> event_geo(const T* geo, const RunParamsT<T>& 
 
 // ---------------------------------------------------------------------------
 // (a2) Tile key of every point: t_base + sum_d nper^(D-1-d) * bin_d
-// (TilesView.hpp:54-64), and the identity permutation.
+// (TilesView.hpp:54-64). Every workgroup takes its event's extremes and geometry from
+// the chunks' results, side = (max - min) / nper (ComputeTiles.hpp:33-34); the
+// event's first chunk stores the geometry, geo[e] = {mn[D], mx[D], side[D]}. The keys'
+// lowest digits are counted as they are made: the histogram of the first sort pass.
 // ---------------------------------------------------------------------------
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_tile_keys(CoordPtrs<T> c, const RunParamsT<T> rp,
-                                                      const Chunk* __restrict__ chunks,
-                                                      const EventDesc* __restrict__ events,
-                                                      const T* __restrict__ geo,
-                                                      uint32_t* __restrict__ keys,
-                                                      int32_t* __restrict__ vals) {
+__global__ __launch_bounds__(kBlock) void k_tile_keys(
+    CoordPtrs<T> c, const RunParamsT<T> rp, const Chunk* __restrict__ chunks,
+    const EventDesc* __restrict__ events, int group,
+    const typename FloatBits<T>::Int* __restrict__ ext, T* __restrict__ geo,
+    uint32_t* __restrict__ keys, int digit_bits, int32_t* __restrict__ hist) {
+  using I = typename FloatBits<T>::Int;
+  constexpr I kHi = std::numeric_limits<I>::max(), kLo = std::numeric_limits<I>::min();
+  __shared__ int32_t cnt[kRsMaxBins];
+  __shared__ I smin[kWaves][kMaxDim], smax[kWaves][kMaxDim];
+  __shared__ T sgeo[3 * kMaxDim];
   const Chunk ch = chunks[blockIdx.x];
   const EventDesc ev = events[ch.event];
-  const GeoT<T> g = event_geo(geo, rp, ch.event, ev.nper);
+  const int D = rp.D;
+  const int bins = 1 << digit_bits;
+  for (int k = threadIdx.x; k < bins; k += kBlock) cnt[k] = 0;
+  const int first = static_cast<int>(blockIdx.x) - (ch.begin - ev.p_off) / kPointChunk;
+  const int n_ext = ((ev.n + kPointChunk - 1) / kPointChunk + group - 1) / group;
+  const int w = threadIdx.x / kWave;
+  for (int d = 0; d < D; ++d) {
+    I lo = kHi, hi = kLo;
+    for (int k = threadIdx.x; k < n_ext; k += kBlock) {
+      const int64_t q = (static_cast<int64_t>(first + k * group) * D + d) * 2;
+      const I l = ext[q], h = ext[q + 1];
+      lo = l < lo ? l : lo;
+      hi = h > hi ? h : hi;
+    }
+    lo = wave_min_i(lo);
+    hi = wave_max_i(hi);
+    if (lane_id() == 0) {
+      smin[w][d] = lo;
+      smax[w][d] = hi;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    const int d = threadIdx.x;
+    I lo = kHi, hi = kLo;
+    for (int k = 0; k < kWaves; ++k) {
+      lo = smin[k][d] < lo ? smin[k][d] : lo;
+      hi = smax[k][d] > hi ? smax[k][d] : hi;
+    }
+    const T mn = lo == kHi ? std::numeric_limits<T>::max() : ordered_to_float(lo);
+    const T mx = hi == kLo ? std::numeric_limits<T>::lowest() : ordered_to_float(hi);
+    const T side = (mx - mn) / static_cast<T>(ev.nper);
+    sgeo[d] = mn;
+    sgeo[D + d] = mx;
+    sgeo[2 * D + d] = side;
+    if (ch.begin == ev.p_off) {
+      T* g = geo + static_cast<int64_t>(ch.event) * 3 * D;
+      g[d] = mn;
+      g[D + d] = mx;
+      g[2 * D + d] = side;
+    }
+  }
+  __syncthreads();
+  GeoT<T> g;
+  g.D = D;
+  g.nper = ev.nper;
+  g.mn = sgeo;
+  g.mx = sgeo + D;
+  g.side = sgeo + 2 * D;
+  g.wrapped = rp.wrapped;
   for (int i = ch.begin + threadIdx.x; i < ch.end; i += kBlock) {
     int t = 0;
-    for (int d = 0; d < rp.D; ++d) t = t * ev.nper + get_bin(g, c.x[d][i], d);
-    keys[i] = static_cast<uint32_t>(ev.t_base + t);
-    vals[i] = i;
+    for (int d = 0; d < D; ++d) t = t * ev.nper + get_bin(g, c.x[d][i], d);
+    const uint32_t key = static_cast<uint32_t>(ev.t_base + t);
+    keys[i] = key;
+    atomicAdd(&cnt[key & (bins - 1)], 1);
   }
+  __syncthreads();
+  for (int k = threadIdx.x; k < bins; k += kBlock)
+    hist[static_cast<int64_t>(k) * gridDim.x + blockIdx.x] = cnt[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -263,7 +301,7 @@ __global__ __launch_bounds__(kBlock) void k_gather(const GatherArgs<T> a, const 
 // (a1-a3 fused) One workgroup per event when every event of the batch has at
 // most kEvtMaxTiles tiles: extremes and geometry, tile ids, a stable counting
 // sort by tile into the sorted SoA copy and the tile offsets, all in one
-// kernel. Same results as k_extremes + k_geometry + k_tile_keys + the radix
+// kernel. Same results as k_extremes + k_tile_keys + the radix
 // sort + k_gather: the extremes are the same ordered-integer min/max (NaN
 // skipped), the bins the same get_bin, and the order (tile, input index).
 // Each wave owns a contiguous sixteenth of the event, walked in
@@ -481,81 +519,33 @@ static void launch_event_tiles(const RunParamsT<T>& rp, const PointArraysT<T>& i
   }
 }
 
-// Work items: ceil(count / 64) per tile.
+// Work items: ceil(count / 64) per tile, from slot ioff[t] on (an exclusive scan of
+// the counts), or, without that scan (ioff NULL), from slot toff[t] / 64 + t on: a
+// tile then has at most one slot more than items, and such slots hold empty items.
+// Small launches save four kernels by it; in large ones the empty items, a seventh of
+// the slots of the 4096-event batch, cost the neighbour stages 1-3 %.
+__device__ __forceinline__ int first_item(const int32_t* __restrict__ ioff, int b, int t) {
+  return ioff ? ioff[t] : b / kWave + t;
+}
 static __global__ void k_item_count(const int32_t* __restrict__ toff, int n_tiles,
-                             int32_t* __restrict__ icount) {
+                                    int32_t* __restrict__ icount) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n_tiles) return;
   icount[k] = (toff[k + 1] - toff[k] + kWave - 1) / kWave;
 }
 
-static __global__ void k_item_fill(const int32_t* __restrict__ toff, const int32_t* __restrict__ ioff,
-                            int n_tiles, const EventDesc* __restrict__ events, int n_events,
-                            Item* __restrict__ items, int32_t* __restrict__ queues) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= kQueueDensity && k < kQueueWords) queues[k] = 0;  // work-item queue counters
-  if (k >= n_tiles) return;
-  // Event of tile k: last event with t_base <= k.
-  int lo = 0, hi = n_events - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (events[mid].t_base <= k)
-      lo = mid;
-    else
-      hi = mid - 1;
+// Event of tile t: the last with t_base <= t (one wave, 64 events per step).
+__device__ __forceinline__ int tile_event(const EventDesc* __restrict__ events, int n_events, int t) {
+  int lo = 0, n = n_events;  // the answer lies in [lo, lo + n)
+  while (n > 1) {
+    const int step = (n + kWave - 1) / kWave;
+    const int k = lane_id() * step;
+    const bool at_or_before = k < n && events[lo + k].t_base <= t;
+    const int last = 63 - __builtin_clzll(ballot(at_or_before));  // lane 0 always is
+    lo += last * step;
+    n = min(step, n - last * step);
   }
-  const int b = toff[k], e = toff[k + 1];
-  int o = ioff[k];
-  for (int s = b; s < e; s += kWave) {
-    Item it;
-    it.tile = k;
-    it.begin = s;
-    it.end = min(e, s + kWave);
-    it.event = lo;
-    items[o++] = it;
-  }
-}
-
-// The three item kernels above in one workgroup, for batches of at most
-// kItemsOneBlockTiles tiles (one launch instead of five): the tiles' item counts
-// and their exclusive scan (kBlock tiles at a time, with a carry), the total and
-// the queue counters, then the items. Each thread fills the tiles whose offsets it
-// wrote, so the fill reads only its own stores.
-constexpr int kItemsOneBlockTiles = 4096;
-static __global__ __launch_bounds__(kBlock) void k_items_one_block(
-    const int32_t* __restrict__ toff, int n_tiles, const EventDesc* __restrict__ events,
-    int n_events, int32_t* __restrict__ ioff, Item* __restrict__ items, int32_t* __restrict__ ctl) {
-  int carry = 0;
-  for (int base = 0; base < n_tiles; base += kBlock) {
-    const int t = base + threadIdx.x;
-    const int c = t < n_tiles ? (toff[t + 1] - toff[t] + kWave - 1) / kWave : 0;
-    int tot;
-    const int ex = block_excl_scan<kBlock>(c, &tot);
-    if (t < n_tiles) ioff[t] = carry + ex;
-    carry += tot;
-  }
-  if (threadIdx.x == 0) ctl[0] = carry;
-  for (int k = kQueueDensity + threadIdx.x; k < kQueueWords; k += kBlock) ctl[k] = 0;
-  for (int t = threadIdx.x; t < n_tiles; t += kBlock) {
-    int lo = 0, hi = n_events - 1;  // event of tile t: last event with t_base <= t
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (events[mid].t_base <= t)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
-    const int b = toff[t], e = toff[t + 1];
-    int o = ioff[t];
-    for (int s = b; s < e; s += kWave) {
-      Item it;
-      it.tile = t;
-      it.begin = s;
-      it.end = min(e, s + kWave);
-      it.event = lo;
-      items[o++] = it;
-    }
-  }
+  return lo;
 }
 
 __device__ __forceinline__ float fmin_t(float a, float b) { return __builtin_fminf(a, b); }
@@ -776,6 +766,25 @@ __device__ __forceinline__ T wave_max_f(T v) {
   for (int off = 32; off > 0; off >>= 1) v = fmax_t(v, __shfl_xor(v, off, 64));
   return v;
 }
+// The same, wave-uniform, float through DPP lane moves (no LDS round trips).
+__device__ __forceinline__ float wave_min_uniform(float v) {
+  return __int_as_float(wave_reduce_dpp(__float_as_int(v), 0x7f800000, [](int a, int b) {
+    return __float_as_int(__builtin_fminf(__int_as_float(a), __int_as_float(b)));
+  }));
+}
+__device__ __forceinline__ float wave_max_uniform(float v) {
+  return __int_as_float(wave_reduce_dpp(__float_as_int(v), static_cast<int>(0xff800000u), [](int a, int b) {
+    return __float_as_int(__builtin_fmaxf(__int_as_float(a), __int_as_float(b)));
+  }));
+}
+__device__ __forceinline__ double wave_min_uniform(double v) {
+  v = wave_min_f(v);
+  return __longlong_as_double(
+      (static_cast<long long>(uniform(static_cast<int>(__double_as_longlong(v) >> 32))) << 32) |
+      static_cast<uint32_t>(uniform(static_cast<int>(__double_as_longlong(v)))));
+}
+__device__ __forceinline__ double wave_max_uniform(double v) { return -wave_min_uniform(-v); }
+
 // Minimum and maximum over each group of N = 8 or 16 lanes (a half row or a row),
 // in every lane of the group (float through DPP lane moves: pair swap, quad swap,
 // half-row mirror, then for 16 the row mirror; lanes a move does not write take
@@ -891,44 +900,68 @@ __device__ __forceinline__ void write_nh_layout(int t, int b, int cnt, const int
   }
 }
 
-// Bounding box of every tile's points, one wave per tile: the density stage leaves
-// out the tiles none of a wave's queries can reach.
+// One wave per tile: its work items and (tbox) its points' bounding box, by which the
+// density stage leaves out the tiles none of a wave's queries can reach.
 template <int D, class T>
-__global__ __launch_bounds__(kBlock) void k_tile_boxes(const int32_t* __restrict__ toff, int n_tiles,
-                                                       const T* __restrict__ sx, int64_t cs,
-                                                       T* __restrict__ tbox) {
+__global__ __launch_bounds__(kBlock) void k_tile_setup(
+    const int32_t* __restrict__ toff, int n_tiles, const EventDesc* __restrict__ events,
+    int n_events, const T* __restrict__ sx, int64_t cs, T* __restrict__ tbox,
+    Item* __restrict__ items, const int32_t* __restrict__ ioff, int32_t max_items,
+    int32_t* __restrict__ ctl) {
+  if (blockIdx.x == 0 && threadIdx.x >= kQueueDensity && threadIdx.x < kQueueWords)
+    ctl[threadIdx.x] = 0;  // work-item queue counters
   const int t = blockIdx.x * kWaves + threadIdx.x / kWave;
   if (t >= n_tiles) return;
-  const int e = toff[t + 1];
-  T lo[D], hi[D];
+  const int b = toff[t], e = toff[t + 1];
+  // The first points' loads go out before the search for the event.
+  T x0[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    x0[d] = (tbox && b + lane_id() < e) ? sx[d * cs + b + lane_id()] : std::numeric_limits<T>::quiet_NaN();
+  const int e_t = tile_event(events, n_events, t);
+  const int first = first_item(ioff, b, t);
+  const int slots = ioff ? (e - b + kWave - 1) / kWave
+                         : (t + 1 < n_tiles ? first_item(ioff, e, t + 1) : max_items) - first;
+  for (int k = lane_id(); k < slots; k += kWave) {
+    Item it;
+    it.tile = t;
+    it.begin = min(e, b + k * kWave);
+    it.end = min(e, it.begin + kWave);
+    it.event = e_t;
+    items[first + k] = it;
+  }
+  if (!tbox) return;
+  T mn[D], mx[D];
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    lo[d] = std::numeric_limits<T>::infinity();
-    hi[d] = -std::numeric_limits<T>::infinity();
+    mn[d] = fmin_t(std::numeric_limits<T>::infinity(), x0[d]);
+    mx[d] = fmax_t(-std::numeric_limits<T>::infinity(), x0[d]);
   }
 #pragma unroll 4
-  for (int s = toff[t] + lane_id(); s < e; s += kWave)
+  for (int s = b + kWave + lane_id(); s < e; s += kWave)
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const T x = sx[d * cs + s];
-      lo[d] = fmin_t(lo[d], x);
-      hi[d] = fmax_t(hi[d], x);
+      mn[d] = fmin_t(mn[d], x);
+      mx[d] = fmax_t(mx[d], x);
     }
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    lo[d] = wave_min_f(lo[d]);
-    hi[d] = wave_max_f(hi[d]);
+    mn[d] = wave_min_uniform(mn[d]);
+    mx[d] = wave_max_uniform(mx[d]);
   }
   if (lane_id() == 0) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      tbox[static_cast<int64_t>(t) * 2 * D + d] = lo[d];
-      tbox[static_cast<int64_t>(t) * 2 * D + D + d] = hi[d];
+      tbox[static_cast<int64_t>(t) * 2 * D + d] = mn[d];
+      tbox[static_cast<int64_t>(t) * 2 * D + D + d] = mx[d];
     }
   }
 }
 
-// The query order of kWaves tiles per workgroup. A tile of at most one wave's
+// The query order of W tiles per workgroup (8 for a lone event, whose dense tiles are
+// the largest, else 4: one event of 2^20 points 81 us at 4 and 54 us at 8, the
+// 4096-event batch 744 us and 990 us). A tile of at most one wave's
 // points keeps its order (one wave each). The others are taken one after the other
 // by the whole workgroup, a counting sort in LDS by the Morton index: the dense
 // tiles, thousands of points where most tiles hold a few dozen, are what one wave
@@ -936,8 +969,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_boxes(const int32_t* __restrict
 // in 2-D: 248 -> 89 us; of 100,000: 87 -> 28 us). Points of equal index are placed by LDS atomics, in no
 // order among themselves: no result depends on the query order or on the order
 // within the nearest-higher layout.
-template <int D, class T>
-__global__ __launch_bounds__(kBlock) void k_query_order(
+template <int D, int W, class T>
+__global__ __launch_bounds__(W * kWave) void k_query_order(
     const RunParamsT<T> rp, const EventDesc* __restrict__ events, const Item* __restrict__ items,
     const int32_t* __restrict__ ioff, const T* __restrict__ geo, const int32_t* __restrict__ toff,
     int n_tiles, const T* __restrict__ sx, int64_t cs, int32_t* __restrict__ qfine,
@@ -945,27 +978,28 @@ __global__ __launch_bounds__(kBlock) void k_query_order(
   constexpr int kD = D < kQueryDims ? D : kQueryDims;
   constexpr int kFineBits = (8 / kD) * kD;
   constexpr int kFine = 1 << kFineBits;
+  constexpr int kOrderBlock = W * kWave;
   constexpr int kHeld = 4;  // rounds whose Morton indices stay in registers
-  static_assert(kFine <= kBlock, "one counter per thread in the scan");
+  static_assert(kFine <= kOrderBlock, "one counter per thread in the scan");
   __shared__ int32_t cnt[kFine];
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   {
-    const int t = blockIdx.x * kWaves + w;
+    const int t = blockIdx.x * W + w;
     const int b = t < n_tiles ? toff[t] : 0, e = t < n_tiles ? toff[t + 1] : 0;
     if (t < n_tiles && e - b <= kWave) {  // one item: the query order is irrelevant
       if (b + lane < e) qfine[b + lane] = b + lane;
       if (hx) write_nh_layout<D>(t, b, e - b, nullptr, 0, 1, sx, cs, hx, hs, hidx, hbox);
     }
   }
-  for (int k = 0; k < kWaves; ++k) {
-    const int t = blockIdx.x * kWaves + k;
+  for (int k = 0; k < W; ++k) {
+    const int t = blockIdx.x * W + k;
     if (t >= n_tiles) break;
     const int b = toff[t], e = toff[t + 1];
     if (e - b <= kWave) continue;
-    // Event of tile t: that of its first work item (ioff: the items' exclusive
-    // scan), two dependent loads where a search over the events takes a dozen.
-    const int ev_i = items[ioff[t]].event;
+    // Event of tile t: that of its first work item, where a search over the events
+    // takes a dozen dependent loads.
+    const int ev_i = items[first_item(ioff, b, t)].event;
     const EventDesc ev = events[ev_i];
     const GeoT<T> g = event_geo(geo, rp, ev_i, ev.nper);
     int tb[D];
@@ -988,28 +1022,30 @@ __global__ __launch_bounds__(kBlock) void k_query_order(
     uint32_t held[kHeld];
 #pragma unroll
     for (int r = 0; r < kHeld; ++r) {
-      const int s = b + r * kBlock + static_cast<int>(threadIdx.x);
+      const int s = b + r * kOrderBlock + static_cast<int>(threadIdx.x);
       held[r] = s < e ? key_of(s) : 0u;
       if (s < e) atomicAdd(&cnt[held[r]], 1);
     }
-    for (int s = b + kHeld * kBlock + static_cast<int>(threadIdx.x); s < e; s += kBlock)
+#pragma unroll 4
+    for (int s = b + kHeld * kOrderBlock + static_cast<int>(threadIdx.x); s < e; s += kOrderBlock)
       atomicAdd(&cnt[key_of(s)], 1);
     __syncthreads();
     int total;
     const int c = threadIdx.x < kFine ? cnt[threadIdx.x] : 0;
-    const int first = block_excl_scan<kBlock>(c, &total);
+    const int first = block_excl_scan<kOrderBlock>(c, &total);
     if (threadIdx.x < kFine) cnt[threadIdx.x] = b + first;
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kHeld; ++r) {
-      const int s = b + r * kBlock + static_cast<int>(threadIdx.x);
+      const int s = b + r * kOrderBlock + static_cast<int>(threadIdx.x);
       if (s < e) qfine[atomicAdd(&cnt[held[r]], 1)] = s;
     }
-    for (int s = b + kHeld * kBlock + static_cast<int>(threadIdx.x); s < e; s += kBlock)
+#pragma unroll 4
+    for (int s = b + kHeld * kOrderBlock + static_cast<int>(threadIdx.x); s < e; s += kOrderBlock)
       qfine[atomicAdd(&cnt[key_of(s)], 1)] = s;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // qfine of the tile
     __syncthreads();
-    if (hx) write_nh_layout<D>(t, b, e - b, qfine, w, kWaves, sx, cs, hx, hs, hidx, hbox);
+    if (hx) write_nh_layout<D>(t, b, e - b, qfine, w, W, sx, cs, hx, hs, hidx, hbox);
   }
 }
 
@@ -1253,9 +1289,9 @@ __device__ __forceinline__ QueryBox<D, T> query_box(const T (&x)[D], const T (&s
   QueryBox<D, T> q;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    q.lo[d] = read_lane(wave_min_f(active ? x[d] : std::numeric_limits<T>::infinity()), 0);
-    q.hi[d] = read_lane(wave_max_f(active ? x[d] : -std::numeric_limits<T>::infinity()), 0);
-    q.s[d] = M == M_MAHALANOBIS ? read_lane(wave_max_f(active ? __builtin_fabs(s[d]) : T(0)), 0) : T(0);
+    q.lo[d] = wave_min_uniform(active ? x[d] : std::numeric_limits<T>::infinity());
+    q.hi[d] = wave_max_uniform(active ? x[d] : -std::numeric_limits<T>::infinity());
+    q.s[d] = M == M_MAHALANOBIS ? wave_max_uniform(active ? __builtin_fabs(s[d]) : T(0)) : T(0);
   }
   return q;
 }
@@ -2080,12 +2116,21 @@ static __global__ __launch_bounds__(kRankBlock) void k_seed_ranks(const uint32_t
   const int wave = threadIdx.x / kWave, lane = lane_id();
   int c[kRankRows][4], incl[kRankRows];
 #pragma unroll
-  for (int r = 0; r < kRankRows; ++r)
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int w = (r * kRankBlock + static_cast<int>(threadIdx.x)) * 4 + k;
-      c[r][k] = w < words ? __popc(bits[w]) : 0;
+  for (int r = 0; r < kRankRows; ++r) {
+    const int w = (r * kRankBlock + static_cast<int>(threadIdx.x)) * 4;
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (w + 3 < words) {
+      v = *reinterpret_cast<const uint4*>(bits + w);
+    } else if (w < words) {
+      v.x = bits[w];
+      if (w + 1 < words) v.y = bits[w + 1];
+      if (w + 2 < words) v.z = bits[w + 2];
     }
+    c[r][0] = __popc(v.x);
+    c[r][1] = __popc(v.y);
+    c[r][2] = __popc(v.z);
+    c[r][3] = __popc(v.w);
+  }
 #pragma unroll
   for (int r = 0; r < kRankRows; ++r) {
     incl[r] = wave_incl_scan(c[r][0] + c[r][1] + c[r][2] + c[r][3]);
@@ -2435,8 +2480,8 @@ static void launch_density_dm(const NeighbourLaunch<T>& L) {
   if (L.rp->team) {
     const BatchBuffersT<T>& b = *L.bb;
     hipLaunchKernelGGL((k_density_team<D, M, T>), dim3(L.grid_team), dim3(kTeam * kWave), 0, L.s,
-                       *L.rp, b.events, b.geo, b.toff, b.items, b.n_items, b.sorted.x[0], L.cs,
-                       b.sorted.w, b.sorted.fw, b.sorted.sigma[0], b.sorted.tag, b.qfine, b.tbox,
+                       *L.rp, b.events, b.geo, b.toff, b.items, b.sorted.x[0], L.cs, b.sorted.w,
+                       b.sorted.fw, b.sorted.sigma[0], b.sorted.tag, b.qfine, b.tbox,
                        b.srho, b.skey);
     return;
   }
@@ -2467,7 +2512,7 @@ static void launch_nh_dm(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
   if (L.rp->team) {
     hipLaunchKernelGGL((k_nearest_higher_team<D, M, T>), dim3(L.grid_team), dim3(kTeam * kWave), 0,
-                       L.s, *L.rp, b.events, b.geo, b.toff, b.items, b.n_items, b.sorted.x[0], L.cs,
+                       L.s, *L.rp, b.events, b.geo, b.toff, b.items, b.sorted.x[0], L.cs,
                        b.sorted.sigma[0], b.sorted.u, b.sorted.tag, b.srho, b.skey, b.qfine,
                        b.tbox, b.snh, b.sdelta);
     return;
@@ -2571,33 +2616,40 @@ CLUE_NEIGHBOUR_EXTERN(10)
 template <int D, class T>
 static void launch_query_order_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
-  const unsigned grid = static_cast<unsigned>((b.n_tiles_total + kWaves - 1) / kWaves);
-  hipLaunchKernelGGL((k_query_order<D, T>), dim3(grid), dim3(kBlock), 0, L.s, *L.rp, b.events,
-                     b.items, b.icount, b.geo, b.toff, b.n_tiles_total, b.sorted.x[0], L.cs,
-                     b.qfine, b.hx, b.h_stride, b.hidx, b.hbox);
+  auto go = [&](auto kern, int waves) {
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((b.n_tiles_total + waves - 1) / waves)),
+                       dim3(waves * kWave), 0, L.s, *L.rp, b.events, b.items, b.icount, b.geo, b.toff,
+                       b.n_tiles_total, b.sorted.x[0], L.cs, b.qfine, b.hx, b.h_stride, b.hidx,
+                       b.hbox);
+  };
+  if (b.n_events == 1)
+    go(k_query_order<D, 8, T>, 8);
+  else
+    go(k_query_order<D, 4, T>, 4);
 }
 
 template <int D, class T>
-static void launch_tile_boxes_d(const NeighbourLaunch<T>& L) {
+static void launch_tile_setup_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
   const unsigned grid = static_cast<unsigned>((b.n_tiles_total + kWaves - 1) / kWaves);
-  hipLaunchKernelGGL((k_tile_boxes<D, T>), dim3(grid), dim3(kBlock), 0, L.s, b.toff,
-                     b.n_tiles_total, b.sorted.x[0], L.cs, b.tbox);
+  hipLaunchKernelGGL((k_tile_setup<D, T>), dim3(grid), dim3(kBlock), 0, L.s, b.toff,
+                     b.n_tiles_total, b.events, b.n_events, b.sorted.x[0], L.cs, b.tbox, b.items,
+                     b.icount, b.max_items, b.n_items);
 }
 
 template <class T>
-static void launch_tile_boxes(const NeighbourLaunch<T>& L) {
+static void launch_tile_setup(const NeighbourLaunch<T>& L) {
   switch (L.rp->D) {
-    case 1: launch_tile_boxes_d<1>(L); break;
-    case 2: launch_tile_boxes_d<2>(L); break;
-    case 3: launch_tile_boxes_d<3>(L); break;
-    case 4: launch_tile_boxes_d<4>(L); break;
-    case 5: launch_tile_boxes_d<5>(L); break;
-    case 6: launch_tile_boxes_d<6>(L); break;
-    case 7: launch_tile_boxes_d<7>(L); break;
-    case 8: launch_tile_boxes_d<8>(L); break;
-    case 9: launch_tile_boxes_d<9>(L); break;
-    default: launch_tile_boxes_d<10>(L); break;
+    case 1: launch_tile_setup_d<1>(L); break;
+    case 2: launch_tile_setup_d<2>(L); break;
+    case 3: launch_tile_setup_d<3>(L); break;
+    case 4: launch_tile_setup_d<4>(L); break;
+    case 5: launch_tile_setup_d<5>(L); break;
+    case 6: launch_tile_setup_d<6>(L); break;
+    case 7: launch_tile_setup_d<7>(L); break;
+    case 8: launch_tile_setup_d<8>(L); break;
+    case 9: launch_tile_setup_d<9>(L); break;
+    default: launch_tile_setup_d<10>(L); break;
   }
 }
 
@@ -2638,7 +2690,6 @@ static void launch_neighbour(const NeighbourLaunch<T>& L, bool density) {
 template <class T>
 void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const BatchBuffersT<T>& bb,
                      const ResultArraysT<T>& out, hipStream_t s, const StageHook* hook) {
-  using I = typename FloatBits<T>::Int;
   auto mark = [&](int stage) {
     if (hook && hook->mark) hook->mark(hook->self, stage, s);
   };
@@ -2654,18 +2705,15 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
     mark(kStageTiles);
     launch_event_tiles(rp, in, bb, s);
   } else {
-  hipLaunchKernelGGL(k_init_extremes<I>,
-                     dim3(static_cast<unsigned>((static_cast<int64_t>(bb.n_events) * D + kBlock - 1) / kBlock)),
-                     dim3(kBlock), 0, s, bb.ext, static_cast<int64_t>(bb.n_events) * D);
-  hipLaunchKernelGGL(k_extremes<T>, dim3(bb.n_chunks), dim3(kBlock), 0, s, cp, D, bb.chunks, bb.ext);
-  hipLaunchKernelGGL(k_geometry<T>, dim3((bb.n_events + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
-                     bb.ext, bb.events, bb.n_events, D, bb.geo);
+  hipLaunchKernelGGL(k_extremes<T>, dim3(bb.n_chunks), dim3(kBlock), 0, s, cp, D, bb.chunks,
+                     bb.events, bb.ext_group, bb.ext);
   mark(kStageTiles);
+  const RadixPlan digits = radix_plan(bb.key_bits);
   hipLaunchKernelGGL(k_tile_keys<T>, dim3(bb.n_chunks), dim3(kBlock), 0, s, cp, rp, bb.chunks,
-                     bb.events, bb.geo, bb.keys0, bb.vals0);
+                     bb.events, bb.ext_group, bb.ext, bb.geo, bb.keys0, digits.bits, bb.rs_hist);
   bool in_first = true;
-  radix_sort_pairs(bb.keys0, bb.vals0, bb.keys1, bb.vals1, n, bb.key_bits, bb.rs_hist, bb.scan_tmp,
-                   &in_first, s);
+  radix_sort_pairs(bb.keys0, bb.vals0, bb.keys1, bb.vals1, n, bb.key_bits, bb.rs_hist, bb.chunks,
+                   bb.n_chunks, &in_first, s);
   const uint32_t* skeys = in_first ? bb.keys0 : bb.keys1;
   const int32_t* sperm = in_first ? bb.vals0 : bb.vals1;
   GatherArgs<T> ga;
@@ -2675,20 +2723,6 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
   hipLaunchKernelGGL(k_gather<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, ga, rp, skeys,
                      sperm, n, bb.n_tiles_total, bb.toff,
                      reinterpret_cast<uint32_t*>(bb.flag));
-  }
-  if (bb.n_tiles_total <= kItemsOneBlockTiles) {
-    hipLaunchKernelGGL(k_items_one_block, dim3(1), dim3(kBlock), 0, s, bb.toff, bb.n_tiles_total,
-                       bb.events, bb.n_events, bb.icount, bb.items, bb.n_items);
-  } else {
-    hipLaunchKernelGGL(k_item_count, dim3((bb.n_tiles_total + kBlock - 1) / kBlock), dim3(kBlock),
-                       0, s, bb.toff, bb.n_tiles_total, bb.icount);
-    scan_exclusive(bb.icount, bb.icount, bb.n_tiles_total, bb.scan_tmp, bb.n_items, s);
-    hipLaunchKernelGGL(k_item_fill,
-                       dim3(static_cast<unsigned>(
-                           (std::max<int64_t>(bb.n_tiles_total, kQueueWords) + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0,
-                       s, bb.toff, bb.icount, bb.n_tiles_total, bb.events, bb.n_events, bb.items,
-                       bb.n_items);
   }
 
   NeighbourLaunch<T> L;
@@ -2706,7 +2740,12 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
   L.grid_team =
       static_cast<unsigned>((static_cast<int64_t>(bb.max_items) + kXcds - 1) / kXcds * kXcds);
   L.s = s;
-  if (bb.tbox) launch_tile_boxes(L);    // bounds of the density stage's candidates
+  if (bb.icount) {
+    hipLaunchKernelGGL(k_item_count, dim3((bb.n_tiles_total + kBlock - 1) / kBlock), dim3(kBlock),
+                       0, s, bb.toff, bb.n_tiles_total, bb.icount);
+    scan_exclusive(bb.icount, bb.icount, bb.n_tiles_total, bb.scan_tmp, bb.n_items, s);
+  }
+  launch_tile_setup(L);                 // work items and tile boxes
   if (bb.qfine) launch_query_order(L);  // query order of the two neighbour stages
 
   // (b), (c)

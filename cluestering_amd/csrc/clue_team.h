@@ -368,7 +368,7 @@ template <int D, int M, class T>
 __global__ __launch_bounds__(kTeam * kWave) void k_density_team(
     const RunParamsT<T> rp, const EventDesc* __restrict__ events, const T* __restrict__ geo,
     const int32_t* __restrict__ toff, const Item* __restrict__ items,
-    const int32_t* __restrict__ n_items, const T* __restrict__ sx, int64_t cs,
+    const T* __restrict__ sx, int64_t cs,
     const T* __restrict__ sw, const T* __restrict__ sfw, const T* __restrict__ ssig,
     const uint32_t* __restrict__ stag, const int32_t* __restrict__ qperm,
     const T* __restrict__ tbox, T* __restrict__ srho, uint64_t* __restrict__ skey) {
@@ -377,11 +377,12 @@ __global__ __launch_bounds__(kTeam * kWave) void k_density_team(
   __shared__ SumRelay<T> relay;
   __shared__ List list;
   const int item = xcd_block(blockIdx.x, gridDim.x, rp.xcd_chunk_log2);
-  if (item >= *n_items) return;
+  if (item >= rp.max_items) return;
+  const Item it = items[item];
+  if (it.begin >= it.end) return;  // an empty slot
   const int wave = uniform(threadIdx.x / kWave);
   if (wave == 0) relay_pass(relay, T(0), 0);
   __syncthreads();
-  const Item it = items[item];
   // A lone event's descriptors are loaded beside the item, not after it.
   const int e = rp.n_events == 1 ? 0 : it.event;
   const EventDesc ev = events[e];
@@ -494,7 +495,7 @@ template <int D, int M, class T>
 __global__ __launch_bounds__(kTeam * kWave) void k_nearest_higher_team(
     const RunParamsT<T> rp, const EventDesc* __restrict__ events, const T* __restrict__ geo,
     const int32_t* __restrict__ toff, const Item* __restrict__ items,
-    const int32_t* __restrict__ n_items, const T* __restrict__ sx, int64_t cs,
+    const T* __restrict__ sx, int64_t cs,
     const T* __restrict__ ssig, const T* __restrict__ su, const uint32_t* __restrict__ stag,
     const T* __restrict__ srho, const uint64_t* __restrict__ skey,
     const int32_t* __restrict__ qperm, const T* __restrict__ tbox, int32_t* __restrict__ snh,
@@ -508,10 +509,11 @@ __global__ __launch_bounds__(kTeam * kWave) void k_nearest_higher_team(
   __shared__ uint32_t best_tag[kTeam][kWave];
   __shared__ int32_t best_nh[kTeam][kWave], best_order[kTeam][kWave];
   const int item = xcd_block(blockIdx.x, gridDim.x, rp.xcd_chunk_log2);
-  if (item >= *n_items) return;
+  if (item >= rp.max_items) return;
+  const Item it = items[item];
+  if (it.begin >= it.end) return;  // an empty slot
   const int wave = uniform(threadIdx.x / kWave);
   const int lane = lane_id();
-  const Item it = items[item];
   // A lone event's descriptors are loaded beside the item, not after it.
   const int e = rp.n_events == 1 ? 0 : it.event;
   const EventDesc ev = events[e];

@@ -26,12 +26,13 @@ constexpr int kPointChunk = 2048;  // points per chunk of the per-point grids
 // Workspace sizes of the scan and radix-sort primitives (clue_primitives.hip),
 // here so that host-only code sizes workspaces exactly as the device path does.
 constexpr int kScanTileElems = 4096;  // elements per block of the exclusive scan
-constexpr int kRsTileKeys = 4096;     // keys per block of a radix pass
-constexpr int kRsDigitBins = 256;     // bins of one radix digit
+constexpr int kRsTileKeys = 2048;     // keys per block of a radix pass
+constexpr int kRsMaxBits = 10;        // of a radix digit
+constexpr int kRsMaxBins = 1 << kRsMaxBits;
+static_assert(kPointChunk == kRsTileKeys, "a chunk is a block of the radix sort");
 inline int64_t scan_temp_elems(int64_t n) { return (n + kScanTileElems - 1) / kScanTileElems + 1; }
-inline int64_t radix_hist_elems(int64_t n) {
-  return kRsDigitBins * ((n + kRsTileKeys - 1) / kRsTileKeys);
-}
+// Digit counts per block, then the digits' totals.
+inline int64_t radix_hist_elems(int64_t blocks) { return kRsMaxBins * (blocks + 1); }
 
 // Constants of the float exp (Cody-Waite reduction x = k ln2 + r with a 15-bit
 // ln2_hi, then the degree-6 minimax polynomial of e^r on [-ln2/2, ln2/2] whose
@@ -98,6 +99,7 @@ struct RunParamsT {
   int32_t has_tags;
   int32_t n_events;
   int32_t n_total;
+  int32_t max_items;       // work-item slots
   T dc;
   T rhoc;
   T dm;
