@@ -50,6 +50,11 @@ inline clue_dev::ExpScaled exp_scaled(int s) {
   return e;
 }
 
+inline bool team_launch(int64_t points, int64_t events) {
+  const bool small = events > 1 && points / events < kTeamSmallEvent;
+  return points <= (small ? kTeamMaxPointsSmall : kTeamMaxPoints);
+}
+
 // Capacity a grow-only device buffer holds after a request of `bytes`: unchanged
 // when it already fits, else the request plus a quarter and 256 bytes.
 inline size_t grown_capacity(size_t cap, size_t bytes) {
@@ -173,9 +178,7 @@ inline clue_status plan_batch(int D, int points_per_tile, const uint32_t* sizes,
   for (const EventDesc& ev : bp->events) largest = std::max<int64_t>(largest, ev.n);
   bp->ext_group = static_cast<int>(std::max<int64_t>(1, (largest + 512 * kChunk - 1) / (512 * kChunk)));
   // A fixed tuning keeps one wave per item.
-  const int64_t mean = bp->events.empty() ? 0 : off / static_cast<int64_t>(bp->events.size());
-  bp->team = !fixed && off <= (mean < kTeamSmallEvent && bp->events.size() > 1 ? kTeamMaxPointsSmall
-                                                                                : kTeamMaxPoints);
+  bp->team = !fixed && team_launch(off, static_cast<int64_t>(bp->events.size()));
   if (bp->team) bp->tuning.group_queries = 1;  // small boxes around each team's points
   bp->max_items = (off + 63) / 64 + tiles;
   int bits = 0;
