@@ -72,25 +72,6 @@ void* scratch_ptr(int device) {
   return t.done[device] ? t.ptr[device] : nullptr;
 }
 
-// The descriptors of one event of n points at p_off 0 (what the host plan holds),
-// written on the device: chunk c covers [c * kChunk, min(n, (c + 1) * kChunk)).
-__global__ void k_single_event_descriptors(EventDesc ev, EventDesc* __restrict__ events,
-                                           int32_t* __restrict__ order, Chunk* __restrict__ chunks,
-                                           int n_chunks) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c == 0) {
-    events[0] = ev;
-    if (order) order[0] = 0;
-  }
-  if (c < n_chunks) {
-    Chunk ch{};
-    ch.event = 0;
-    ch.begin = c * kChunk;
-    ch.end = min(ev.n, (c + 1) * kChunk);
-    chunks[c] = ch;
-  }
-}
-
 }  // namespace
 
 struct clue_ctx {
@@ -162,19 +143,8 @@ clue_status run_batch(clue_ctx* ctx, const P* p, const Pts* pts, const uint32_t*
   if (st) return st;
   BatchBuffersT<T> bb;
   ResultArraysT<T> ra;
-  // One event: its descriptors are written by a kernel (one launch where the
-  // host-to-device copies of the plan take two or three).
-  const bool single = bp.events.size() == 1 && bp.events[0].p_off == 0;
-  st = prepare_batch(ctx->ws, bp, p, pts, res, ctx->stream, &bb, &ra, !single);
+  st = prepare_batch(ctx->ws, bp, p, pts, res, ctx->stream, &bb, &ra);
   if (st) return st;
-  if (single) {
-    const int n_chunks = static_cast<int>(bp.chunks.size());
-    hipLaunchKernelGGL(k_single_event_descriptors, dim3(static_cast<unsigned>((n_chunks + 255) / 256)),
-                       dim3(256), 0, ctx->stream, bp.events[0],
-                       static_cast<EventDesc*>(ctx->ws.buf[S_EVENTS].p),
-                       bb.event_order ? static_cast<int32_t*>(ctx->ws.buf[S_EORDER].p) : nullptr,
-                       static_cast<Chunk*>(ctx->ws.buf[S_CHUNKS].p), n_chunks);
-  }
   ra.event_of_cluster = event_of_cluster;
   const RunParamsT<T> rp = make_run_params(p, pts, bp);
   StageHook hook{mark_stage, ctx};
@@ -307,7 +277,7 @@ clue_status clue_make_clusters_batched(clue_ctx* ctx, const clue_params* params,
 // Allocation-free variant of clue_make_clusters: the pipeline workspace lives in
 // the static scratch of the context's device instead of the context's pooled
 // buffers. No hipMalloc, hipFree, memset or host-to-device copy: the event's
-// descriptors are written by a kernel, and every stage initialises what it reads.
+// descriptors are written by its first kernel, and every stage initialises what it reads.
 clue_status clue_make_clusters_noalloc(clue_ctx* ctx, const clue_params* params,
                                        const clue_points* points, clue_results* results) {
   if (!ctx) return fail(CLUE_ERR_INVALID_ARGUMENT, "null context");
@@ -350,12 +320,8 @@ clue_status clue_make_clusters_noalloc(clue_ctx* ctx, const clue_params* params,
                                        std::to_string(kNoAllocScratchBytes));
   BatchBuffers bb;
   ResultArrays ra;
-  st = bind_batch(slot, bp, params, points, results, ctx->stream, &bb, &ra, false);
+  st = bind_batch(slot, bp, params, points, results, ctx->stream, &bb, &ra);
   if (st) return st;
-  hipLaunchKernelGGL(k_single_event_descriptors, dim3(static_cast<unsigned>((n_chunks + 255) / 256)),
-                     dim3(256), 0, ctx->stream, bp.events[0], at<EventDesc>(slot, S_EVENTS),
-                     bp.event_order.empty() ? nullptr : at<int32_t>(slot, S_EORDER),
-                     at<Chunk>(slot, S_CHUNKS), static_cast<int>(n_chunks));
   const RunParams rp = make_run_params(params, points, bp);
   for (bool& r : ctx->ev_recorded) r = false;
   launch_pipeline(rp, point_arrays(params, points), bb, ra, ctx->stream, nullptr);

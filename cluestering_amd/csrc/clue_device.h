@@ -318,6 +318,16 @@ __device__ __forceinline__ int cvt_trunc(double q) {
   return static_cast<int>(q);
 }
 
+// Chunk k of a lone event.
+__device__ __forceinline__ Chunk lone_chunk(const LoneEvent& lone, int k) {
+  Chunk c;
+  c.event = 0;
+  c.begin = k * kPointChunk;
+  c.end = min(lone.ev.n, c.begin + kPointChunk);
+  c.pad = 0;
+  return c;
+}
+
 // Tile geometry of one event (TilesView.hpp:38-104).
 template <class T>
 struct GeoT {

@@ -76,9 +76,10 @@ struct BatchBuffersT {
   int32_t n_tiles_total;  // sum of ntiles over events
   int32_t max_items;      // upper bound of work items
   int32_t key_bits;
-  const EventDesc* events;
+  LoneEvent lone;
+  EventDesc* events;
   const int32_t* event_order;  // events largest first for the fused tile build; NULL: radix path
-  const Chunk* chunks;
+  Chunk* chunks;
   typename FloatBits<T>::Int* ext;  // [n_chunks][D][2] ordered-integer extremes
   int32_t ext_group;                // chunks per result of the extremes
   T* geo;                           // [E][3][D] mn, mx, side

@@ -120,18 +120,18 @@ U* at(void* const (&slot)[S_NUM], int k) {
 }
 // Fills the BatchBuffers and result pointers of one batch from workspace slots
 // that hold at least workspace_requests' bytes each (NULL results use workspace
-// slots) and, with `upload`, copies its descriptors from the host on stream s
-// (without, the caller writes slot[S_EVENTS] and slot[S_CHUNKS] on the device).
+// slots) and copies its descriptors from the host on stream s (a lone event's are
+// written by its first kernel, LoneEvent).
 template <class P, class Pts, class Res>
 clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P* p, const Pts* pts,
                        Res* res, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
-                       ResultArraysT<value_t<P>>* ra, bool upload);
+                       ResultArraysT<value_t<P>>* ra);
 // Reserves the workspace of one batch, uploads its descriptors on stream s and
 // fills the BatchBuffers and result pointers (NULL results use workspace buffers).
 template <class P, class Pts, class Res>
 clue_status prepare_batch(Workspace& ws, const BatchPlan& bp, const P* p, const Pts* pts,
                           Res* res, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
-                          ResultArraysT<value_t<P>>* ra, bool upload = true);
+                          ResultArraysT<value_t<P>>* ra);
 
 struct ScopedDevice {
   int prev = 0;

@@ -246,12 +246,12 @@ WorkspaceShape workspace_shape(const BatchPlan& bp, const P* p, const Pts* pts, 
 }
 
 // Fills the BatchBuffers and result pointers of one batch from workspace slots
-// (each at least workspace_requests' bytes) and, with `upload`, enqueues the
+// (each at least workspace_requests' bytes) and, for several events, enqueues the
 // descriptor uploads on the stream (they precede any kernel that reads them).
 template <class P, class Pts, class Res>
 clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P* p, const Pts* pts,
                        Res* res, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
-                       ResultArraysT<value_t<P>>* ra, bool upload) {
+                       ResultArraysT<value_t<P>>* ra) {
   using T = value_t<P>;
   using I = typename FloatBits<T>::Int;
   const int D = p->ndim;
@@ -264,7 +264,8 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   const bool nhb = nh_blocks_enabled(p, pts, bp);
   const int64_t h_blocks = nhb ? (n + kNhBlock - 1) / kNhBlock + NT + 1 : 0;
   const int64_t h_slots = h_blocks * kNhBlock;
-  if (upload) {
+  const bool lone = E == 1 && bp.events[0].p_off == 0;
+  if (!lone) {
     CLUE_HIP(hipMemcpyAsync(slot[S_EVENTS], bp.events.data(), sizeof(EventDesc) * E,
                             hipMemcpyHostToDevice, s));
     CLUE_HIP(hipMemcpyAsync(slot[S_CHUNKS], bp.chunks.data(), sizeof(Chunk) * C,
@@ -281,6 +282,8 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   b.n_tiles_total = static_cast<int32_t>(NT);
   b.max_items = static_cast<int32_t>(bp.max_items);
   b.key_bits = bp.key_bits;
+  b.lone.is = lone ? 1 : 0;
+  if (lone) b.lone.ev = bp.events[0];
   b.events = at<EventDesc>(slot, S_EVENTS);
   b.event_order = bp.event_order.empty() ? nullptr : at<int32_t>(slot, S_EORDER);
   b.chunks = at<Chunk>(slot, S_CHUNKS);
@@ -341,13 +344,13 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
 template <class P, class Pts, class Res>
 clue_status prepare_batch(Workspace& ws, const BatchPlan& bp, const P* p, const Pts* pts,
                           Res* res, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
-                          ResultArraysT<value_t<P>>* ra, bool upload) {
+                          ResultArraysT<value_t<P>>* ra) {
   size_t need[S_NUM];
   workspace_requests(workspace_shape(bp, p, pts, res), need);
   for (int k = 0; k < S_NUM; ++k) CLUE_HIP(ws.buf[k].reserve(need[k]));
   void* slot[S_NUM];
   for (int k = 0; k < S_NUM; ++k) slot[k] = ws.buf[k].p;
-  return bind_batch(slot, bp, p, pts, res, s, bb, ra, upload);
+  return bind_batch(slot, bp, p, pts, res, s, bb, ra);
 }
 
 template <class P, class Pts>
@@ -386,15 +389,15 @@ template WorkspaceShape workspace_shape(const BatchPlan&, const clue_params_f64*
                                        const clue_points_f64*, const clue_results_f64*);
 template clue_status bind_batch(void* const (&)[S_NUM], const BatchPlan&, const clue_params*,
                                 const clue_points*, clue_results*, hipStream_t,
-                                BatchBuffersT<float>*, ResultArraysT<float>*, bool);
+                                BatchBuffersT<float>*, ResultArraysT<float>*);
 template clue_status bind_batch(void* const (&)[S_NUM], const BatchPlan&, const clue_params_f64*,
                                 const clue_points_f64*, clue_results_f64*, hipStream_t,
-                                BatchBuffersT<double>*, ResultArraysT<double>*, bool);
+                                BatchBuffersT<double>*, ResultArraysT<double>*);
 template clue_status prepare_batch(Workspace&, const BatchPlan&, const clue_params*,
                                    const clue_points*, clue_results*, hipStream_t,
-                                   BatchBuffersT<float>*, ResultArraysT<float>*, bool);
+                                   BatchBuffersT<float>*, ResultArraysT<float>*);
 template clue_status prepare_batch(Workspace&, const BatchPlan&, const clue_params_f64*,
                                    const clue_points_f64*, clue_results_f64*, hipStream_t,
-                                   BatchBuffersT<double>*, ResultArraysT<double>*, bool);
+                                   BatchBuffersT<double>*, ResultArraysT<double>*);
 
 }  // namespace clue_rt

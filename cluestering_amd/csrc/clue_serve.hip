@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "clue_amd.h"
+#include "clue_device.h"
 #include "clue_runtime.h"
 #include "clue_serve_core.h"
 
@@ -40,11 +41,14 @@ struct ReqDesc {
   int32_t dst;  // first point in the batch
 };
 
-// Staging block of every event -> batch SoA columns (coordinates, then weights).
-__global__ void k_repack(const ReqDesc* __restrict__ reqs, const clue_dev::Chunk* __restrict__ chunks,
+// Staging block of every event -> batch SoA columns (coordinates, then weights). It
+// runs before the pipeline, whose first kernel writes a lone event's chunks.
+__global__ void k_repack(const ReqDesc* __restrict__ reqs, const clue_dev::LoneEvent lone,
+                         const clue_dev::Chunk* __restrict__ chunks,
                          const float* __restrict__ staging, float* __restrict__ cols, int D,
                          int64_t n_total) {
-  const clue_dev::Chunk ch = chunks[blockIdx.x];
+  const clue_dev::Chunk ch =
+      lone.is ? clue_dev::lone_chunk(lone, blockIdx.x) : chunks[blockIdx.x];
   const ReqDesc r = reqs[ch.event];
   for (int i = ch.begin + threadIdx.x; i < ch.end; i += blockDim.x) {
     const int k = i - r.dst;
@@ -285,7 +289,7 @@ class HipLanes : public clue_srv::ServeBackend {
     if (st) return st;
     ra.local_ids = 1;
     hipLaunchKernelGGL(k_repack, dim3(bb.n_chunks), dim3(256), 0, L.stream,
-                       L.reqdesc.as<ReqDesc>(), bb.chunks, staging, cols, D, n_total);
+                       L.reqdesc.as<ReqDesc>(), bb.lone, bb.chunks, staging, cols, D, n_total);
     const RunParams rp = make_run_params(&p, &pts, L.plan);
     launch_pipeline(rp, point_arrays(&p, &pts), bb, ra, L.stream, nullptr);
     CLUE_HIP(hipGetLastError());

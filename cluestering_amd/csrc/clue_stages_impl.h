@@ -121,15 +121,25 @@ struct CoordPtrs {
 // address as there are workgroups (18 us for 2^20 points, 9 us this way).
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_extremes(CoordPtrs<T> c, int D,
-                                                     const Chunk* __restrict__ chunks,
-                                                     const EventDesc* __restrict__ events, int group,
+                                                     const LoneEvent lone,
+                                                     Chunk* __restrict__ chunks,
+                                                     EventDesc* __restrict__ events, int group,
                                                      typename FloatBits<T>::Int* __restrict__ ext) {
   using I = typename FloatBits<T>::Int;
   constexpr I kHi = std::numeric_limits<I>::max(), kLo = std::numeric_limits<I>::min();
-  const Chunk ch = chunks[blockIdx.x];
+  Chunk ch;
+  if (lone.is) {  // its descriptors, for the stages that follow
+    ch = lone_chunk(lone, blockIdx.x);
+    if (threadIdx.x == 0) {
+      chunks[blockIdx.x] = ch;
+      if (blockIdx.x == 0) events[0] = lone.ev;
+    }
+  } else {
+    ch = chunks[blockIdx.x];
+  }
   int end = ch.end;
   if (group > 1) {
-    const EventDesc ev = events[ch.event];
+    const EventDesc ev = lone.is ? lone.ev : events[ch.event];
     if ((ch.begin - ev.p_off) / kPointChunk % group != 0) return;
     end = min(ev.p_off + ev.n, ch.begin + group * kPointChunk);
   }
@@ -319,8 +329,9 @@ constexpr int kEvtRounds = 4;
 
 template <int D, class T>
 __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
-    const RunParamsT<T> rp, const EventDesc* __restrict__ events, const int32_t* __restrict__ order,
-    const PointArraysT<T> in, const SortedArraysT<T> out, T* __restrict__ geo,
+    const RunParamsT<T> rp, const LoneEvent lone, EventDesc* __restrict__ events,
+    const int32_t* __restrict__ order, const PointArraysT<T> in, const SortedArraysT<T> out,
+    T* __restrict__ geo,
     int32_t* __restrict__ toff, int32_t* __restrict__ iperm, int n_tiles_total, int n_total) {
   using I = typename FloatBits<T>::Int;
   constexpr I kHi = std::numeric_limits<I>::max(), kLo = std::numeric_limits<I>::min();
@@ -328,8 +339,9 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
   __shared__ I red[kEvtWaves][2 * D];
   __shared__ T sgeo[3 * D];
   __shared__ int32_t wsum[kEvtWaves];
-  const int e = order[blockIdx.x];
-  const EventDesc ev = events[e];
+  const int e = lone.is ? 0 : order[blockIdx.x];
+  const EventDesc ev = lone.is ? lone.ev : events[e];
+  if (lone.is && threadIdx.x == 0) events[0] = ev;  // for the stages that follow
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   const int b0 = ev.p_off, n = ev.n;
@@ -498,7 +510,7 @@ template <int D, class T>
 static void launch_event_tiles_d(const RunParamsT<T>& rp, const PointArraysT<T>& in,
                                  const BatchBuffersT<T>& bb, hipStream_t s) {
   hipLaunchKernelGGL((k_event_tiles<D, T>), dim3(static_cast<unsigned>(bb.n_events)),
-                     dim3(kEvtBlock), 0, s, rp, bb.events, bb.event_order, in, bb.sorted, bb.geo,
+                     dim3(kEvtBlock), 0, s, rp, bb.lone, bb.events, bb.event_order, in, bb.sorted, bb.geo,
                      bb.toff, bb.iperm, bb.n_tiles_total, bb.n_total);
 }
 
@@ -900,35 +912,35 @@ __device__ __forceinline__ void write_nh_layout(int t, int b, int cnt, const int
   }
 }
 
-// One wave per tile: its work items and (tbox) its points' bounding box, by which the
+// Tile t (one wave): its work items and (tbox) its points' bounding box, by which the
 // density stage leaves out the tiles none of a wave's queries can reach.
+struct TileSetup {
+  const EventDesc* events;
+  int n_events;
+  Item* items;
+  const int32_t* ioff;
+  int32_t max_items;
+};
 template <int D, class T>
-__global__ __launch_bounds__(kBlock) void k_tile_setup(
-    const int32_t* __restrict__ toff, int n_tiles, const EventDesc* __restrict__ events,
-    int n_events, const T* __restrict__ sx, int64_t cs, T* __restrict__ tbox,
-    Item* __restrict__ items, const int32_t* __restrict__ ioff, int32_t max_items,
-    int32_t* __restrict__ ctl) {
-  if (blockIdx.x == 0 && threadIdx.x >= kQueueDensity && threadIdx.x < kQueueWords)
-    ctl[threadIdx.x] = 0;  // work-item queue counters
-  const int t = blockIdx.x * kWaves + threadIdx.x / kWave;
-  if (t >= n_tiles) return;
-  const int b = toff[t], e = toff[t + 1];
+__device__ __forceinline__ void tile_setup(const TileSetup& a, int t, int n_tiles, int b, int e,
+                                           const T* __restrict__ sx, int64_t cs,
+                                           T* __restrict__ tbox) {
   // The first points' loads go out before the search for the event.
   T x0[D];
 #pragma unroll
   for (int d = 0; d < D; ++d)
     x0[d] = (tbox && b + lane_id() < e) ? sx[d * cs + b + lane_id()] : std::numeric_limits<T>::quiet_NaN();
-  const int e_t = tile_event(events, n_events, t);
-  const int first = first_item(ioff, b, t);
-  const int slots = ioff ? (e - b + kWave - 1) / kWave
-                         : (t + 1 < n_tiles ? first_item(ioff, e, t + 1) : max_items) - first;
+  const int e_t = tile_event(a.events, a.n_events, t);
+  const int first = first_item(a.ioff, b, t);
+  const int slots = a.ioff ? (e - b + kWave - 1) / kWave
+                         : (t + 1 < n_tiles ? first_item(a.ioff, e, t + 1) : a.max_items) - first;
   for (int k = lane_id(); k < slots; k += kWave) {
     Item it;
     it.tile = t;
     it.begin = min(e, b + k * kWave);
     it.end = min(e, it.begin + kWave);
     it.event = e_t;
-    items[first + k] = it;
+    a.items[first + k] = it;
   }
   if (!tbox) return;
   T mn[D], mx[D];
@@ -959,6 +971,22 @@ __global__ __launch_bounds__(kBlock) void k_tile_setup(
   }
 }
 
+__device__ __forceinline__ void zero_queues(int32_t* __restrict__ ctl) {
+  if (threadIdx.x >= kQueueDensity && threadIdx.x < kQueueWords) ctl[threadIdx.x] = 0;
+}
+
+// The setup alone, where the queries keep their order.
+template <int D, class T>
+__global__ __launch_bounds__(kBlock) void k_tile_setup(const TileSetup setup,
+                                                       const int32_t* __restrict__ toff, int n_tiles,
+                                                       const T* __restrict__ sx, int64_t cs,
+                                                       T* __restrict__ tbox,
+                                                       int32_t* __restrict__ ctl) {
+  if (blockIdx.x == 0) zero_queues(ctl);
+  const int t = blockIdx.x * kWaves + threadIdx.x / kWave;
+  if (t < n_tiles) tile_setup<D>(setup, t, n_tiles, toff[t], toff[t + 1], sx, cs, tbox);
+}
+
 // The query order of W tiles per workgroup (8 for a lone event, whose dense tiles are
 // the largest, else 4: one event of 2^20 points 81 us at 4 and 54 us at 8, the
 // 4096-event batch 744 us and 990 us). A tile of at most one wave's
@@ -971,9 +999,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_setup(
 // within the nearest-higher layout.
 template <int D, int W, class T>
 __global__ __launch_bounds__(W * kWave) void k_query_order(
-    const RunParamsT<T> rp, const EventDesc* __restrict__ events, const Item* __restrict__ items,
-    const int32_t* __restrict__ ioff, const T* __restrict__ geo, const int32_t* __restrict__ toff,
-    int n_tiles, const T* __restrict__ sx, int64_t cs, int32_t* __restrict__ qfine,
+    const RunParamsT<T> rp, const TileSetup setup, T* __restrict__ tbox, int32_t* __restrict__ ctl,
+    const T* __restrict__ geo, const int32_t* __restrict__ toff, int n_tiles, const T* __restrict__ sx, int64_t cs, int32_t* __restrict__ qfine,
     T* __restrict__ hx, int64_t hs, int32_t* __restrict__ hidx, T* __restrict__ hbox) {
   constexpr int kD = D < kQueryDims ? D : kQueryDims;
   constexpr int kFineBits = (8 / kD) * kD;
@@ -987,6 +1014,8 @@ __global__ __launch_bounds__(W * kWave) void k_query_order(
   {
     const int t = blockIdx.x * W + w;
     const int b = t < n_tiles ? toff[t] : 0, e = t < n_tiles ? toff[t + 1] : 0;
+    if (blockIdx.x == 0) zero_queues(ctl);
+    if (t < n_tiles) tile_setup<D>(setup, t, n_tiles, b, e, sx, cs, tbox);
     if (t < n_tiles && e - b <= kWave) {  // one item: the query order is irrelevant
       if (b + lane < e) qfine[b + lane] = b + lane;
       if (hx) write_nh_layout<D>(t, b, e - b, nullptr, 0, 1, sx, cs, hx, hs, hidx, hbox);
@@ -997,10 +1026,8 @@ __global__ __launch_bounds__(W * kWave) void k_query_order(
     if (t >= n_tiles) break;
     const int b = toff[t], e = toff[t + 1];
     if (e - b <= kWave) continue;
-    // Event of tile t: that of its first work item, where a search over the events
-    // takes a dozen dependent loads.
-    const int ev_i = items[first_item(ioff, b, t)].event;
-    const EventDesc ev = events[ev_i];
+    const int ev_i = tile_event(setup.events, setup.n_events, t);
+    const EventDesc ev = setup.events[ev_i];
     const GeoT<T> g = event_geo(geo, rp, ev_i, ev.nper);
     int tb[D];
     {
@@ -2196,15 +2223,15 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
     const T* __restrict__ srho, int32_t* __restrict__ snh, const T* __restrict__ sdelta,
     const T* __restrict__ su, T* __restrict__ rho, int32_t* __restrict__ nh, T* __restrict__ delta,
     int32_t* __restrict__ is_seed, int32_t* __restrict__ rank, int32_t* __restrict__ event_seeds,
-    int32_t* __restrict__ lone_offsets, int32_t* __restrict__ lone_total,
-    int32_t* __restrict__ cluster) {
+    const LoneEvent lone, int32_t* __restrict__ lone_total, int32_t* __restrict__ lone_seeds,
+    int32_t* __restrict__ event_of_cluster, int32_t* __restrict__ cluster) {
   constexpr int kWordsPerThread = kEvtBitWords / kEvtBlock;
   __shared__ uint32_t pool[kSeedPoolWords];
   __shared__ int32_t wsum[kEvtWaves];
   uint32_t* bits = pool;
   int16_t* links = reinterpret_cast<int16_t*>(pool + kLdsBitWords);
-  const int e = order[blockIdx.x];
-  const EventDesc ev = events[e];
+  const int e = lone.is ? 0 : order[blockIdx.x];
+  const EventDesc ev = lone.is ? lone.ev : events[e];
   const int b0 = ev.p_off, n = ev.n;
   const bool in_lds = n <= kEvtLdsLinks;
   const int n_words = in_lds ? kLdsBitWords : kEvtBitWords;  // bit words in use
@@ -2276,7 +2303,13 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
       if (in_lds) {
         // The event's seed list in rank order, and the seed's link: its rank as
         // a code (-3 - rank) that the jumping passes carry to its followers.
-        rank[b0 + run] = b0 + ii;
+        // A lone event's ranks are final.
+        if (lone.is) {
+          lone_seeds[run] = ii;
+          if (event_of_cluster) event_of_cluster[run] = ev.index;
+        } else {
+          rank[b0 + run] = b0 + ii;
+        }
         links[iperm[b0 + ii] - b0] = static_cast<int16_t>(-3 - run);
         ++run;
       } else {
@@ -2286,10 +2319,7 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
   }
   if (threadIdx.x == 0) {
     event_seeds[e] = total;
-    if (lone_total) {  // a batch of one event: the scan over events is the identity
-      lone_offsets[0] = 0;
-      *lone_total = total;
-    }
+    if (lone.is) *lone_total = total;
   }
   // Pointer jumping on the event's links: a pass replaces a link by its target's link
   // when that target is itself a follower, which halves every chain (at least); any
@@ -2616,9 +2646,10 @@ CLUE_NEIGHBOUR_EXTERN(10)
 template <int D, class T>
 static void launch_query_order_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
+  const TileSetup setup{b.events, b.n_events, b.items, b.icount, b.max_items};
   auto go = [&](auto kern, int waves) {
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((b.n_tiles_total + waves - 1) / waves)),
-                       dim3(waves * kWave), 0, L.s, *L.rp, b.events, b.items, b.icount, b.geo, b.toff,
+                       dim3(waves * kWave), 0, L.s, *L.rp, setup, b.tbox, b.n_items, b.geo, b.toff,
                        b.n_tiles_total, b.sorted.x[0], L.cs, b.qfine, b.hx, b.h_stride, b.hidx,
                        b.hbox);
   };
@@ -2632,9 +2663,9 @@ template <int D, class T>
 static void launch_tile_setup_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
   const unsigned grid = static_cast<unsigned>((b.n_tiles_total + kWaves - 1) / kWaves);
-  hipLaunchKernelGGL((k_tile_setup<D, T>), dim3(grid), dim3(kBlock), 0, L.s, b.toff,
-                     b.n_tiles_total, b.events, b.n_events, b.sorted.x[0], L.cs, b.tbox, b.items,
-                     b.icount, b.max_items, b.n_items);
+  const TileSetup setup{b.events, b.n_events, b.items, b.icount, b.max_items};
+  hipLaunchKernelGGL((k_tile_setup<D, T>), dim3(grid), dim3(kBlock), 0, L.s, setup, b.toff,
+                     b.n_tiles_total, b.sorted.x[0], L.cs, b.tbox, b.n_items);
 }
 
 template <class T>
@@ -2653,7 +2684,7 @@ static void launch_tile_setup(const NeighbourLaunch<T>& L) {
   }
 }
 
-// The query order of both neighbour stages.
+// The query order of both neighbour stages, with the work items and tile boxes.
 template <class T>
 static void launch_query_order(const NeighbourLaunch<T>& L) {
   switch (L.rp->D) {
@@ -2705,8 +2736,8 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
     mark(kStageTiles);
     launch_event_tiles(rp, in, bb, s);
   } else {
-  hipLaunchKernelGGL(k_extremes<T>, dim3(bb.n_chunks), dim3(kBlock), 0, s, cp, D, bb.chunks,
-                     bb.events, bb.ext_group, bb.ext);
+  hipLaunchKernelGGL(k_extremes<T>, dim3(bb.n_chunks), dim3(kBlock), 0, s, cp, D, bb.lone,
+                     bb.chunks, bb.events, bb.ext_group, bb.ext);
   mark(kStageTiles);
   const RadixPlan digits = radix_plan(bb.key_bits);
   hipLaunchKernelGGL(k_tile_keys<T>, dim3(bb.n_chunks), dim3(kBlock), 0, s, cp, rp, bb.chunks,
@@ -2745,8 +2776,10 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
                        0, s, bb.toff, bb.n_tiles_total, bb.icount);
     scan_exclusive(bb.icount, bb.icount, bb.n_tiles_total, bb.scan_tmp, bb.n_items, s);
   }
-  launch_tile_setup(L);                 // work items and tile boxes
-  if (bb.qfine) launch_query_order(L);  // query order of the two neighbour stages
+  if (bb.qfine)
+    launch_query_order(L);  // with the work items and tile boxes
+  else
+    launch_tile_setup(L);
 
   // (b), (c)
   mark(kStageDensity);
@@ -2757,17 +2790,19 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
   // (d), (e)
   mark(kStageSeeds);
   if (bb.event_order) {
-    const bool lone = bb.n_events == 1;
     hipLaunchKernelGGL(k_event_seeds<T>, dim3(static_cast<unsigned>(bb.n_events)), dim3(kEvtBlock),
                        0, s, rp, bb.events, bb.event_order, bb.sorted.perm, bb.iperm, bb.srho, bb.snh,
                        bb.sdelta, bb.sorted.u, out.rho, out.nh, out.delta, out.is_seed, bb.rank,
-                       bb.event_seeds, lone ? bb.event_offsets : nullptr, lone ? bb.n_seeds : nullptr,
+                       bb.event_seeds, bb.lone, bb.n_seeds, bb.seeds, out.event_of_cluster,
                        out.cluster);
-    if (!lone) scan_exclusive(bb.event_seeds, bb.event_offsets, bb.n_events, bb.scan_tmp, bb.n_seeds, s);
     mark(kStageLabels);
-    hipLaunchKernelGGL(k_event_labels, dim3(bb.n_chunks), dim3(kBlock), 0, s, bb.chunks, bb.events,
-                       bb.sorted.perm, bb.snh, bb.rank, bb.event_offsets, bb.event_seeds,
-                       out.cluster, bb.seeds, out.event_of_cluster, out.local_ids);
+    // A lone event (small enough for the LDS links, plan_batch) is done.
+    if (!bb.lone.is) {
+      scan_exclusive(bb.event_seeds, bb.event_offsets, bb.n_events, bb.scan_tmp, bb.n_seeds, s);
+      hipLaunchKernelGGL(k_event_labels, dim3(bb.n_chunks), dim3(kBlock), 0, s, bb.chunks, bb.events,
+                         bb.sorted.perm, bb.snh, bb.rank, bb.event_offsets, bb.event_seeds,
+                         out.cluster, bb.seeds, out.event_of_cluster, out.local_ids);
+    }
   } else {
     const int words = (n + 31) / 32;
     uint32_t* bits = reinterpret_cast<uint32_t*>(bb.flag);

@@ -78,6 +78,14 @@ struct Chunk {
   int32_t pad;
 };
 
+// The descriptor of a run's only event, as a kernel argument: the pipeline's first
+// kernel writes the descriptors in memory from it (a launch, or two copies, fewer per
+// call). A kernel before the pipeline takes its chunks from here too (lone_chunk).
+struct LoneEvent {
+  int32_t is;  // the run has one event, at offset 0
+  EventDesc ev;
+};
+
 // A work item of the neighbour stages: up to 64 consecutive tile-sorted points of
 // one tile (one lane each).
 struct Item {

@@ -444,3 +444,21 @@ def test_equal_tags_keep_the_first_candidate(gpu_ctx, oracle_mod, fixed):
                oracle_mod)
     finally:
         gpu_ctx.set_tuning()
+
+
+@pytest.mark.parametrize("sizes", [(0, 0, 300, 0), (0, 8193, 0), (0, 30000)])
+def test_lone_event_among_empty_ones(gpu_ctx, oracle_mod, sizes):
+    """One event with points in the batch: its descriptor goes as a kernel argument."""
+    from cluestering_amd.device import Clusterer, PointsDevice
+    rng = np.random.default_rng(4)
+    sizes = np.array(sizes, np.uint32)
+    c, w = (np.ascontiguousarray(a) for a in synthetic._event2d(rng, int(sizes.sum())))
+    kern = K.GaussianKernel(1.0, 1.0)
+    _, ref = _check(Case(c, w, 1.5, 5.0, 2.0, kernel=kern, sizes=sizes, name=f"lone {sizes}"),
+                    gpu_ctx, oracle_mod)
+    pts = PointsDevice.from_host(gpu_ctx, c, w)
+    eoc = gpu_ctx.empty(w.size, np.int32)
+    k = Clusterer(gpu_ctx, 1.5, 5.0, 2.0).make_clusters_batched(pts, sizes, None, kern,
+                                                              event_of_cluster=eoc)
+    assert k == ref.n_seeds
+    np.testing.assert_array_equal(eoc.to_host()[:k], ref.event_of_cluster)

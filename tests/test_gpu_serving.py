@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from cluestering_amd import _capi
-from cluestering_amd.serving import Server, make_pool, run_stream, served_params
+from cluestering_amd.serving import ServedEvent, Server, make_pool, run_stream, served_params
 
 pytestmark = pytest.mark.gpu
 
@@ -89,3 +89,16 @@ def test_batches_respect_the_hbm_budget():
             srv.submit(huge.params, huge.data)
     assert all(t["batch_points"] * 100 <= budget // 2 for _, t in results)
     assert max(t["batch_events"] for _, t in results) >= 1
+
+
+@pytest.mark.parametrize("n", [1, 64, 2049, 8193, 120000])
+def test_served_one_at_a_time(gpu_ctx, n):
+    """A launch of one event, whose descriptor the pipeline's first kernel writes."""
+    rng = np.random.default_rng(n)
+    side = max(1.0, np.sqrt(n / 20.0))
+    data = np.concatenate([rng.uniform(0, side, (2, n)), rng.uniform(0.5, 1.5, (1, n))])
+    ev = ServedEvent(2, np.ascontiguousarray(data, dtype=np.float32), served_params(2))
+    with Server(n_lanes=1) as srv:
+        labels, t = srv.wait(srv.submit(ev.params, ev.data))
+    assert t["batch_events"] == 1
+    np.testing.assert_array_equal(labels, _alone(gpu_ctx, ev))
