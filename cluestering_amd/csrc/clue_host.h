@@ -201,7 +201,7 @@ struct WorkspaceShape {
   bool event_tiles = false;        // the fused per-event tile build (no radix-sort buffers)
   bool group_queries = false;
   bool separate_dm_order = false;  // dm != dc and the plain nearest-higher scan
-  bool nh_blocks = false;          // nearest-higher over the Morton block layout
+  bool nh_blocks = false;          // nearest-higher over the Hilbert block layout
   bool flat_kernel = false;
   bool has_sigma = false;
   bool has_u = false;
@@ -209,7 +209,7 @@ struct WorkspaceShape {
   bool own_nh = false;
   bool own_is_seed = false;
   bool sorted_boxes = false;       // density leaves out tiles by their bounding boxes
-  bool density_morton = false;     // density takes the Morton order (no class order for dc)
+  bool density_morton = false;     // density takes the Hilbert order (no class order for dc)
 };
 
 // Bytes of every workspace slot for a batch of this shape (0: unused).

@@ -93,7 +93,7 @@ struct BatchBuffersT {
   int32_t* icount;     // [n_tiles_total] first item of every tile; NULL: from the offsets (teams)
   int32_t* n_items;    // number of items (with icount), then the work-item queue counters
   Item* items;         // [max_items]
-  int32_t* qfine;      // [n_total] query order of both neighbour stages, the Morton order
+  int32_t* qfine;      // [n_total] query order of both neighbour stages, the Hilbert order
                        // within tiles; NULL = sorted order
   T* srho;
   uint64_t* skey;      // ordering key of every sorted point: float (rho, tag); double rho
@@ -110,7 +110,7 @@ struct BatchBuffersT {
   SortedArraysT<T> sorted;
   int64_t sorted_stride;  // column stride of sorted.x[] and sorted.sigma[] blocks
   // Nearest-higher block layout (NULL when not used): each tile's candidates in
-  // Morton order from block ceil(toff[t] / kNhBlock) + t on, padded to whole
+  // Hilbert order from block ceil(toff[t] / kNhBlock) + t on, padded to whole
   // blocks with key 0 (never higher) and index -1.
   T* hx;             // [D][h_stride] coordinates
   uint64_t* hkey;    // [h_stride] ordering keys

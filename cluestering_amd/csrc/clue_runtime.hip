@@ -94,8 +94,8 @@ bool sorted_boxes_enabled(const P* p) {
   return p->metric != CLUE_METRIC_MAHALANOBIS && weights_not_negative(p);
 }
 
-// Whether the nearest-higher stage runs over the Morton-ordered block layout:
-// it needs the Morton order of the query grouping, candidates visited in any
+// Whether the nearest-higher stage runs over the Hilbert-ordered block layout:
+// it needs the Hilbert order of the query grouping, candidates visited in any
 // order (unique tags: the default ones), and a metric with a lower bound over a
 // bounding box.
 template <class P, class Pts>

@@ -5,7 +5,7 @@
 //       points of one tile, one lane each) walks the union of the lanes' search
 //       boxes in the reference's lexicographic tile order; candidates are
 //       wave-uniform and come through the scalar cache. With the default tags,
-//       (c) instead scans each tile's candidates in Morton-ordered blocks and
+//       (c) instead scans each tile's candidates in Hilbert-ordered blocks and
 //       skips the blocks that cannot hold the answer (its result does not
 //       depend on the visiting order);
 //   (d) seeds, numbered by an exclusive scan in input order;
@@ -734,21 +734,34 @@ __device__ __forceinline__ void walk_tiles(const int (&lo)[D], const int (&hi)[D
 // ---------------------------------------------------------------------------
 // Query order within a tile. A wave pays for the candidates that any of its lanes can
 // reach, so the points of every tile with more than one wave's worth are ordered by
-// the Morton index of their sub-cell of the tile; items then take 64 consecutive
+// the Hilbert index of their sub-cell of the tile; items then take 64 consecutive
 // entries. Results do not depend on the order: a point's traversal is its own,
 // whichever lane runs it. (An order by which neighbouring tiles a point's search box
-// reaches, kept within the Morton order, measured no faster once candidates were
+// reaches, kept within the Hilbert order, measured no faster once candidates were
 // culled by the wave's box.)
 // ---------------------------------------------------------------------------
 constexpr int kQueryDims = 3;  // dimensions that enter the keys
 
-// Morton index of the point's sub-cell: 8 bits over the first (up to) three
-// dimensions of the tile, bits interleaved from the most significant.
-template <int D, class T>
-__device__ __forceinline__ uint32_t query_fine(const GeoT<T>& g, const T (&xi)[D],
+// Hilbert index of the point's sub-cell over the first (up to) three dimensions of the
+// tile, kCellBits bits per dimension: the curve's steps between neighbouring cells keep
+// the 64 consecutive points of an item in a smaller box than a Morton order's jumps
+// (4096-event batch, 4 bits: density 23.0 -> 22.4 ms, nearest-higher 7.6 -> 6.8 ms).
+// Fine cells order dense tiles further (5 bits: 22.1 and 6.5 ms; 2^20 points in 2-D,
+// nearest-higher 404 -> 275 us; 6 bits gain no more and sort slower); small launches
+// take the coarse ones, whose sort is shorter (5,003 points: 12 against 15 us). The
+// index follows Skilling's transform ("Programming the Hilbert curve", AIP Conf. Proc. 707,
+// 2004): rotations undone from the top bit down, a Gray code, the bits interleaved.
+template <int D, bool Fine>
+struct QueryCells {
+  static constexpr int kDims = D < kQueryDims ? D : kQueryDims;
+  static constexpr int kCellBits = kDims == 1 ? 8 : kDims == 2 ? (Fine ? 5 : 4) : (Fine ? 3 : 2);
+  static constexpr int kBins = 1 << (kDims * kCellBits);
+};
+template <int D, bool Fine, class T>
+__device__ __forceinline__ uint32_t query_cell(const GeoT<T>& g, const T (&xi)[D],
                                                const int (&tb)[D]) {
-  constexpr int kD = D < kQueryDims ? D : kQueryDims;
-  constexpr int kB = 8 / kD;  // bits per dimension
+  constexpr int kD = QueryCells<D, Fine>::kDims;
+  constexpr int kB = QueryCells<D, Fine>::kCellBits;
   constexpr int kS = 1 << kB;
   uint32_t q[kD];
 #pragma unroll
@@ -756,6 +769,26 @@ __device__ __forceinline__ uint32_t query_fine(const GeoT<T>& g, const T (&xi)[D
     const T c = g.wrapped[d] ? normalize(g, xi[d], d) : xi[d];
     const T f = ((c - g.mn[d]) / g.side[d] - static_cast<T>(tb[d])) * static_cast<T>(kS);
     q[d] = (f >= T(0)) ? (f < static_cast<T>(kS) ? static_cast<uint32_t>(f) : kS - 1u) : 0u;
+  }
+  if constexpr (kD > 1) {
+#pragma unroll
+    for (int b = kB - 1; b > 0; --b) {
+      const uint32_t low = (1u << b) - 1u;
+#pragma unroll
+      for (int d = 0; d < kD; ++d) {
+        const bool set = (q[d] >> b) & 1u;
+        const uint32_t t = (q[0] ^ q[d]) & low;
+        q[d] = set ? q[d] : q[d] ^ t;
+        q[0] = set ? q[0] ^ low : (d == 0 ? q[0] : q[0] ^ t);
+      }
+    }
+#pragma unroll
+    for (int d = 1; d < kD; ++d) q[d] ^= q[d - 1];
+    uint32_t t = 0;
+#pragma unroll
+    for (int b = kB - 1; b > 0; --b) t ^= ((q[kD - 1] >> b) & 1u) ? (1u << b) - 1u : 0u;
+#pragma unroll
+    for (int d = 0; d < kD; ++d) q[d] ^= t;
   }
   uint32_t key = 0;
 #pragma unroll
@@ -861,10 +894,10 @@ __device__ __forceinline__ int64_t nh_first_block(int b, int t) {
 }
 
 // The nearest-higher layout of tile t, written by the query-order pass (wave w of
-// n_waves takes every n_waves-th 64 slots): the tile's candidates in Morton order (order[k], k < cnt) from block
+// n_waves takes every n_waves-th 64 slots): the tile's candidates in Hilbert order (order[k], k < cnt) from block
 // nh_first_block on, padded to whole blocks (index -1), with each block's
 // bounding box. The keys, known after the density stage, are written by the
-// density stage itself (k_density, from the same Morton order).
+// density stage itself (k_density, from the same Hilbert order).
 template <int D, class T>
 __device__ __forceinline__ void write_nh_layout(int t, int b, int cnt, const int32_t* order,
                                                 int w, int n_waves,
@@ -991,24 +1024,22 @@ __global__ __launch_bounds__(kBlock) void k_tile_setup(const TileSetup setup,
 // the largest, else 4: one event of 2^20 points 81 us at 4 and 54 us at 8, the
 // 4096-event batch 744 us and 990 us). A tile of at most one wave's
 // points keeps its order (one wave each). The others are taken one after the other
-// by the whole workgroup, a counting sort in LDS by the Morton index: the dense
+// by the whole workgroup, a counting sort in LDS by the Hilbert index: the dense
 // tiles, thousands of points where most tiles hold a few dozen, are what one wave
 // per tile waited for (4096-event batch: 1043 -> 789 us; one event of 2^20 points
 // in 2-D: 248 -> 89 us; of 100,000: 87 -> 28 us). Points of equal index are placed by LDS atomics, in no
 // order among themselves: no result depends on the query order or on the order
 // within the nearest-higher layout.
-template <int D, int W, class T>
+template <int D, int W, bool Fine, class T>
 __global__ __launch_bounds__(W * kWave) void k_query_order(
     const RunParamsT<T> rp, const TileSetup setup, T* __restrict__ tbox, int32_t* __restrict__ ctl,
     const T* __restrict__ geo, const int32_t* __restrict__ toff, int n_tiles, const T* __restrict__ sx, int64_t cs, int32_t* __restrict__ qfine,
     T* __restrict__ hx, int64_t hs, int32_t* __restrict__ hidx, T* __restrict__ hbox) {
-  constexpr int kD = D < kQueryDims ? D : kQueryDims;
-  constexpr int kFineBits = (8 / kD) * kD;
-  constexpr int kFine = 1 << kFineBits;
+  constexpr int kBins = QueryCells<D, Fine>::kBins;
   constexpr int kOrderBlock = W * kWave;
-  constexpr int kHeld = 4;  // rounds whose Morton indices stay in registers
-  static_assert(kFine <= kOrderBlock, "one counter per thread in the scan");
-  __shared__ int32_t cnt[kFine];
+  constexpr int kHeld = 4;  // rounds whose indices stay in registers
+  constexpr int kPer = (kBins + kOrderBlock - 1) / kOrderBlock;  // bins per thread in the scan
+  __shared__ int32_t cnt[kBins];
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   {
@@ -1038,13 +1069,13 @@ __global__ __launch_bounds__(W * kWave) void k_query_order(
         r /= ev.nper;
       }
     }
-    if (threadIdx.x < kFine) cnt[threadIdx.x] = 0;
+    for (int k2 = threadIdx.x; k2 < kBins; k2 += kOrderBlock) cnt[k2] = 0;
     __syncthreads();
     auto key_of = [&](int s) {
       T xi[D];
 #pragma unroll
       for (int d = 0; d < D; ++d) xi[d] = sx[d * cs + s];
-      return query_fine<D>(g, xi, tb);
+      return query_cell<D, Fine>(g, xi, tb);
     };
     uint32_t held[kHeld];
 #pragma unroll
@@ -1058,9 +1089,19 @@ __global__ __launch_bounds__(W * kWave) void k_query_order(
       atomicAdd(&cnt[key_of(s)], 1);
     __syncthreads();
     int total;
-    const int c = threadIdx.x < kFine ? cnt[threadIdx.x] : 0;
-    const int first = block_excl_scan<kOrderBlock>(c, &total);
-    if (threadIdx.x < kFine) cnt[threadIdx.x] = b + first;
+    const int bin0 = static_cast<int>(threadIdx.x) * kPer;
+    int c[kPer], sum = 0;
+#pragma unroll
+    for (int k2 = 0; k2 < kPer; ++k2) {
+      c[k2] = bin0 + k2 < kBins ? cnt[bin0 + k2] : 0;
+      sum += c[k2];
+    }
+    int run = b + block_excl_scan<kOrderBlock>(sum, &total);
+#pragma unroll
+    for (int k2 = 0; k2 < kPer; ++k2) {
+      if (bin0 + k2 < kBins) cnt[bin0 + k2] = run;
+      run += c[k2];
+    }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kHeld; ++r) {
@@ -1596,7 +1637,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
     }
     if (hkey) {
       // The nearest-higher block layout takes the keys here: the lanes are the
-      // tile's points in Morton order (qfine) from a multiple of 64, so
+      // tile's points in Hilbert order (qfine) from a multiple of 64, so
       // lane k's point fills layout slot k of the tile and each row of 16 lanes
       // is one block, whose largest key a row reduction gives. Lanes past the
       // tile's points write the padding's key 0 up to the last block.
@@ -1863,12 +1904,12 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_nearest_higher(
 }
 
 // ---------------------------------------------------------------------------
-// (c') Nearest-higher over Morton-ordered candidate blocks. The accepted
+// (c') Nearest-higher over Hilbert-ordered candidate blocks. The accepted
 // candidate of the reference's scan is the one of smallest distance, equal
 // distances going to the larger (rho, tag); with unique tags (the default ones:
 // the input index) no two candidates tie on all three, so the result does not
 // depend on the order in which candidates are visited. Each tile's candidates
-// are laid out in Morton order in blocks of kNhBlock with the block's bounding
+// are laid out in Hilbert order in blocks of kNhBlock with the block's bounding
 // box and largest key; a wave skips a block when for each lane either no
 // candidate of the block is higher or the box lies beyond the lane's current
 // bound. A skipped block holds no candidate that the scan would accept (the box
@@ -2572,7 +2613,7 @@ static void launch_nh_blocks_dm(const NeighbourLaunch<T>& L) {
 }
 
 // Nearest-higher over the block layout: the layout pass, then the scan. Its
-// waves take each tile's points in Morton order (qfine): the scan visits only the
+// waves take each tile's points in Hilbert order (qfine): the scan visits only the
 // blocks its lanes want, so grouping lanes by search-box class buys nothing here.
 template <int D, class T>
 static void launch_nh_blocks_d(const NeighbourLaunch<T>& L) {
@@ -2653,10 +2694,11 @@ static void launch_query_order_d(const NeighbourLaunch<T>& L) {
                        b.n_tiles_total, b.sorted.x[0], L.cs, b.qfine, b.hx, b.h_stride, b.hidx,
                        b.hbox);
   };
+  const bool fine = !L.rp->team;
   if (b.n_events == 1)
-    go(k_query_order<D, 8, T>, 8);
+    go(fine ? k_query_order<D, 8, true, T> : k_query_order<D, 8, false, T>, 8);
   else
-    go(k_query_order<D, 4, T>, 4);
+    go(fine ? k_query_order<D, 4, true, T> : k_query_order<D, 4, false, T>, 4);
 }
 
 template <int D, class T>

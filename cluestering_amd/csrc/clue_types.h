@@ -128,7 +128,7 @@ struct RunParamsT {
   T mparam[kMaxDim];
   int32_t xcd_chunk_log2;  // neighbour stages: 2^k consecutive blocks per XCD turn; < 0: none
   int32_t block_waves;     // neighbour stages: waves per workgroup (1, 2, 4, 8 or 16)
-  int32_t nh_blocks;       // nearest-higher over the Morton-ordered block layout
+  int32_t nh_blocks;       // nearest-higher over the Hilbert-ordered block layout
   int32_t cull;            // density: candidates bounded by the metric's lower bound (no weight below 0)
   int32_t team;            // neighbour stages: a team of waves per item (clue_team.h)
   int32_t persistent;      // neighbour stages: persistent waves per CU pulling items (0: none)

@@ -247,11 +247,11 @@ clue_status clue_stage_times(clue_ctx* ctx, const char** names, float* us, int32
  * of the built-in table (measured on MI355X per ndim and mean event size by
  * cluestering_amd/autotune.py) that matches its batch. */
 typedef struct {
-  int32_t group_queries;  /* 1: order each tile's queries by box class and position */
+  int32_t group_queries;  /* 1: order each tile's queries by position (Hilbert) */
   int32_t xcd_chunk_log2; /* deal 2^k consecutive work-item blocks per XCD turn; -1: none */
   int32_t block_waves;    /* waves per workgroup of the neighbour stages: 1..16, power of 2 (0: 4) */
   int32_t nh_plain_scan;  /* 1: nearest-higher scans whole tiles in sorted order; 0 (default): over
-                             Morton-ordered candidate blocks, skipping blocks that cannot hold the
+                             Hilbert-ordered candidate blocks, skipping blocks that cannot hold the
                              answer, whenever tags are the default ones and the metric allows it */
   int32_t persistent;     /* 0: one wave per work item, dispatched by the hardware; k > 0: k
                              persistent waves per CU pull (event, tile) work items from per-XCD
