@@ -20,18 +20,16 @@ namespace {
 
 constexpr int kBlock = 256;
 
-__global__ void k_assoc_init(int32_t* __restrict__ stats) {
-  if (threadIdx.x == 0) {
-    stats[0] = INT32_MIN;  // max key
-    stats[1] = 0;          // keys >= 0
-  }
-}
-
+// Largest key and number of keys >= 0 of each workgroup's share, stats[2 * block] on
+// (the host combines them: results kept in one place took an atomic update per
+// workgroup, 50 us for 2^20 keys).
 __global__ __launch_bounds__(kBlock) void k_assoc_stats(const int32_t* __restrict__ keys, int n,
                                                         int32_t* __restrict__ stats) {
   __shared__ int32_t smax[kBlock / kWave], scnt[kBlock / kWave];
   int mx = INT32_MIN, cnt = 0;
-  for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+#pragma unroll 8
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * kBlock) {
     const int k = keys[i];
     mx = max(mx, k);
     cnt += k >= 0 ? 1 : 0;
@@ -51,20 +49,32 @@ __global__ __launch_bounds__(kBlock) void k_assoc_stats(const int32_t* __restric
       m = max(m, smax[k]);
       c += scnt[k];
     }
-    atomicMax(&stats[0], m);
-    atomicAdd(&stats[1], c);
+    stats[2 * blockIdx.x] = m;
+    stats[2 * blockIdx.x + 1] = c;
   }
 }
 
-// Sort key: the key itself, negative keys after every bin.
+// Sort key: the key itself, negative keys after every bin; with the first digits'
+// counts per block of the sort.
 __global__ __launch_bounds__(kBlock) void k_assoc_keys(const int32_t* __restrict__ keys, int n,
                                                        int bins, uint32_t* __restrict__ k0,
-                                                       int32_t* __restrict__ v0) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const int k = keys[i];
-  k0[i] = static_cast<uint32_t>(k >= 0 ? k : bins);
-  v0[i] = i;
+                                                       int digit_bits, int32_t* __restrict__ hist) {
+  __shared__ int32_t cnt[kRsMaxBins];
+  const int digits = 1 << digit_bits;
+  for (int d = threadIdx.x; d < digits; d += kBlock) cnt[d] = 0;
+  __syncthreads();
+  const int64_t b = static_cast<int64_t>(blockIdx.x) * kRsTileKeys;
+  const int64_t e = b + kRsTileKeys < n ? b + kRsTileKeys : n;
+#pragma unroll 8
+  for (int64_t i = b + threadIdx.x; i < e; i += kBlock) {
+    const int k = keys[i];
+    const uint32_t key = static_cast<uint32_t>(k >= 0 ? k : bins);
+    k0[i] = key;
+    atomicAdd(&cnt[key & (digits - 1)], 1);
+  }
+  __syncthreads();
+  for (int d = threadIdx.x; d < digits; d += kBlock)
+    hist[static_cast<int64_t>(d) * gridDim.x + blockIdx.x] = cnt[d];
 }
 
 // offsets[b] = first sorted position whose key is >= b (lower bound), b in [0, bins].
@@ -85,37 +95,35 @@ __global__ __launch_bounds__(kBlock) void k_assoc_offsets(const uint32_t* __rest
 
 }  // namespace
 
-void assoc_scratch_elems(int64_t n, int64_t* hist_elems, int64_t* scan_elems) {
-  *hist_elems = radix_hist_elems((n + kRsTileKeys - 1) / kRsTileKeys);
-  *scan_elems = scan_temp_elems(n) + 16;
+int64_t assoc_hist_elems(int64_t n) {
+  return radix_hist_elems((n + kRsTileKeys - 1) / kRsTileKeys);
 }
 
-hipError_t assoc_stats(const int32_t* keys, int n, int32_t* stats_dev, hipStream_t s) {
-  hipLaunchKernelGGL(k_assoc_init, dim3(1), dim3(kWave), 0, s, stats_dev);
-  const int blocks = static_cast<int>(std::min<int64_t>((n + kBlock - 1) / kBlock, 2048));
+hipError_t assoc_stats(const int32_t* keys, int n, int32_t* stats_dev, int* blocks, hipStream_t s) {
+  *blocks = static_cast<int>(
+      std::min<int64_t>((static_cast<int64_t>(n) + 8 * kBlock - 1) / (8 * kBlock), kAssocStatBlocks));
   if (n > 0)
-    hipLaunchKernelGGL(k_assoc_stats, dim3(blocks), dim3(kBlock), 0, s, keys, n, stats_dev);
+    hipLaunchKernelGGL(k_assoc_stats, dim3(*blocks), dim3(kBlock), 0, s, keys, n, stats_dev);
   return hipGetLastError();
 }
 
 hipError_t assoc_build(const int32_t* keys, int n, int bins, const AssocScratch& w,
                        int32_t* offsets, int32_t* members, int n_members, hipStream_t s) {
   if (n > 0) {
-    hipLaunchKernelGGL(k_assoc_keys, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, keys, n,
-                       bins, w.k0, w.v0);
     int bits = 0;
     while ((int64_t(1) << bits) <= bins) ++bits;  // keys lie in [0, bins]
+    const unsigned blocks =
+        static_cast<unsigned>((static_cast<int64_t>(n) + kRsTileKeys - 1) / kRsTileKeys);
+    hipLaunchKernelGGL(k_assoc_keys, dim3(blocks), dim3(kBlock), 0, s, keys, n, bins, w.k0,
+                       radix_plan(bits).bits, w.hist);
     bool in_first = true;
-    radix_sort_pairs(w.k0, w.v0, w.k1, w.v1, n, bits, w.hist, nullptr, 0, &in_first, s);
+    // The last pass leaves the members, which are the sorted values but for the
+    // negative keys' behind them, where the caller wants them.
+    radix_sort_pairs(w.k0, w.v0, w.k1, w.v1, n, bits, w.hist, nullptr, 0, members, n_members, &in_first,
+                     s);
     const uint32_t* sk = in_first ? w.k0 : w.k1;
-    const int32_t* sv = in_first ? w.v0 : w.v1;
     hipLaunchKernelGGL(k_assoc_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0,
                        s, sk, n, bins, offsets);
-    if (n_members > 0) {
-      hipError_t e = hipMemcpyAsync(members, sv, sizeof(int32_t) * n_members,
-                                    hipMemcpyDeviceToDevice, s);
-      if (e != hipSuccess) return e;
-    }
   } else {
     hipLaunchKernelGGL(k_assoc_offsets, dim3(1), dim3(kBlock), 0, s, w.k0, 0, 0, offsets);
   }

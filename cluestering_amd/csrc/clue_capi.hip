@@ -468,20 +468,25 @@ clue_status clue_make_association(clue_ctx* ctx, const int32_t* keys, int32_t n,
   if (n < 0) return fail(CLUE_ERR_INVALID_ARGUMENT, "negative size");
   ScopedDevice dev(ctx->device);
   Workspace& w = ctx->aux;
-  int64_t hist = 0, scan = 0;
-  assoc_scratch_elems(n, &hist, &scan);
   CLUE_HIP(w.buf[S_K0].reserve(sizeof(uint32_t) * n + 4));
   CLUE_HIP(w.buf[S_V0].reserve(sizeof(int32_t) * n + 4));
   CLUE_HIP(w.buf[S_K1].reserve(sizeof(uint32_t) * n + 4));
   CLUE_HIP(w.buf[S_V1].reserve(sizeof(int32_t) * n + 4));
-  CLUE_HIP(w.buf[S_HIST].reserve(sizeof(int32_t) * hist));
-  CLUE_HIP(w.buf[S_SCAN].reserve(sizeof(int32_t) * scan));
-  CLUE_HIP(w.buf[S_NSEEDS].reserve(sizeof(int32_t) * 4));
+  CLUE_HIP(w.buf[S_HIST].reserve(sizeof(int32_t) * assoc_hist_elems(n)));
+  CLUE_HIP(w.buf[S_NSEEDS].reserve(sizeof(int32_t) * 2 * kAssocStatBlocks));
   int32_t* stats = w.buf[S_NSEEDS].as<int32_t>();
-  CLUE_HIP(assoc_stats(keys, n, stats, ctx->stream));
-  int32_t hs[2] = {0, 0};
-  CLUE_HIP(hipMemcpyAsync(hs, stats, sizeof(hs), hipMemcpyDeviceToHost, ctx->stream));
+  int blocks = 0;
+  CLUE_HIP(assoc_stats(keys, n, stats, &blocks, ctx->stream));
+  int32_t share[2 * kAssocStatBlocks];
+  if (blocks > 0)
+    CLUE_HIP(hipMemcpyAsync(share, stats, sizeof(int32_t) * 2 * blocks, hipMemcpyDeviceToHost,
+                            ctx->stream));
   CLUE_HIP(hipStreamSynchronize(ctx->stream));
+  int32_t hs[2] = {INT32_MIN, 0};
+  for (int k = 0; k < blocks; ++k) {
+    hs[0] = std::max(hs[0], share[2 * k]);
+    hs[1] += share[2 * k + 1];
+  }
   // bins = max + 1 (make_associator), never below 0.
   const int64_t bins = std::max<int64_t>(0, static_cast<int64_t>(hs[0]) + 1);
   if (bins >= INT32_MAX) return fail(CLUE_ERR_CAPACITY, "key too large for an offsets array");
@@ -492,7 +497,7 @@ clue_status clue_make_association(clue_ctx* ctx, const int32_t* keys, int32_t n,
   if (hs[1] > 0 && !members) return fail(CLUE_ERR_INVALID_ARGUMENT, "null members");
   AssocScratch sc{w.buf[S_K0].as<uint32_t>(), w.buf[S_V0].as<int32_t>(),
                   w.buf[S_K1].as<uint32_t>(), w.buf[S_V1].as<int32_t>(),
-                  w.buf[S_HIST].as<int32_t>(), w.buf[S_SCAN].as<int32_t>()};
+                  w.buf[S_HIST].as<int32_t>()};
   CLUE_HIP(assoc_build(keys, hs[1] > 0 ? n : 0, static_cast<int>(bins), sc, offsets, members,
                        hs[1], ctx->stream));
   CLUE_HIP(hipStreamSynchronize(ctx->stream));

@@ -15,18 +15,19 @@ void scan_exclusive(const int32_t* in, int32_t* out, int64_t n, int32_t* temp, i
                     hipStream_t s);
 // Stable radix sort of (key, value) by the low key_bits bits, in passes of
 // radix_plan(key_bits).bits. Blocks take the chunks given (contiguous ranges in order
-// that cover [0, n)), or kRsTileKeys keys each (chunks NULL). With chunks the caller
-// has counted the first pass's digits into hist ([digit][chunk]) and the values are the
-// keys' places; without, the values are v0 and the sort counts for itself. hist:
-// radix_hist_elems(n_blocks) ints. The result is in (k0, v0) or (k1, v1).
+// that cover [0, n)), or kRsTileKeys keys each (chunks NULL). The values are the keys'
+// places (0 to n - 1). The caller has counted the first pass's digits into hist
+// ([digit][block], then room for the totals: radix_hist_elems(n_blocks) ints). The
+// result is in (k0, v0) or (k1, v1); or, with last_values, the first last_count
+// values there and only the keys in k0 or k1.
 struct RadixPlan {
   int bits;    // of a digit
   int passes;
 };
 RadixPlan radix_plan(int key_bits);
 void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int64_t n, int key_bits,
-                      int32_t* hist, const Chunk* chunks, int n_chunks, bool* in_first,
-                      hipStream_t s);
+                      int32_t* hist, const Chunk* chunks, int n_chunks, int32_t* last_values,
+                      int64_t last_count, bool* in_first, hipStream_t s);
 
 // ---- stages (clue_stages_impl.h, instantiated in clue_stages_f32.hip / _f64.hip) ----
 

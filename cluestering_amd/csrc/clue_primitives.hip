@@ -203,7 +203,8 @@ __global__ __launch_bounds__(kBlock) void k_rs_rows(int32_t* __restrict__ hist, 
 template <int MaxBits>
 __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(
     const uint32_t* __restrict__ kin, const int32_t* __restrict__ vin, uint32_t* __restrict__ kout,
-    int32_t* __restrict__ vout, int64_t n, const Chunk* __restrict__ chunks, int shift, int bits,
+    int32_t* __restrict__ vout, int64_t n_out, int64_t n, const Chunk* __restrict__ chunks,
+    int shift, int bits,
     const int32_t* __restrict__ rows, const int32_t* __restrict__ total) {
   __shared__ int cnt[kRsWaves << MaxBits];  // [kRsWaves][bins]
   const int bins = 1 << bits;
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(
     __builtin_amdgcn_wave_barrier();
     if (valid) {
       kout[pos] = key[r];
-      vout[pos] = vin ? vin[i] : static_cast<int32_t>(i);
+      if (pos < n_out) vout[pos] = vin ? vin[i] : static_cast<int32_t>(i);
     }
   }
 }
@@ -274,8 +275,8 @@ RadixPlan radix_plan(int key_bits) {
 }
 
 void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int64_t n, int key_bits,
-                      int32_t* hist, const Chunk* chunks, int n_chunks, bool* in_first,
-                      hipStream_t s) {
+                      int32_t* hist, const Chunk* chunks, int n_chunks, int32_t* last_values,
+                      int64_t last_count, bool* in_first, hipStream_t s) {
   *in_first = true;
   if (n <= 0) return;
   const RadixPlan plan = radix_plan(key_bits);
@@ -287,14 +288,16 @@ void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int6
   int32_t *va = v0, *vb = v1;
   for (int pass = 0; pass < plan.passes; ++pass) {
     const int shift = pass * plan.bits;
-    if (!chunks || pass > 0)
+    const bool last = last_values && pass + 1 == plan.passes;
+    if (pass > 0)
       hipLaunchKernelGGL(k_rs_hist, dim3(nblocks), dim3(kBlock), 0, s, ka, n, chunks, shift,
                          plan.bits, hist);
     hipLaunchKernelGGL(k_rs_rows, dim3(static_cast<unsigned>(bins)), dim3(kBlock), 0, s, hist,
                        static_cast<int64_t>(nblocks), total);
     hipLaunchKernelGGL(plan.bits <= 8 ? k_rs_scatter<8> : k_rs_scatter<kRsMaxBits>, dim3(nblocks),
-                       dim3(kRsBlock), 0, s, ka, (chunks && pass == 0) ? nullptr : va, kb, vb, n,
-                       chunks, shift, plan.bits, hist, total);
+                       dim3(kRsBlock), 0, s, ka, pass == 0 ? nullptr : va, kb,
+                       last ? last_values : vb, last ? last_count : n, n, chunks, shift, plan.bits,
+                       hist, total);
     std::swap(ka, kb);
     std::swap(va, vb);
     *in_first = !*in_first;

@@ -2786,7 +2786,7 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
                      bb.events, bb.ext_group, bb.ext, bb.geo, bb.keys0, digits.bits, bb.rs_hist);
   bool in_first = true;
   radix_sort_pairs(bb.keys0, bb.vals0, bb.keys1, bb.vals1, n, bb.key_bits, bb.rs_hist, bb.chunks,
-                   bb.n_chunks, &in_first, s);
+                   bb.n_chunks, nullptr, 0, &in_first, s);
   const uint32_t* skeys = in_first ? bb.keys0 : bb.keys1;
   const int32_t* sperm = in_first ? bb.vals0 : bb.vals1;
   GatherArgs<T> ga;

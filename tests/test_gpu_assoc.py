@@ -44,6 +44,17 @@ def test_association_keys_edge_cases(gpu_ctx):
     _check(gpu_ctx, keys)
 
 
+@pytest.mark.parametrize("n", [1, 2047, 2049, 300001])
+@pytest.mark.parametrize("bins", [1, 255, 256, 1023, 1024, 1 << 20])
+def test_association_radix_widths(gpu_ctx, bins, n):
+    """Keys on both sides of the radix digits' widths, in one or two passes, with the
+    last bin empty or full and unassociated points in between."""
+    rng = np.random.default_rng(bins + n)
+    keys = rng.integers(-1, bins, n)
+    keys[n // 2] = bins - 1
+    _check(gpu_ctx, keys)
+
+
 def test_get_clusters_of_device_points(gpu_ctx):
     w = synthetic.blobs2d_16k()
     pts = PointsDevice.from_host(gpu_ctx, w.coords, w.weight)
