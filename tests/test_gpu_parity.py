@@ -462,3 +462,25 @@ def test_lone_event_among_empty_ones(gpu_ctx, oracle_mod, sizes):
                                                               event_of_cluster=eoc)
     assert k == ref.n_seeds
     np.testing.assert_array_equal(eoc.to_host()[:k], ref.event_of_cluster)
+
+
+@pytest.mark.parametrize("points_per_tile", [20000, 79, 70, 20, 19, 1])
+def test_tile_key_widths(gpu_ctx, oracle_mod, points_per_tile):
+    """1, 256, 289, 1,024, 1,089 and 20,164 tiles: keys of 0 to 15 bits, in one or two
+    radix passes of one of the two widths."""
+    rng = np.random.default_rng(points_per_tile)
+    c = rng.uniform(0, 100, (2, 20000)).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, 20000).astype(np.float32)
+    _check(Case(c, w, 1.0, 3.0, 1.5, points_per_tile=points_per_tile,
+                name=f"points_per_tile={points_per_tile}"), gpu_ctx, oracle_mod)
+
+
+def test_lone_event_above_a_million_points(gpu_ctx, oracle_mod):
+    """More than 512 chunks (each result of the extremes stage covers two) and more
+    than 32,768 words of seed bits (counted by a scan, not by one kernel)."""
+    rng = np.random.default_rng(21)
+    n = (1 << 20) + 1
+    c = rng.uniform(0, 1000, (2, n)).astype(np.float32)
+    c[:, -1] = 1003.0                     # the last point, alone in its chunk, is the maximum
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    _check(Case(c, w, 1.0, 3.0, 1.5, name="2^20+1"), gpu_ctx, oracle_mod)
