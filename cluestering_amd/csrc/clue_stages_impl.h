@@ -1020,8 +1020,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_setup(const TileSetup setup,
   if (t < n_tiles) tile_setup<D>(setup, t, n_tiles, toff[t], toff[t + 1], sx, cs, tbox);
 }
 
-// The query order of W tiles per workgroup (8 for a lone event, whose dense tiles are
-// the largest, else 4: one event of 2^20 points 81 us at 4 and 54 us at 8, the
+// The query order of per <= W tiles per workgroup of W waves (8 for a lone event, whose
+// dense tiles are the largest, else 4: one event of 2^20 points 81 us at 4 and 54 us at 8, the
 // 4096-event batch 744 us and 990 us). A tile of at most one wave's
 // points keeps its order (one wave each). The others are taken one after the other
 // by the whole workgroup, a counting sort in LDS by the Hilbert index: the dense
@@ -1033,8 +1033,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_setup(const TileSetup setup,
 template <int D, int W, bool Fine, class T>
 __global__ __launch_bounds__(W * kWave) void k_query_order(
     const RunParamsT<T> rp, const TileSetup setup, T* __restrict__ tbox, int32_t* __restrict__ ctl,
-    const T* __restrict__ geo, const int32_t* __restrict__ toff, int n_tiles, const T* __restrict__ sx, int64_t cs, int32_t* __restrict__ qfine,
-    T* __restrict__ hx, int64_t hs, int32_t* __restrict__ hidx, T* __restrict__ hbox) {
+    const T* __restrict__ geo, const int32_t* __restrict__ toff, int n_tiles, int per,
+    const T* __restrict__ sx, int64_t cs, int32_t* __restrict__ qfine, T* __restrict__ hx, int64_t hs, int32_t* __restrict__ hidx, T* __restrict__ hbox) {
   constexpr int kBins = QueryCells<D, Fine>::kBins;
   constexpr int kOrderBlock = W * kWave;
   constexpr int kHeld = 4;  // rounds whose indices stay in registers
@@ -1043,17 +1043,18 @@ __global__ __launch_bounds__(W * kWave) void k_query_order(
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   {
-    const int t = blockIdx.x * W + w;
-    const int b = t < n_tiles ? toff[t] : 0, e = t < n_tiles ? toff[t + 1] : 0;
+    const int t = blockIdx.x * per + w;
+    const bool mine = w < per && t < n_tiles;
+    const int b = mine ? toff[t] : 0, e = mine ? toff[t + 1] : 0;
     if (blockIdx.x == 0) zero_queues(ctl);
-    if (t < n_tiles) tile_setup<D>(setup, t, n_tiles, b, e, sx, cs, tbox);
-    if (t < n_tiles && e - b <= kWave) {  // one item: the query order is irrelevant
+    if (mine) tile_setup<D>(setup, t, n_tiles, b, e, sx, cs, tbox);
+    if (mine && e - b <= kWave) {  // one item: the query order is irrelevant
       if (b + lane < e) qfine[b + lane] = b + lane;
       if (hx) write_nh_layout<D>(t, b, e - b, nullptr, 0, 1, sx, cs, hx, hs, hidx, hbox);
     }
   }
-  for (int k = 0; k < W; ++k) {
-    const int t = blockIdx.x * W + k;
+  for (int k = 0; k < per; ++k) {
+    const int t = blockIdx.x * per + k;
     if (t >= n_tiles) break;
     const int b = toff[t], e = toff[t + 1];
     if (e - b <= kWave) continue;
@@ -2684,14 +2685,25 @@ CLUE_NEIGHBOUR_EXTERN(9)
 CLUE_NEIGHBOUR_EXTERN(10)
 #undef CLUE_NEIGHBOUR_EXTERN
 
+constexpr int kOrderTilesAlone = 2048;  // 8 workgroups of 8 waves per CU
+
 template <int D, class T>
 static void launch_query_order_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
   const TileSetup setup{b.events, b.n_events, b.items, b.icount, b.max_items};
+  // Tiles per workgroup, whose sorts run one after the other. Few tiles leave CUs idle,
+  // so each takes a workgroup of its own (5,003 points in 2-D: 13.4 us with eight
+  // tiles, 7.2 with two, 5.7 with one; 16,384 points 13.2 -> 6.1, 20,011 in 6-D 12.2 ->
+  // 8.4). A large lone event's dense tiles are too uneven for eight in a row (2^20
+  // points in 2-D: 72 us, 58 with two, 65 with one); batches are not (the 4096-event
+  // batch: 1.05 ms with four, 1.22 with two), nor tiles that mostly need no sort.
+  const int64_t tiles = b.n_tiles_total;
+  const bool uneven = b.n_events == 1 && b.n_total >= kWave * tiles;
   auto go = [&](auto kern, int waves) {
-    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((b.n_tiles_total + waves - 1) / waves)),
+    const int per = tiles <= kOrderTilesAlone ? 1 : uneven ? 2 : waves;
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((tiles + per - 1) / per)),
                        dim3(waves * kWave), 0, L.s, *L.rp, setup, b.tbox, b.n_items, b.geo, b.toff,
-                       b.n_tiles_total, b.sorted.x[0], L.cs, b.qfine, b.hx, b.h_stride, b.hidx,
+                       b.n_tiles_total, per, b.sorted.x[0], L.cs, b.qfine, b.hx, b.h_stride, b.hidx,
                        b.hbox);
   };
   const bool fine = !L.rp->team;
