@@ -59,16 +59,6 @@ __device__ __forceinline__ int block_excl_scan(int v, int* total) {
   return before + incl - v;
 }
 
-__device__ __forceinline__ int wave_min_i(int v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
-  return v;
-}
-__device__ __forceinline__ int wave_max_i(int v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-  return v;
-}
 __device__ __forceinline__ long long wave_min_i(long long v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -112,6 +102,8 @@ __device__ __forceinline__ int wave_min_uniform(int v) {
 __device__ __forceinline__ int wave_max_uniform(int v) {
   return wave_reduce_dpp(v, INT32_MIN, [](int a, int b) { return a > b ? a : b; });
 }
+__device__ __forceinline__ int wave_min_i(int v) { return wave_min_uniform(v); }
+__device__ __forceinline__ int wave_max_i(int v) { return wave_max_uniform(v); }
 
 // Peers: the set of active lanes whose key equals this lane's key, built from one
 // ballot per key bit. Lanes with valid == false are excluded.

@@ -24,7 +24,7 @@ using clue_dev::radix_hist_elems;
 using clue_dev::scan_temp_elems;
 
 constexpr int kChunk = clue_dev::kPointChunk;
-constexpr int kEvtSoloMaxPoints = 8192;  // largest lone event for the fused per-event stages
+constexpr int kEvtSoloMaxPoints = clue_dev::kLoneMaxPoints;
 constexpr int kDefaultPointsPerTile = 128;
 // Launches up to this many points have their neighbour stages run by teams of waves
 // (clue_team.h). Lone events on MI355X, one wave per item against a team of eight,

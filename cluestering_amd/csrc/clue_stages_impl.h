@@ -329,7 +329,7 @@ constexpr int kEvtRounds = 4;
 
 template <int D, class T>
 __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
-    const RunParamsT<T> rp, const LoneEvent lone, EventDesc* __restrict__ events,
+    const RunParamsT<T> rp, const EventDesc* __restrict__ events,
     const int32_t* __restrict__ order, const PointArraysT<T> in, const SortedArraysT<T> out,
     T* __restrict__ geo,
     int32_t* __restrict__ toff, int32_t* __restrict__ iperm, int n_tiles_total, int n_total) {
@@ -339,9 +339,8 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
   __shared__ I red[kEvtWaves][2 * D];
   __shared__ T sgeo[3 * D];
   __shared__ int32_t wsum[kEvtWaves];
-  const int e = lone.is ? 0 : order[blockIdx.x];
-  const EventDesc ev = lone.is ? lone.ev : events[e];
-  if (lone.is && threadIdx.x == 0) events[0] = ev;  // for the stages that follow
+  const int e = order[blockIdx.x];
+  const EventDesc ev = events[e];
   const int w = threadIdx.x / kWave;
   const int lane = lane_id();
   const int b0 = ev.p_off, n = ev.n;
@@ -384,7 +383,9 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
     gq[D + d] = mx;
     gq[2 * D + d] = side;
   }
-  for (int k = threadIdx.x; k < kEvtWaves * kEvtMaxTiles; k += kEvtBlock) (&cnt[0][0])[k] = 0;
+  if (static_cast<int>(threadIdx.x) < ev.ntiles)
+#pragma unroll
+    for (int k = 0; k < kEvtWaves; ++k) cnt[k][threadIdx.x] = 0;
   __syncthreads();
   GeoT<T> g;
   g.D = D;
@@ -407,7 +408,8 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
   const int wb = w * per_wave;
   const int we = min(n, wb + per_wave);
   const uint64_t lt = lanemask_lt();
-  // Per-wave tile counts.
+  // Per-wave tile counts (LDS atomics; by ballots, as the ranks below, the kernel
+  // took 1,010 us on the 4096-event batch, against 973).
   for (int k0 = wb; k0 < we; k0 += kWave * kEvtRounds) {
     uint32_t t[kEvtRounds];
     bool valid[kEvtRounds];
@@ -421,10 +423,8 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
       t[u] = valid[u] ? tile_of(x) : 0u;
     }
 #pragma unroll
-    for (int u = 0; u < kEvtRounds; ++u) {
-      const uint64_t peers = match_peers(t[u], bits, valid[u]);
-      if (valid[u] && (peers & lt) == 0) cnt[w][t[u]] += __popcll(peers);
-    }
+    for (int u = 0; u < kEvtRounds; ++u)
+      if (valid[u]) atomicAdd(&cnt[w][t[u]], 1);
   }
   __syncthreads();
   // Tile offsets: exclusive scan over tiles (one per thread), then each wave's
@@ -506,11 +506,223 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_tiles(
   }
 }
 
+// The same for a lone event of at most kLoneMaxPoints points: every thread has at most
+// kLoneRounds of them, so each pass issues all its loads together and what a pass needs
+// again stays in registers (coordinates of up to 16 bytes per point, tile ids, sorted
+// positions). One workgroup waits out every load of its chain alone: the kernel
+// above took 21.8 us for 5,003 points in 2-D and 9.0 for 300, this one 14.2 and 6.3.
+constexpr int kLoneRounds = kLoneMaxPoints / kEvtBlock;
+static_assert(kLoneMaxPoints == kLoneRounds * kEvtBlock && kLoneMaxPoints <= 1 << 15,
+              "whole rounds; 16-bit positions");
+
+template <int D, class T>
+__global__ __launch_bounds__(kEvtBlock) void k_lone_tiles(
+    const RunParamsT<T> rp, const EventDesc ev, EventDesc* __restrict__ events,
+    const PointArraysT<T> in, const SortedArraysT<T> out, T* __restrict__ geo,
+    int32_t* __restrict__ toff, int32_t* __restrict__ iperm) {
+  using I = typename FloatBits<T>::Int;
+  constexpr I kHi = std::numeric_limits<I>::max(), kLo = std::numeric_limits<I>::min();
+  constexpr int R = kLoneRounds;
+  constexpr bool kKeep = D * sizeof(T) <= 16;
+  __shared__ alignas(8) int32_t cnt[kEvtWaves][kEvtMaxTiles];
+  static_assert(sizeof(cnt) >= kLoneMaxPoints * sizeof(T), "a column fits the counters' space");
+  __shared__ I red[kEvtWaves][2 * D];
+  __shared__ T sgeo[3 * D];
+  __shared__ int32_t wsum[kEvtWaves];
+  if (threadIdx.x == 0) events[0] = ev;  // for the stages that follow
+  const int w = threadIdx.x / kWave;
+  const int lane = lane_id();
+  const int n = ev.n;
+  // Each wave owns a contiguous sixteenth of the event, R rounds of 64 (loads past the
+  // event read its last point, which the extremes see anyway).
+  const int per_wave = (n + kEvtWaves - 1) / kEvtWaves;
+  const int k0 = w * per_wave + lane;
+  const int we = min(n, (w + 1) * per_wave);
+  const int rounds = (n + kEvtBlock - 1) / kEvtBlock;
+  T x[kKeep ? D : 1][R], wt[R];
+  auto load = [&](const auto* src, auto& v) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= rounds) break;
+      v[r] = src[min(k0 + r * kWave, n - 1)];
+    }
+  };
+  auto column = [&](int d) -> T (&)[R] {
+    load(in.x[d], x[kKeep ? d : 0]);
+    return x[kKeep ? d : 0];
+  };
+  if constexpr (kKeep)
+#pragma unroll
+    for (int d = 0; d < D; ++d) column(d);
+  load(in.w, wt);
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const T(&v)[R] = kKeep ? x[kKeep ? d : 0] : column(d);
+    I lo = kHi, hi = kLo;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= rounds) break;
+      const I o = float_to_ordered(v[r]);
+      const bool ok = v[r] == v[r];  // NaN coordinates are skipped
+      lo = (ok && o < lo) ? o : lo;
+      hi = (ok && o > hi) ? o : hi;
+    }
+    lo = wave_min_i(lo);
+    hi = wave_max_i(hi);
+    if (lane == 0) {
+      red[w][2 * d] = lo;
+      red[w][2 * d + 1] = hi;
+    }
+  }
+  if (static_cast<int>(threadIdx.x) < ev.ntiles)
+#pragma unroll
+    for (int k = 0; k < kEvtWaves; ++k) cnt[k][threadIdx.x] = 0;
+  __syncthreads();
+  if (threadIdx.x < D) {
+    const int d = threadIdx.x;
+    I lo = kHi, hi = kLo;
+#pragma unroll
+    for (int k = 0; k < kEvtWaves; ++k) {
+      lo = red[k][2 * d] < lo ? red[k][2 * d] : lo;
+      hi = red[k][2 * d + 1] > hi ? red[k][2 * d + 1] : hi;
+    }
+    const T mn = lo == kHi ? std::numeric_limits<T>::max() : ordered_to_float(lo);
+    const T mx = hi == kLo ? std::numeric_limits<T>::lowest() : ordered_to_float(hi);
+    const T side = (mx - mn) / static_cast<T>(ev.nper);
+    sgeo[d] = geo[d] = mn;
+    sgeo[D + d] = geo[D + d] = mx;
+    sgeo[2 * D + d] = geo[2 * D + d] = side;
+  }
+  __syncthreads();
+  GeoT<T> g;
+  g.D = D;
+  g.nper = ev.nper;
+  g.mn = sgeo;
+  g.mx = sgeo + D;
+  g.side = sgeo + 2 * D;
+  g.wrapped = rp.wrapped;
+  uint32_t t[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) t[r] = 0u;
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    const T(&v)[R] = kKeep ? x[kKeep ? d : 0] : column(d);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= rounds) break;
+      t[r] = t[r] * g.nper + get_bin(g, v[r], d);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r >= rounds) break;
+    if (k0 + r * kWave < we) atomicAdd(&cnt[w][t[r]], 1);
+  }
+  __syncthreads();
+  {
+    const int tile = threadIdx.x;
+    int c[kEvtWaves], tot = 0;
+#pragma unroll
+    for (int k = 0; k < kEvtWaves; ++k) {
+      c[k] = tile < ev.ntiles ? cnt[k][tile] : 0;
+      tot += c[k];
+    }
+    int incl = tot;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int y = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += y;
+    }
+    if (lane == kWave - 1) wsum[w] = incl;
+    __syncthreads();
+    int run = incl - tot;
+    for (int k = 0; k < w; ++k) run += wsum[k];
+    if (tile < ev.ntiles) {
+      toff[tile] = run;
+#pragma unroll
+      for (int k = 0; k < kEvtWaves; ++k) {
+        cnt[k][tile] = run;
+        run += c[k];
+      }
+    }
+    if (tile == 0) toff[ev.ntiles] = n;
+  }
+  __syncthreads();
+  int bits = 0;
+  while ((1 << bits) < ev.ntiles) ++bits;
+  const uint64_t lt = lanemask_lt();
+  int pos[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r >= rounds) break;
+    const int k = k0 + r * kWave;
+    const bool valid = k < we;
+    const uint64_t peers = match_peers(t[r], bits, valid);
+    pos[r] = 0;
+    if (valid) pos[r] = cnt[w][t[r]] + __popcll(peers & lt);
+    __builtin_amdgcn_wave_barrier();
+    if (valid && (peers & lt) == 0) cnt[w][t[r]] += __popcll(peers);
+    if (valid) iperm[k] = pos[r];
+  }
+  // The columns go to their sorted places through LDS (the counters' space), so that
+  // global loads and stores are whole lines (gathered: 15.4 us for 5,003 points).
+  auto place = [&](const auto& v, auto&& store) {
+    auto* col = reinterpret_cast<std::remove_cv_t<std::remove_reference_t<decltype(v[0])>>*>(cnt);
+    __syncthreads();  // the counters, or the column before, are done with
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= rounds) break;
+      if (k0 + r * kWave < we) col[pos[r]] = v[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int s = static_cast<int>(threadIdx.x) + r * kEvtBlock;
+      if (s >= n) break;
+      store(s, col[s]);
+    }
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    place(kKeep ? x[kKeep ? d : 0] : column(d), [&](int s, T v) { out.x[d][s] = v; });
+  place(wt, [&](int s, T v) {
+    out.w[s] = v;
+    if (out.fw) out.fw[s] = rp.kp0 * v;  // flat kernel: K * w for j != i
+  });
+  if (rp.has_sigma)
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      load(in.sigma[d], wt);
+      place(wt, [&](int s, T v) { out.sigma[d][s] = v; });
+    }
+  if (rp.has_u) {
+    load(in.u, wt);
+    place(wt, [&](int s, T v) { out.u[s] = v; });
+  }
+  int index[R];
+  if (rp.has_tags) {
+    uint32_t tags[R];
+    load(in.tags, tags);
+    place(tags, [&](int s, uint32_t v) { out.tag[s] = v; });
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) index[r] = k0 + r * kWave;
+  place(index, [&](int s, int v) {
+    out.perm[s] = v;
+    if (!rp.has_tags) out.tag[s] = static_cast<uint32_t>(v);
+  });
+}
+
 template <int D, class T>
 static void launch_event_tiles_d(const RunParamsT<T>& rp, const PointArraysT<T>& in,
                                  const BatchBuffersT<T>& bb, hipStream_t s) {
+  if (bb.lone.is) {
+    hipLaunchKernelGGL((k_lone_tiles<D, T>), dim3(1), dim3(kEvtBlock), 0, s, rp, bb.lone.ev,
+                       bb.events, in, bb.sorted, bb.geo, bb.toff, bb.iperm);
+    return;
+  }
   hipLaunchKernelGGL((k_event_tiles<D, T>), dim3(static_cast<unsigned>(bb.n_events)),
-                     dim3(kEvtBlock), 0, s, rp, bb.lone, bb.events, bb.event_order, in, bb.sorted, bb.geo,
+                     dim3(kEvtBlock), 0, s, rp, bb.events, bb.event_order, in, bb.sorted, bb.geo,
                      bb.toff, bb.iperm, bb.n_tiles_total, bb.n_total);
 }
 
@@ -2265,15 +2477,14 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
     const T* __restrict__ srho, int32_t* __restrict__ snh, const T* __restrict__ sdelta,
     const T* __restrict__ su, T* __restrict__ rho, int32_t* __restrict__ nh, T* __restrict__ delta,
     int32_t* __restrict__ is_seed, int32_t* __restrict__ rank, int32_t* __restrict__ event_seeds,
-    const LoneEvent lone, int32_t* __restrict__ lone_total, int32_t* __restrict__ lone_seeds,
-    int32_t* __restrict__ event_of_cluster, int32_t* __restrict__ cluster) {
+    int32_t* __restrict__ cluster) {
   constexpr int kWordsPerThread = kEvtBitWords / kEvtBlock;
   __shared__ uint32_t pool[kSeedPoolWords];
   __shared__ int32_t wsum[kEvtWaves];
   uint32_t* bits = pool;
   int16_t* links = reinterpret_cast<int16_t*>(pool + kLdsBitWords);
-  const int e = lone.is ? 0 : order[blockIdx.x];
-  const EventDesc ev = lone.is ? lone.ev : events[e];
+  const int e = order[blockIdx.x];
+  const EventDesc ev = events[e];
   const int b0 = ev.p_off, n = ev.n;
   const bool in_lds = n <= kEvtLdsLinks;
   const int n_words = in_lds ? kLdsBitWords : kEvtBitWords;  // bit words in use
@@ -2345,13 +2556,7 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
       if (in_lds) {
         // The event's seed list in rank order, and the seed's link: its rank as
         // a code (-3 - rank) that the jumping passes carry to its followers.
-        // A lone event's ranks are final.
-        if (lone.is) {
-          lone_seeds[run] = ii;
-          if (event_of_cluster) event_of_cluster[run] = ev.index;
-        } else {
-          rank[b0 + run] = b0 + ii;
-        }
+        rank[b0 + run] = b0 + ii;
         links[iperm[b0 + ii] - b0] = static_cast<int16_t>(-3 - run);
         ++run;
       } else {
@@ -2359,10 +2564,7 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
       }
     }
   }
-  if (threadIdx.x == 0) {
-    event_seeds[e] = total;
-    if (lone.is) *lone_total = total;
-  }
+  if (threadIdx.x == 0) event_seeds[e] = total;
   // Pointer jumping on the event's links: a pass replaces a link by its target's link
   // when that target is itself a follower, which halves every chain (at least); any
   // interleaving of the updates leaves every link on its own chain.
@@ -2400,6 +2602,123 @@ __global__ __launch_bounds__(kEvtBlock) void k_event_seeds(
         if (l2 >= 0) snh[s] = l2;
       }
     }
+  }
+}
+
+// The same for a lone event of at most kLoneMaxPoints points, whose labels, seeds and
+// total are final: no label stage follows. Everything that is read in another order
+// than it was loaded goes through LDS (the kernel above: 16.6 us for 5,003 points, 5.3
+// for 300; this one: 9.0 and 4.1).
+template <class T>
+__global__ __launch_bounds__(kEvtBlock) void k_lone_seeds(
+    const RunParamsT<T> rp, const EventDesc ev, const int32_t* __restrict__ perm,
+    const int32_t* __restrict__ iperm, const T* __restrict__ srho, const int32_t* __restrict__ snh,
+    const T* __restrict__ sdelta, const T* __restrict__ su, T* __restrict__ rho,
+    int32_t* __restrict__ nh, T* __restrict__ delta, int32_t* __restrict__ is_seed,
+    int32_t* __restrict__ total, int32_t* __restrict__ seeds,
+    int32_t* __restrict__ event_of_cluster, int32_t* __restrict__ cluster) {
+  constexpr int R = kLoneRounds;
+  constexpr int kWords = kLoneMaxPoints / 32;
+  static_assert(kWords <= kEvtBlock, "one word per thread");
+  __shared__ uint32_t bits[kWords];            // a bit per seed, in input order
+  __shared__ int16_t links[kLoneMaxPoints];    // k_event_seeds' links and codes
+  __shared__ uint16_t input[kLoneMaxPoints];   // sorted position -> input index
+  __shared__ uint16_t sorted[kLoneMaxPoints];  // input index -> sorted position
+  __shared__ T lrho[kLoneMaxPoints];
+  __shared__ int32_t wsum[kEvtWaves];
+  const int n = ev.n;
+  const int w = threadIdx.x / kWave;
+  const int lane = lane_id();
+  const int rounds = (n + kEvtBlock - 1) / kEvtBlock;
+  if (threadIdx.x < kWords) bits[threadIdx.x] = 0u;
+  int h[R], p[R], q[R];
+  T ro[R], u[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (r >= rounds) break;
+    const int k = min(static_cast<int>(threadIdx.x) + r * kEvtBlock, n - 1);
+    h[r] = snh[k];
+    p[r] = perm[k];
+    q[r] = iperm[k];
+    ro[r] = srho[k];
+    u[r] = rp.has_u ? su[k] : T(1);
+  }
+  __syncthreads();
+  // Seed flags (ClusteringKernels.hpp:300-316), in sorted order.
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = static_cast<int>(threadIdx.x) + r * kEvtBlock;
+    if (k >= n) break;
+    const bool seed = (h[r] == -1) && (ro[r] >= rp.rhoc * u[r]);
+    links[k] = static_cast<int16_t>(seed ? -2 : h[r]);
+    lrho[k] = ro[r];
+    input[k] = static_cast<uint16_t>(p[r]);
+    sorted[k] = static_cast<uint16_t>(q[r]);
+    if (seed) atomicOr(&bits[p[r] >> 5], 1u << (p[r] & 31));
+  }
+  __syncthreads();
+  // Results in input order.
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = static_cast<int>(threadIdx.x) + r * kEvtBlock;
+    if (k >= n) break;
+    const int l = links[q[r]];
+    rho[k] = lrho[q[r]];
+    nh[k] = l >= 0 ? input[l] : -1;
+    is_seed[k] = l == -2 ? 1 : 0;
+  }
+  if (delta) {
+    T v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= rounds) break;
+      v[r] = sdelta[q[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int k = static_cast<int>(threadIdx.x) + r * kEvtBlock;
+      if (k >= n) break;
+      delta[k] = v[r];
+    }
+  }
+  // Ranks of the seeds in input order.
+  uint32_t word = threadIdx.x < kWords ? bits[threadIdx.x] : 0u;
+  const int mine = __popc(word);
+  int incl = mine;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int y = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += y;
+  }
+  if (lane == kWave - 1) wsum[w] = incl;
+  __syncthreads();  // and the results have read the links
+  int run = incl - mine;
+  for (int k = 0; k < w; ++k) run += wsum[k];
+  if (threadIdx.x == kEvtBlock - 1) *total = run;  // no words: all seeds are before it
+  while (word) {
+    const int ii = static_cast<int>(threadIdx.x) * 32 + __builtin_ctz(word);
+    word &= word - 1u;
+    seeds[run] = ii;
+    if (event_of_cluster) event_of_cluster[run] = ev.index;
+    links[sorted[ii]] = static_cast<int16_t>(-3 - run);
+    ++run;
+  }
+  // Pointer jumping, as in k_event_seeds, then the label of what each link names.
+  for (int pass = 0; pass < kLdsJumpPasses; ++pass) {
+    __syncthreads();
+    for (int k = threadIdx.x; k < n; k += kEvtBlock) {
+      const int l = links[k];
+      if (l >= 0) links[k] = links[l];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int k = static_cast<int>(threadIdx.x) + r * kEvtBlock;
+    if (k >= n) break;
+    int l = links[q[r]];
+    while (l >= 0) l = links[l];
+    cluster[k] = l <= -3 ? -3 - l : -1;
   }
 }
 
@@ -2843,20 +3162,22 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
 
   // (d), (e)
   mark(kStageSeeds);
-  if (bb.event_order) {
+  if (bb.event_order && bb.lone.is) {
+    hipLaunchKernelGGL(k_lone_seeds<T>, dim3(1), dim3(kEvtBlock), 0, s, rp, bb.lone.ev,
+                       bb.sorted.perm, bb.iperm, bb.srho, bb.snh, bb.sdelta, bb.sorted.u, out.rho,
+                       out.nh, out.delta, out.is_seed, bb.n_seeds, bb.seeds, out.event_of_cluster,
+                       out.cluster);
+    mark(kStageLabels);
+  } else if (bb.event_order) {
     hipLaunchKernelGGL(k_event_seeds<T>, dim3(static_cast<unsigned>(bb.n_events)), dim3(kEvtBlock),
                        0, s, rp, bb.events, bb.event_order, bb.sorted.perm, bb.iperm, bb.srho, bb.snh,
                        bb.sdelta, bb.sorted.u, out.rho, out.nh, out.delta, out.is_seed, bb.rank,
-                       bb.event_seeds, bb.lone, bb.n_seeds, bb.seeds, out.event_of_cluster,
-                       out.cluster);
+                       bb.event_seeds, out.cluster);
     mark(kStageLabels);
-    // A lone event (small enough for the LDS links, plan_batch) is done.
-    if (!bb.lone.is) {
-      scan_exclusive(bb.event_seeds, bb.event_offsets, bb.n_events, bb.scan_tmp, bb.n_seeds, s);
-      hipLaunchKernelGGL(k_event_labels, dim3(bb.n_chunks), dim3(kBlock), 0, s, bb.chunks, bb.events,
-                         bb.sorted.perm, bb.snh, bb.rank, bb.event_offsets, bb.event_seeds,
-                         out.cluster, bb.seeds, out.event_of_cluster, out.local_ids);
-    }
+    scan_exclusive(bb.event_seeds, bb.event_offsets, bb.n_events, bb.scan_tmp, bb.n_seeds, s);
+    hipLaunchKernelGGL(k_event_labels, dim3(bb.n_chunks), dim3(kBlock), 0, s, bb.chunks, bb.events,
+                       bb.sorted.perm, bb.snh, bb.rank, bb.event_offsets, bb.event_seeds,
+                       out.cluster, bb.seeds, out.event_of_cluster, out.local_ids);
   } else {
     const int words = (n + 31) / 32;
     uint32_t* bits = reinterpret_cast<uint32_t*>(bb.flag);

@@ -20,6 +20,8 @@ constexpr int kMetricPeriodicLast = 7;
 constexpr int kEvtMaxTiles = 1024;
 // Largest event the fused per-event stages take (one bit per point in LDS).
 constexpr int kEvtMaxPoints = 1 << 17;
+// Largest lone event of the fused stages.
+constexpr int kLoneMaxPoints = 8192;
 
 constexpr int kPointChunk = 2048;  // points per chunk of the per-point grids
 

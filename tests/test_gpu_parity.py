@@ -484,3 +484,23 @@ def test_lone_event_above_a_million_points(gpu_ctx, oracle_mod):
     c[:, -1] = 1003.0                     # the last point, alone in its chunk, is the maximum
     w = rng.uniform(0.5, 1.5, n).astype(np.float32)
     _check(Case(c, w, 1.0, 3.0, 1.5, name="2^20+1"), gpu_ctx, oracle_mod)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("ndim", [1, 3, 5])
+@pytest.mark.parametrize("n,points_per_tile", [(1, 0), (1023, 0), (1025, 0), (8191, 8), (8192, 0),
+                                               (8192, 7)])
+def test_small_lone_events(gpu_ctx, oracle_mod, n, points_per_tile, ndim, dtype):
+    """A lone event's own tile and seed kernels (up to 8,192 points and 1,024 tiles):
+    whole and partial rounds, with every optional column and without."""
+    rng = np.random.default_rng(n + ndim)
+    c = rng.uniform(0, 20, (ndim, n)).astype(dtype)
+    w = rng.uniform(0.5, 1.5, n).astype(dtype)
+    u = rng.uniform(0.5, 1.5, n).astype(dtype)
+    sigma = rng.uniform(0.0, 0.3, size=(ndim, n)).astype(dtype)
+    tags = rng.permutation(n).astype(np.uint32)
+    for more in ({}, {"u": u, "sigma": sigma, "tags": tags}):
+        case = Case(c, w, 1.0, 2.0, 1.5, points_per_tile=points_per_tile, dtype=dtype,
+                    name=f"lone n={n} ndim={ndim} {np.dtype(dtype)} {sorted(more)}", **more)
+        print(f"[case] {case.name}", flush=True)
+        assert_same(case.run_gpu(gpu_ctx), case.run_oracle(oracle_mod), case.name)
