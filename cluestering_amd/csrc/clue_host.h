@@ -213,6 +213,16 @@ struct WorkspaceShape {
 };
 
 // Bytes of every workspace slot for a batch of this shape (0: unused).
+// Bytes of the tiles' bounding boxes, 0 where the stages do without. Small tables are
+// always worth it; of the large ones those that hold fewer than 16 points per tile are
+// left out: in many dimensions, or with very small tiles, they would take more memory
+// than the columns of the points.
+constexpr int64_t kTileBoxAlways = 4 << 20;
+inline size_t tile_box_bytes(int64_t n, int64_t tiles, int D, int value_bytes) {
+  const int64_t bytes = tiles * 2 * D * value_bytes;
+  return bytes <= kTileBoxAlways || 16 * tiles <= n ? static_cast<size_t>(bytes) : 0;
+}
+
 inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) {
   std::memset(bytes, 0, sizeof(bytes));
   const int64_t n = w.n, NT = w.tiles;
@@ -247,7 +257,7 @@ inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) 
   bytes[S_HIDX] = sizeof(int32_t) * h_slots;
   bytes[S_HBOX] = T * h_blocks * 2 * D;
   bytes[S_HBKEY] = sizeof(uint64_t) * h_blocks;
-  bytes[S_SBOX] = w.sorted_boxes ? T * NT * 2 * D : 0;  // one box per tile
+  bytes[S_SBOX] = w.sorted_boxes ? tile_box_bytes(n, NT, w.D, w.value_bytes) : 0;
   bytes[S_SRHO] = T * n;
   bytes[S_SKEY] = w.nh_blocks ? 0 : sizeof(uint64_t) * n;  // the block scan's keys: S_HKEY
   bytes[S_SFW] = w.flat_kernel ? T * n : 0;

@@ -319,7 +319,9 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   b.hbox = nhb ? at<T>(slot, S_HBOX) : nullptr;
   b.hbkey = nhb ? at<uint64_t>(slot, S_HBKEY) : nullptr;
   b.h_stride = h_slots;
-  b.tbox = sorted_boxes_enabled(p) ? at<T>(slot, S_SBOX) : nullptr;
+  b.tbox = sorted_boxes_enabled(p) && tile_box_bytes(n, NT, D, sizeof(T)) > 0
+               ? at<T>(slot, S_SBOX)
+               : nullptr;
   for (int d = 0; d < kMaxDim; ++d) {
     b.sorted.x[d] = d < D ? at<T>(slot, S_SX) + stride * d : nullptr;
     b.sorted.sigma[d] = (has_sigma && d < D) ? at<T>(slot, S_SSIG) + stride * d : nullptr;

@@ -504,3 +504,14 @@ def test_small_lone_events(gpu_ctx, oracle_mod, n, points_per_tile, ndim, dtype)
                     name=f"lone n={n} ndim={ndim} {np.dtype(dtype)} {sorted(more)}", **more)
         print(f"[case] {case.name}", flush=True)
         assert_same(case.run_gpu(gpu_ctx), case.run_oracle(oracle_mod), case.name)
+
+
+@pytest.mark.parametrize("ndim,n", [(5, 100000), (3, 200000)])
+def test_many_nearly_empty_tiles(gpu_ctx, oracle_mod, ndim, n):
+    """Tiles of less than a point on average, whose boxes would exceed their 4 MiB: the
+    stages do without (161,051 tiles for teams of waves, 205,379 for one wave per item)."""
+    rng = np.random.default_rng(ndim)
+    c = rng.uniform(0, 10, (ndim, n)).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    _check(Case(c, w, 0.2, 1.5, 0.3, points_per_tile=1, name=f"ndim={ndim} n={n}"), gpu_ctx,
+           oracle_mod)
