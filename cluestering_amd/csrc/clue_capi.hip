@@ -89,6 +89,7 @@ struct clue_ctx {
   hipEvent_t ev[kNumStages + 1] = {};
   bool ev_ready = false;
   bool ev_recorded[kNumStages + 1] = {};
+  PinnedStage stage;  // small copies between the host and ws
   Workspace aux;  // association maps (its own buffers: a pending run keeps ws)
   bool tuned = false;  // clue_set_tuning fixed `tuning`
   clue_tuning tuning{};
@@ -123,18 +124,28 @@ clue_status read_stage_times(hipEvent_t* ev, const bool* recorded, const char** 
   return CLUE_OK;
 }
 
+// Waits for a run that may still read the context's host descriptors and stage.
+clue_status settle(clue_ctx* ctx) {
+  if (ctx->pending) {
+    CLUE_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->pending = false;
+  }
+  ctx->stage.reset();
+  return CLUE_OK;
+}
+
 template <class P, class Pts, class Res>
 clue_status run_batch(clue_ctx* ctx, const P* p, const Pts* pts, const uint32_t* sizes,
-                      int32_t n_events, Res* res, int32_t* event_of_cluster) {
+                      int32_t n_events, Res* res, int32_t* event_of_cluster, bool settled = false) {
   using T = value_t<P>;
   clue_status st = validate(p);
   if (st) return st;
   if (!res || !res->cluster_index) return fail(CLUE_ERR_INVALID_ARGUMENT, "cluster_index is required");
   if (!sizes || n_events < 1) return fail(CLUE_ERR_INVALID_ARGUMENT, "no events");
   ScopedDevice dev(ctx->device);
-  if (ctx->pending) {
-    CLUE_HIP(hipStreamSynchronize(ctx->stream));
-    ctx->pending = false;
+  if (!settled) {
+    st = settle(ctx);
+    if (st) return st;
   }
   BatchPlan& bp = ctx->plan;
   st = make_batch_plan(p, sizes, n_events, &bp, ctx->tuned ? &ctx->tuning : nullptr);
@@ -143,7 +154,7 @@ clue_status run_batch(clue_ctx* ctx, const P* p, const Pts* pts, const uint32_t*
   if (st) return st;
   BatchBuffersT<T> bb;
   ResultArraysT<T> ra;
-  st = prepare_batch(ctx->ws, bp, p, pts, res, ctx->stream, &bb, &ra);
+  st = prepare_batch(ctx->ws, bp, p, pts, res, &ctx->stage, ctx->stream, &bb, &ra);
   if (st) return st;
   ra.event_of_cluster = event_of_cluster;
   const RunParamsT<T> rp = make_run_params(p, pts, bp);
@@ -212,6 +223,7 @@ clue_status clue_context_create(int32_t device, void* stream, clue_ctx** out) {
   // (its failure is reported by that entry point only), and host descriptors with
   // room for any event the scratch can hold, so that planning it allocates nothing.
   (void)init_scratch(device);
+  c->stage.create();
   c->plan.events.reserve(1);
   c->plan.event_order.reserve(1);
   c->plan.chunks.reserve(kNoAllocScratchBytes / kChunk / 64 + 1);
@@ -320,7 +332,7 @@ clue_status clue_make_clusters_noalloc(clue_ctx* ctx, const clue_params* params,
                                        std::to_string(kNoAllocScratchBytes));
   BatchBuffers bb;
   ResultArrays ra;
-  st = bind_batch(slot, bp, params, points, results, ctx->stream, &bb, &ra);
+  st = bind_batch(slot, bp, params, points, results, nullptr, ctx->stream, &bb, &ra);
   if (st) return st;
   const RunParams rp = make_run_params(params, points, bp);
   for (bool& r : ctx->ev_recorded) r = false;
@@ -356,7 +368,10 @@ clue_status run_host(clue_ctx* ctx, const P* params, int32_t n, const value_t<P>
   CLUE_HIP(ws.buf[S_HIN].reserve(col * (D + 1)));
   CLUE_HIP(ws.buf[S_HCL].reserve(sizeof(int32_t) * static_cast<size_t>(n)));
   T* din = ws.buf[S_HIN].as<T>();
-  CLUE_HIP(hipMemcpyAsync(din, host_data, col * (D + 1), hipMemcpyHostToDevice, ctx->stream));
+  st = settle(ctx);
+  if (st) return st;
+  ctx->pending = true;  // also if this call ends early
+  CLUE_HIP(ctx->stage.upload(din, host_data, col * (D + 1), ctx->stream));
   Pts pts{};
   pts.n = n;
   for (int d = 0; d < D; ++d) pts.coords[d] = din + static_cast<size_t>(n) * d;
@@ -368,20 +383,29 @@ clue_status run_host(clue_ctx* ctx, const P* params, int32_t n, const value_t<P>
     sizes = &one;
     n_events = 1;
   }
-  st = run_batch(ctx, params, &pts, sizes, n_events, &res, nullptr);
+  st = run_batch(ctx, params, &pts, sizes, n_events, &res, nullptr, true);
   if (st) return st;
-  CLUE_HIP(hipMemcpyAsync(host_cluster_index, res.cluster_index, sizeof(int32_t) * n,
-                          hipMemcpyDeviceToHost, ctx->stream));
-  if (host_is_seed)
-    CLUE_HIP(hipMemcpyAsync(host_is_seed, ws.buf[S_ISSEED].p, sizeof(int32_t) * n,
-                            hipMemcpyDeviceToHost, ctx->stream));
-  if (host_rho)
-    CLUE_HIP(hipMemcpyAsync(host_rho, ws.buf[S_RHO].p, sizeof(T) * n, hipMemcpyDeviceToHost,
+  struct Output {
+    void* host;
+    const void* device;
+    size_t bytes;
+    char* staged;
+  } outputs[] = {
+      {host_cluster_index, res.cluster_index, sizeof(int32_t) * n, nullptr},
+      {host_is_seed, ws.buf[S_ISSEED].p, sizeof(int32_t) * n, nullptr},
+      {host_rho, ws.buf[S_RHO].p, sizeof(T) * n, nullptr},
+      {host_nearest_higher, ws.buf[S_NH].p, sizeof(int32_t) * n, nullptr},
+  };
+  for (Output& o : outputs) {
+    if (!o.host) continue;
+    o.staged = ctx->stage.take(o.bytes);
+    CLUE_HIP(hipMemcpyAsync(o.staged ? o.staged : o.host, o.device, o.bytes, hipMemcpyDeviceToHost,
                             ctx->stream));
-  if (host_nearest_higher)
-    CLUE_HIP(hipMemcpyAsync(host_nearest_higher, ws.buf[S_NH].p, sizeof(int32_t) * n,
-                            hipMemcpyDeviceToHost, ctx->stream));
+  }
   CLUE_HIP(hipStreamSynchronize(ctx->stream));
+  ctx->pending = false;
+  for (const Output& o : outputs)
+    if (o.staged) std::memcpy(o.host, o.staged, o.bytes);
   return CLUE_OK;
 }
 
@@ -439,9 +463,11 @@ clue_status clue_get_n_clusters(clue_ctx* ctx, int64_t* n_clusters) {
   if (!ctx->has_run)
     return fail(CLUE_ERR_RUNTIME, "Seeds are not available. Please run make_clusters first.");
   int32_t k = 0;
-  CLUE_HIP(hipMemcpyAsync(&k, ctx->last_nseeds, sizeof(int32_t), hipMemcpyDeviceToHost,
+  void* to = ctx->stage.scratch() ? static_cast<void*>(ctx->stage.scratch()) : &k;
+  CLUE_HIP(hipMemcpyAsync(to, ctx->last_nseeds, sizeof(int32_t), hipMemcpyDeviceToHost,
                           ctx->stream));
   CLUE_HIP(hipStreamSynchronize(ctx->stream));
+  std::memmove(&k, to, sizeof(int32_t));
   *n_clusters = k;
   return CLUE_OK;
 }
@@ -477,7 +503,10 @@ clue_status clue_make_association(clue_ctx* ctx, const int32_t* keys, int32_t n,
   int32_t* stats = w.buf[S_NSEEDS].as<int32_t>();
   int blocks = 0;
   CLUE_HIP(assoc_stats(keys, n, stats, &blocks, ctx->stream));
-  int32_t share[2 * kAssocStatBlocks];
+  int32_t direct[2 * kAssocStatBlocks];
+  static_assert(sizeof(direct) <= PinnedStage::kScratch, "the statistics fit");
+  int32_t* share =
+      ctx->stage.scratch() ? reinterpret_cast<int32_t*>(ctx->stage.scratch()) : direct;
   if (blocks > 0)
     CLUE_HIP(hipMemcpyAsync(share, stats, sizeof(int32_t) * 2 * blocks, hipMemcpyDeviceToHost,
                             ctx->stream));
@@ -593,7 +622,7 @@ clue_status clue_plan_create(clue_ctx* ctx, const clue_params* params, const clu
   plan->ctx = ctx;
   BatchBuffers bb;
   ResultArrays ra;
-  st = prepare_batch(plan->ws, bp, params, points, results, ctx->stream, &bb, &ra);
+  st = prepare_batch(plan->ws, bp, params, points, results, nullptr, ctx->stream, &bb, &ra);
   if (st) return st;
   CLUE_HIP(hipStreamSynchronize(ctx->stream));  // descriptors uploaded before capture
   ra.event_of_cluster = event_of_cluster;

@@ -250,7 +250,7 @@ WorkspaceShape workspace_shape(const BatchPlan& bp, const P* p, const Pts* pts, 
 // descriptor uploads on the stream (they precede any kernel that reads them).
 template <class P, class Pts, class Res>
 clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P* p, const Pts* pts,
-                       Res* res, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
+                       Res* res, PinnedStage* stage, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
                        ResultArraysT<value_t<P>>* ra) {
   using T = value_t<P>;
   using I = typename FloatBits<T>::Int;
@@ -266,13 +266,14 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   const int64_t h_slots = h_blocks * kNhBlock;
   const bool lone = E == 1 && bp.events[0].p_off == 0;
   if (!lone) {
-    CLUE_HIP(hipMemcpyAsync(slot[S_EVENTS], bp.events.data(), sizeof(EventDesc) * E,
-                            hipMemcpyHostToDevice, s));
-    CLUE_HIP(hipMemcpyAsync(slot[S_CHUNKS], bp.chunks.data(), sizeof(Chunk) * C,
-                            hipMemcpyHostToDevice, s));
+    auto upload = [&](int k, const void* src, size_t bytes) {
+      return stage ? stage->upload(slot[k], src, bytes, s)
+                   : hipMemcpyAsync(slot[k], src, bytes, hipMemcpyHostToDevice, s);
+    };
+    CLUE_HIP(upload(S_EVENTS, bp.events.data(), sizeof(EventDesc) * E));
+    CLUE_HIP(upload(S_CHUNKS, bp.chunks.data(), sizeof(Chunk) * C));
     if (!bp.event_order.empty())
-      CLUE_HIP(hipMemcpyAsync(slot[S_EORDER], bp.event_order.data(), sizeof(int32_t) * E,
-                              hipMemcpyHostToDevice, s));
+      CLUE_HIP(upload(S_EORDER, bp.event_order.data(), sizeof(int32_t) * E));
   }
   auto& b = *bb;
   b = BatchBuffersT<T>{};
@@ -345,14 +346,14 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
 // Reserves the workspace of one batch in grow-only buffers, then binds it.
 template <class P, class Pts, class Res>
 clue_status prepare_batch(Workspace& ws, const BatchPlan& bp, const P* p, const Pts* pts,
-                          Res* res, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
+                          Res* res, PinnedStage* stage, hipStream_t s, BatchBuffersT<value_t<P>>* bb,
                           ResultArraysT<value_t<P>>* ra) {
   size_t need[S_NUM];
   workspace_requests(workspace_shape(bp, p, pts, res), need);
   for (int k = 0; k < S_NUM; ++k) CLUE_HIP(ws.buf[k].reserve(need[k]));
   void* slot[S_NUM];
   for (int k = 0; k < S_NUM; ++k) slot[k] = ws.buf[k].p;
-  return bind_batch(slot, bp, p, pts, res, s, bb, ra);
+  return bind_batch(slot, bp, p, pts, res, stage, s, bb, ra);
 }
 
 template <class P, class Pts>
@@ -390,16 +391,16 @@ template WorkspaceShape workspace_shape(const BatchPlan&, const clue_params*, co
 template WorkspaceShape workspace_shape(const BatchPlan&, const clue_params_f64*,
                                        const clue_points_f64*, const clue_results_f64*);
 template clue_status bind_batch(void* const (&)[S_NUM], const BatchPlan&, const clue_params*,
-                                const clue_points*, clue_results*, hipStream_t,
+                                const clue_points*, clue_results*, PinnedStage*, hipStream_t,
                                 BatchBuffersT<float>*, ResultArraysT<float>*);
 template clue_status bind_batch(void* const (&)[S_NUM], const BatchPlan&, const clue_params_f64*,
-                                const clue_points_f64*, clue_results_f64*, hipStream_t,
+                                const clue_points_f64*, clue_results_f64*, PinnedStage*, hipStream_t,
                                 BatchBuffersT<double>*, ResultArraysT<double>*);
 template clue_status prepare_batch(Workspace&, const BatchPlan&, const clue_params*,
-                                   const clue_points*, clue_results*, hipStream_t,
+                                   const clue_points*, clue_results*, PinnedStage*, hipStream_t,
                                    BatchBuffersT<float>*, ResultArraysT<float>*);
 template clue_status prepare_batch(Workspace&, const BatchPlan&, const clue_params_f64*,
-                                   const clue_points_f64*, clue_results_f64*, hipStream_t,
+                                   const clue_points_f64*, clue_results_f64*, PinnedStage*, hipStream_t,
                                    BatchBuffersT<double>*, ResultArraysT<double>*);
 
 }  // namespace clue_rt

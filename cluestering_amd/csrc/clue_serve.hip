@@ -105,6 +105,7 @@ class HipLanes : public clue_srv::ServeBackend {
     hipEvent_t done = nullptr;
     Workspace ws;
     BatchPlan plan;
+    PinnedStage stage;  // the batch's descriptors
     DevBuf staging, cols, labels, reqdesc;
     int32_t* labels_host = nullptr;   // pinned, lane point cap
     ReqDesc* reqdesc_host = nullptr;  // pinned
@@ -155,6 +156,7 @@ class HipLanes : public clue_srv::ServeBackend {
     }
     CLUE_HIP(hipHostMalloc(reinterpret_cast<void**>(&L->labels_host),
                            sizeof(int32_t) * static_cast<size_t>(lane_points), hipHostMallocDefault));
+    L->stage.create();
     lanes_.push_back(std::move(L));
     return CLUE_OK;
   }
@@ -285,7 +287,8 @@ class HipLanes : public clue_srv::ServeBackend {
     res.cluster_index = L.labels.as<int32_t>();
     BatchBuffers bb;
     ResultArrays ra;
-    st = prepare_batch(L.ws, L.plan, &p, &pts, &res, L.stream, &bb, &ra);
+    L.stage.reset();  // the lane is idle
+    st = prepare_batch(L.ws, L.plan, &p, &pts, &res, &L.stage, L.stream, &bb, &ra);
     if (st) return st;
     ra.local_ids = 1;
     hipLaunchKernelGGL(k_repack, dim3(bb.n_chunks), dim3(256), 0, L.stream,

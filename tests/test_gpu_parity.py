@@ -515,3 +515,32 @@ def test_many_nearly_empty_tiles(gpu_ctx, oracle_mod, ndim, n):
     w = rng.uniform(0.5, 1.5, n).astype(np.float32)
     _check(Case(c, w, 0.2, 1.5, 0.3, points_per_tile=1, name=f"ndim={ndim} n={n}"), gpu_ctx,
            oracle_mod)
+
+
+@pytest.mark.parametrize("n", [1, 21845, 21846, 65536, 65537])
+def test_host_arrays_of_staged_sizes(gpu_ctx, n):
+    """Host calls on both sides of the largest copy that goes through pinned memory
+    (262,140 and 262,152 bytes of points; 256 KiB and more per result, which together
+    exceed the block), one after the other, against the device-resident call."""
+    import ctypes as C
+
+    from cluestering_amd import _capi
+    from cluestering_amd.device import Clusterer, PointsDevice
+    rng = np.random.default_rng(n)
+    lib = _capi.load()
+    kern = K.GaussianKernel(1.0, 1.0)
+    for _ in range(2):
+        c, w = (np.ascontiguousarray(a) for a in synthetic._event2d(rng, n))
+        data = np.ascontiguousarray(np.vstack([c, w[None, :]]), dtype=np.float32)
+        p = _capi.make_params(2, 1.5, 5.0, 2.0, None, kern.kind, kern.params)
+        out = [np.empty(n, t) for t in (np.int32, np.int32, np.float32, np.int32)]
+        at = [a.ctypes.data_as(C.c_void_p) for a in out]
+        _capi.check(lib.clue_make_clusters_host(gpu_ctx.handle, C.byref(p), n,
+                                                data.ctypes.data_as(C.c_void_p), at[0], None, 0,
+                                                at[1], at[2], at[3]))
+        pts = PointsDevice.from_host(gpu_ctx, c, w)
+        Clusterer(gpu_ctx, 1.5, 5.0, 2.0).make_clusters(pts, kernel=kern)
+        np.testing.assert_array_equal(out[0], pts.cluster_index.to_host())
+        np.testing.assert_array_equal(out[1], pts.is_seed.to_host())
+        np.testing.assert_array_equal(out[2].view(np.uint32), pts.rho.to_host().view(np.uint32))
+        np.testing.assert_array_equal(out[3], pts.nearest_higher.to_host())
