@@ -194,9 +194,17 @@ __device__ __forceinline__ GeoT<T> event_geo(const T* geo, const RunParamsT<T>& 
 // the chunks' results, side = (max - min) / nper (ComputeTiles.hpp:33-34); the
 // event's first chunk stores the geometry, geo[e] = {mn[D], mx[D], side[D]}. The keys'
 // lowest digits are counted as they are made: the histogram of the first sort pass.
+// A thread has two points of the chunk, whose loads it issues together; with 256
+// threads of eight points, one after the other, the chain of loads set the time
+// (16,384 points in 2-D: 8.8 -> 6.2 us; 20,011 in 6-D: 17.6 -> 8.3; 2^20 in 2-D: 12.2 ->
+// 9.1).
 // ---------------------------------------------------------------------------
+constexpr int kKeysBlock = 1024;
+constexpr int kKeysWaves = kKeysBlock / kWave;
+static_assert(kPointChunk % kKeysBlock == 0, "whole rounds");
+
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_tile_keys(
+__global__ __launch_bounds__(kKeysBlock) void k_tile_keys(
     CoordPtrs<T> c, const RunParamsT<T> rp, const Chunk* __restrict__ chunks,
     const EventDesc* __restrict__ events, int group,
     const typename FloatBits<T>::Int* __restrict__ ext, T* __restrict__ geo,
@@ -204,19 +212,19 @@ __global__ __launch_bounds__(kBlock) void k_tile_keys(
   using I = typename FloatBits<T>::Int;
   constexpr I kHi = std::numeric_limits<I>::max(), kLo = std::numeric_limits<I>::min();
   __shared__ int32_t cnt[kRsMaxBins];
-  __shared__ I smin[kWaves][kMaxDim], smax[kWaves][kMaxDim];
+  __shared__ I smin[kKeysWaves][kMaxDim], smax[kKeysWaves][kMaxDim];
   __shared__ T sgeo[3 * kMaxDim];
   const Chunk ch = chunks[blockIdx.x];
   const EventDesc ev = events[ch.event];
   const int D = rp.D;
   const int bins = 1 << digit_bits;
-  for (int k = threadIdx.x; k < bins; k += kBlock) cnt[k] = 0;
+  for (int k = threadIdx.x; k < bins; k += kKeysBlock) cnt[k] = 0;
   const int first = static_cast<int>(blockIdx.x) - (ch.begin - ev.p_off) / kPointChunk;
   const int n_ext = ((ev.n + kPointChunk - 1) / kPointChunk + group - 1) / group;
   const int w = threadIdx.x / kWave;
   for (int d = 0; d < D; ++d) {
     I lo = kHi, hi = kLo;
-    for (int k = threadIdx.x; k < n_ext; k += kBlock) {
+    for (int k = threadIdx.x; k < n_ext; k += kKeysBlock) {
       const int64_t q = (static_cast<int64_t>(first + k * group) * D + d) * 2;
       const I l = ext[q], h = ext[q + 1];
       lo = l < lo ? l : lo;
@@ -233,7 +241,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_keys(
   if (threadIdx.x < D) {
     const int d = threadIdx.x;
     I lo = kHi, hi = kLo;
-    for (int k = 0; k < kWaves; ++k) {
+    for (int k = 0; k < kKeysWaves; ++k) {
       lo = smin[k][d] < lo ? smin[k][d] : lo;
       hi = smax[k][d] > hi ? smax[k][d] : hi;
     }
@@ -258,15 +266,26 @@ __global__ __launch_bounds__(kBlock) void k_tile_keys(
   g.mx = sgeo + D;
   g.side = sgeo + 2 * D;
   g.wrapped = rp.wrapped;
-  for (int i = ch.begin + threadIdx.x; i < ch.end; i += kBlock) {
-    int t = 0;
-    for (int d = 0; d < D; ++d) t = t * ev.nper + get_bin(g, c.x[d][i], d);
-    const uint32_t key = static_cast<uint32_t>(ev.t_base + t);
+  constexpr int kPer = kPointChunk / kKeysBlock;
+  int t[kPer] = {};
+  const int i0 = ch.begin + static_cast<int>(threadIdx.x);
+  for (int d = 0; d < D; ++d) {
+    T v[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) v[u] = c.x[d][min(i0 + u * kKeysBlock, ch.end - 1)];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) t[u] = t[u] * ev.nper + get_bin(g, v[u], d);
+  }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int i = i0 + u * kKeysBlock;
+    if (i >= ch.end) break;
+    const uint32_t key = static_cast<uint32_t>(ev.t_base + t[u]);
     keys[i] = key;
     atomicAdd(&cnt[key & (bins - 1)], 1);
   }
   __syncthreads();
-  for (int k = threadIdx.x; k < bins; k += kBlock)
+  for (int k = threadIdx.x; k < bins; k += kKeysBlock)
     hist[static_cast<int64_t>(k) * gridDim.x + blockIdx.x] = cnt[k];
 }
 
@@ -3113,7 +3132,7 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
                      bb.chunks, bb.events, bb.ext_group, bb.ext);
   mark(kStageTiles);
   const RadixPlan digits = radix_plan(bb.key_bits);
-  hipLaunchKernelGGL(k_tile_keys<T>, dim3(bb.n_chunks), dim3(kBlock), 0, s, cp, rp, bb.chunks,
+  hipLaunchKernelGGL(k_tile_keys<T>, dim3(bb.n_chunks), dim3(kKeysBlock), 0, s, cp, rp, bb.chunks,
                      bb.events, bb.ext_group, bb.ext, bb.geo, bb.keys0, digits.bits, bb.rs_hist);
   bool in_first = true;
   radix_sort_pairs(bb.keys0, bb.vals0, bb.keys1, bb.vals1, n, bb.key_bits, bb.rs_hist, bb.chunks,
