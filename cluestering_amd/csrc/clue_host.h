@@ -209,7 +209,7 @@ struct WorkspaceShape {
   bool own_nh = false;
   bool own_is_seed = false;
   bool sorted_boxes = false;       // density leaves out tiles by their bounding boxes
-  bool density_morton = false;     // density takes the Hilbert order (no class order for dc)
+  bool density_morton = false;     // density takes the Hilbert order of qfine
 };
 
 // Bytes of every workspace slot for a batch of this shape (0: unused).

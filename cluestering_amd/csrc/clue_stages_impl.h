@@ -9,7 +9,9 @@
 //       skips the blocks that cannot hold the answer (its result does not
 //       depend on the visiting order);
 //   (d) seeds, numbered by an exclusive scan in input order;
-//   (e) follower labels: pointer jumping, then a chase to the seed.
+//   (e) follower labels: a few hops along the links, or pointer jumping in LDS, then a
+//       chase to the seed.
+// Launches of few points have (b) and (c) done by teams of waves (clue_team.h).
 //
 // Semantics follow the reference's serial backend:
 //   geometry  core/detail/SetupTiles.hpp:23-57, core/detail/ComputeTiles.hpp:17-37
