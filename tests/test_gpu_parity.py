@@ -544,3 +544,18 @@ def test_host_arrays_of_staged_sizes(gpu_ctx, n):
         np.testing.assert_array_equal(out[1], pts.is_seed.to_host())
         np.testing.assert_array_equal(out[2].view(np.uint32), pts.rho.to_host().view(np.uint32))
         np.testing.assert_array_equal(out[3], pts.nearest_higher.to_host())
+
+
+@pytest.mark.parametrize("n", [1, 3, 5000, 32700, 33000])
+def test_work_item_scans(gpu_ctx, oracle_mod, n):
+    """1 to 33,124 tiles in launches of one wave per item: the items per tile are scanned
+    by one workgroup up to 32,768 tiles, by the general scan above."""
+    rng = np.random.default_rng(n)
+    c = rng.uniform(0, 50, (2, n)).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    gpu_ctx.set_tuning(group_queries=True, xcd_chunk_log2=4, block_waves=1)
+    try:
+        _check(Case(c, w, 0.6, 3.0, 0.9, points_per_tile=1, name=f"items n={n}"), gpu_ctx,
+               oracle_mod)
+    finally:
+        gpu_ctx.set_tuning()
