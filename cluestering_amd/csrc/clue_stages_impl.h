@@ -1091,6 +1091,20 @@ __device__ __forceinline__ uint32_t query_cell(const GeoT<T>& g, const T (&xi)[D
   return key;
 }
 
+// What a coordinate adds to a bounding box. A NaN adds every value: the Chebyshev
+// distances leave a NaN difference out of their maximum, so the point may be near
+// any other in that dimension. (Under the other metrics it is near none, and a
+// candidate's box that holds it is only wider than it need be; their query boxes leave
+// it out.)
+template <class T>
+__device__ __forceinline__ T box_low(T x) {
+  return x == x ? x : -std::numeric_limits<T>::infinity();
+}
+template <class T>
+__device__ __forceinline__ T box_high(T x) {
+  return x == x ? x : std::numeric_limits<T>::infinity();
+}
+
 // Wave-wide minimum and maximum of floating-point values.
 template <class T>
 __device__ __forceinline__ T wave_min_f(T v) {
@@ -1219,8 +1233,8 @@ __device__ __forceinline__ void write_nh_layout(int t, int b, int cnt, const int
     T lo[D], hi[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      lo[d] = real ? x[d] : std::numeric_limits<T>::infinity();
-      hi[d] = real ? x[d] : -std::numeric_limits<T>::infinity();
+      lo[d] = real ? box_low(x[d]) : std::numeric_limits<T>::infinity();
+      hi[d] = real ? box_high(x[d]) : -std::numeric_limits<T>::infinity();
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -1252,10 +1266,10 @@ __device__ __forceinline__ void tile_setup(const TileSetup& a, int t, int n_tile
                                            const T* __restrict__ sx, int64_t cs,
                                            T* __restrict__ tbox) {
   // The first points' loads go out before the search for the event.
+  const bool first_in = b + lane_id() < e;
   T x0[D];
 #pragma unroll
-  for (int d = 0; d < D; ++d)
-    x0[d] = (tbox && b + lane_id() < e) ? sx[d * cs + b + lane_id()] : std::numeric_limits<T>::quiet_NaN();
+  for (int d = 0; d < D; ++d) x0[d] = (tbox && first_in) ? sx[d * cs + b + lane_id()] : T(0);
   const int e_t = tile_event(a.events, a.n_events, t);
   const int first = first_item(a.ioff, b, t);
   const int slots = a.ioff ? (e - b + kWave - 1) / kWave
@@ -1270,10 +1284,12 @@ __device__ __forceinline__ void tile_setup(const TileSetup& a, int t, int n_tile
   }
   if (!tbox) return;
   T mn[D], mx[D];
+  bool nan[D];  // a NaN widens the box as in box_low
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    mn[d] = fmin_t(std::numeric_limits<T>::infinity(), x0[d]);
-    mx[d] = fmax_t(-std::numeric_limits<T>::infinity(), x0[d]);
+    mn[d] = first_in ? x0[d] : std::numeric_limits<T>::infinity();
+    mx[d] = first_in ? x0[d] : -std::numeric_limits<T>::infinity();
+    nan[d] = x0[d] != x0[d];
   }
 #pragma unroll 4
   for (int s = b + kWave + lane_id(); s < e; s += kWave)
@@ -1282,11 +1298,13 @@ __device__ __forceinline__ void tile_setup(const TileSetup& a, int t, int n_tile
       const T x = sx[d * cs + s];
       mn[d] = fmin_t(mn[d], x);
       mx[d] = fmax_t(mx[d], x);
+      nan[d] = nan[d] || x != x;
     }
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    mn[d] = wave_min_uniform(mn[d]);
-    mx[d] = wave_max_uniform(mx[d]);
+    const bool any = ballot(nan[d]) != 0ull;
+    mn[d] = any ? -std::numeric_limits<T>::infinity() : wave_min_uniform(mn[d]);
+    mx[d] = any ? std::numeric_limits<T>::infinity() : wave_max_uniform(mx[d]);
   }
   if (lane_id() == 0) {
 #pragma unroll
@@ -1641,7 +1659,8 @@ __device__ __forceinline__ bool box_holds(const TileGroup<D>& g, int i, const in
 }
 
 // Box of a wave's query points, and their largest sigmas (wave-uniform, in scalar
-// registers).
+// registers). A query with a NaN coordinate widens it where it can be near any
+// candidate (box_low); under the other metrics it is near none and left out.
 template <int D, class T>
 struct QueryBox {
   T lo[D], hi[D], s[D];
@@ -1651,15 +1670,20 @@ __device__ __forceinline__ QueryBox<D, T> query_box(const T (&x)[D], const T (&s
   QueryBox<D, T> q;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    q.lo[d] = wave_min_uniform(active ? x[d] : std::numeric_limits<T>::infinity());
-    q.hi[d] = wave_max_uniform(active ? x[d] : -std::numeric_limits<T>::infinity());
+    T lo = x[d], hi = x[d];
+    if constexpr (M == M_CHEBYSHEV || M == M_WCHEBYSHEV) {
+      lo = box_low(lo);
+      hi = box_high(hi);
+    }
+    q.lo[d] = wave_min_uniform(active ? lo : std::numeric_limits<T>::infinity());
+    q.hi[d] = wave_max_uniform(active ? hi : -std::numeric_limits<T>::infinity());
     q.s[d] = M == M_MAHALANOBIS ? wave_max_uniform(active ? __builtin_fabs(s[d]) : T(0)) : T(0);
   }
   return q;
 }
 // A lower bound of the metric between any query of the box and a candidate at x (with
 // sigma sx, Mahalanobis): the metric's own operations on the gaps and, Mahalanobis, on
-// the largest sigma, each monotone after rounding. A NaN excludes nothing.
+// the largest sigma, each monotone after rounding. A candidate's NaN excludes nothing.
 template <int D, int M, class T>
 __device__ __forceinline__ bool out_of_reach(const QueryBox<D, T>& q, const T (&x)[D],
                                              const T (&sx)[D], const RunParamsT<T>& rp, T thr) {
@@ -2346,8 +2370,13 @@ __attribute__((amdgpu_waves_per_eu(D <= 2 ? 8 : 1))) void k_nh_blocks(
       T qlo[D], qhi[D];
   #pragma unroll
       for (int d = 0; d < D; ++d) {
-        qlo[d] = wave_min_f(in ? xi[d] : std::numeric_limits<T>::infinity());
-        qhi[d] = wave_max_f(in ? xi[d] : -std::numeric_limits<T>::infinity());
+        T lo = xi[d], hi = xi[d];
+        if constexpr (M == M_CHEBYSHEV || M == M_WCHEBYSHEV) {
+          lo = box_low(lo);
+          hi = box_high(hi);
+        }
+        qlo[d] = wave_min_f(in ? lo : std::numeric_limits<T>::infinity());
+        qhi[d] = wave_max_f(in ? hi : -std::numeric_limits<T>::infinity());
       }
       const uint64_t kmin = wave_min_key_bound(in ? key_i : ~0ull);
       for (int c0 = 0; c0 < nblk; c0 += kWave) {

@@ -1,0 +1,70 @@
+"""Coordinates and weights that are NaN, infinite or negative, compared bit for bit
+with the oracle through every form of the neighbour stages."""
+import numpy as np
+import pytest
+
+from cluestering_amd import CLUE_Convolutional_Kernels as K
+
+from _support import Case, assert_same
+
+pytestmark = pytest.mark.gpu
+
+# None: the library's choice (teams of waves at these sizes). The others keep one wave
+# per item: over candidate blocks, scanning whole tiles, and in the tiles' own order.
+TUNINGS = [None, dict(group_queries=True), dict(group_queries=True, nh_plain_scan=True),
+           dict(group_queries=False)]
+
+METRICS = [None, K.EuclideanMetric([1.0, 2.0]), K.EuclideanMetric([1.0, 0.0]),
+           K.PeriodicEuclideanMetric([0.0, 90.0]), K.PeriodicEuclideanMetric([110.0, 90.0]),
+           K.ManhattanMetric(), K.ChebyshevMetric(), K.ChebyshevMetric([1.0, 2.0]),
+           K.MahalanobisMetric()]
+
+
+def _check(case, ctx, oracle, tuning=None):
+    print(f"[case] {case.name} n={case.n} ndim={case.ndim} {case.dtype}", flush=True)
+    if tuning is not None:
+        ctx.set_tuning(xcd_chunk_log2=4, block_waves=1, **tuning)
+    try:
+        gpu = case.run_gpu(ctx)
+    finally:
+        ctx.set_tuning()
+    assert_same(gpu, case.run_oracle(oracle), case.name)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("tuning", TUNINGS)
+@pytest.mark.parametrize("metric", METRICS)
+@pytest.mark.parametrize("special", [np.nan, np.inf])
+def test_special_coordinates(gpu_ctx, oracle_mod, special, metric, tuning, dtype):
+    """Some points have NaN or infinite coordinates, in one dimension or both. The
+    Chebyshev distances leave a NaN difference out of their maximum, so such a point
+    is near others by its other coordinates; under the other metrics it is near none.
+    Flat kernel: beyond the radius, the oracle's other kernels make a NaN distance a NaN
+    density of every point that looks at the candidate's tile."""
+    for n, ppt, every in ((120, 1000, 120), (3000, 0, 97), (3000, 12, 10)):
+        rng = np.random.default_rng(n + ppt)
+        x = rng.uniform(0, 100 if n == 120 else 60, (2, n))
+        odd = np.arange(0, n, every)
+        x[rng.integers(0, 2, odd.size), odd] = special
+        x[:, odd[::7]] = special
+        if np.isinf(special):
+            x[:, odd] *= rng.choice([-1.0, 1.0], odd.size)
+        sigma = rng.uniform(0.5, 1.5, (2, n)) if metric is not None and metric.tag == "mahalanobis" else None
+        _check(Case(x, rng.uniform(0.5, 1.5, n), 5.0 if n == 120 else 2.0, 3.0, 6.0 if n == 120 else 3.0,
+                    metric=metric, sigma=sigma, points_per_tile=ppt, dtype=dtype,
+                    name=f"{special} {metric} {tuning} ppt={ppt}"), gpu_ctx, oracle_mod, tuning)
+
+
+@pytest.mark.parametrize("kernel", [K.ExponentialKernel(0.5, 1.0), K.GaussianKernel(0.8, 1.3)])
+@pytest.mark.parametrize("tuning", TUNINGS)
+def test_nan_coordinates_chebyshev_kernels(gpu_ctx, oracle_mod, tuning, kernel):
+    """The Chebyshev distances of NaN coordinates are numbers, also under the kernels
+    that compute with them; three dimensions, one of them NaN in whole tiles."""
+    rng = np.random.default_rng(11)
+    n = 4000
+    x = rng.uniform(0, 20, (3, n))
+    x[1, rng.random(n) < 0.05] = np.nan
+    x[2, x[0] < 3] = np.nan
+    for metric in (K.ChebyshevMetric(), K.ChebyshevMetric([1.0, 0.5, 2.0])):
+        _check(Case(x, rng.uniform(0.5, 1.5, n), 1.5, 3.0, 2.5, kernel=kernel, metric=metric,
+                    points_per_tile=40, name=f"nan {metric} {kernel} {tuning}"), gpu_ctx, oracle_mod, tuning)
