@@ -134,8 +134,10 @@ RunParamsT<value_t<P>> make_run_params(const P* p, const Pts* pts, const BatchPl
   rp.seed_sq_max = sq_max(p->seed_dc);
   // The flat kernel's test v <= t as clamp((t+ - v) * 2^k): 2^k t+ in [2^60, 2^61)
   // (double: 2^120), so the unit in the last place of t+ is far above one and the
-  // products of values within the radius are finite.
-  {
+  // products of values within the radius are finite. Outside a query's search box the
+  // same test runs on -t+, which no value passes that is not below 0: not where a
+  // negative weight allows such sums (compare and select there).
+  if (rp.cull) {
     const bool root = p->metric != CLUE_METRIC_MANHATTAN && p->metric != CLUE_METRIC_CHEBYSHEV &&
                       p->metric != CLUE_METRIC_WEIGHTED_CHEBYSHEV;
     const T next = std::nextafter(root ? rp.dc_sq_max : rp.dc, std::numeric_limits<T>::infinity());

@@ -68,3 +68,16 @@ def test_nan_coordinates_chebyshev_kernels(gpu_ctx, oracle_mod, tuning, kernel):
     for metric in (K.ChebyshevMetric(), K.ChebyshevMetric([1.0, 0.5, 2.0])):
         _check(Case(x, rng.uniform(0.5, 1.5, n), 1.5, 3.0, 2.5, kernel=kernel, metric=metric,
                     points_per_tile=40, name=f"nan {metric} {kernel} {tuning}"), gpu_ctx, oracle_mod, tuning)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("tuning", TUNINGS)
+def test_negative_metric_weight_out_of_box(gpu_ctx, oracle_mod, tuning, dtype):
+    """A negative metric weight makes the sum under the root negative: here between
+    the first point and the third, whose tile its search box does not hold, while the
+    second point, of the first's tile, looks at it. No pair within a search box
+    has a negative sum."""
+    x = np.array([[0.0, 2.0, 0.0, 10.0], [0.0, 4.8, 5.6, 10.0]])
+    _check(Case(x, [1.0, 2.0, 4.0, 8.0], 0.5, 1.0, 0.5, metric=K.EuclideanMetric([1.0, -0.02]),
+                points_per_tile=1, dtype=dtype, name=f"negative weight {tuning}"), gpu_ctx, oracle_mod,
+           tuning)
