@@ -96,7 +96,7 @@ __global__ __launch_bounds__(kBlock) void k_assoc_offsets(const uint32_t* __rest
 }  // namespace
 
 int64_t assoc_hist_elems(int64_t n) {
-  return radix_hist_elems((n + kRsTileKeys - 1) / kRsTileKeys);
+  return radix_hist_elems((n + kRsTileKeys - 1) / kRsTileKeys, kRsMaxBits);
 }
 
 hipError_t assoc_stats(const int32_t* keys, int n, int32_t* stats_dev, int* blocks, hipStream_t s) {
@@ -119,8 +119,8 @@ hipError_t assoc_build(const int32_t* keys, int n, int bins, const AssocScratch&
     bool in_first = true;
     // The last pass leaves the members, which are the sorted values but for the
     // negative keys' behind them, where the caller wants them.
-    radix_sort_pairs(w.k0, w.v0, w.k1, w.v1, n, bits, w.hist, nullptr, 0, members, n_members, &in_first,
-                     s);
+    radix_sort_pairs(w.k0, w.v0, w.k1, w.v1, n, bits, w.hist, true, nullptr, 0, members, n_members,
+                     &in_first, s);
     const uint32_t* sk = in_first ? w.k0 : w.k1;
     hipLaunchKernelGGL(k_assoc_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0,
                        s, sk, n, bins, offsets);

@@ -69,6 +69,31 @@ enum Slot {
   S_QPERM, S_QPERM_NH, S_QFINE, S_HX, S_HKEY, S_HIDX, S_HBOX, S_HBKEY, S_EORDER, S_ESEEDS, S_EOFF, S_IPERM, S_SBOX, S_NUM
 };
 
+// Bits of the tile keys of a batch.
+inline int tile_key_bits(int64_t tiles) {
+  int bits = 0;
+  while ((int64_t(1) << bits) < tiles) ++bits;
+  return bits;
+}
+
+// Blocks of the tile sort: the events' chunks, whose first digits the key stage counts
+// on the way; or, where small events make more than twice as many of them as the
+// points fill, 2,048 consecutive points whatever their events (the keys are the
+// batch's). A table of digit counts per chunk would then outgrow the points, and so
+// would the workgroups. One event of 140,000 points in 2-D beside 100,000 of 10: 5,127 us
+// and 393 MB of counts by chunks, 1,773 us and 0.6 MB by points; beside 20,000 of 256
+// 2,981 and 2,235 us, 4,000 of 256 1,114 and 1,021, 2,000 of 600 1,092 and 1,063; beside
+// 1,200 of 1,024, still by chunks, 1,295.
+inline bool sort_by_chunk(int64_t points, int64_t chunks) {
+  return chunks <= 2 * ((points + clue_dev::kRsTileKeys - 1) / clue_dev::kRsTileKeys);
+}
+inline int64_t sort_hist_elems(int64_t points, int64_t chunks, int64_t tiles) {
+  const int64_t blocks =
+      sort_by_chunk(points, chunks) ? chunks
+                                    : (points + clue_dev::kRsTileKeys - 1) / clue_dev::kRsTileKeys;
+  return radix_hist_elems(blocks, clue_dev::radix_plan(tile_key_bits(tiles)).bits);
+}
+
 // Host-side description of one batch (all derived from the event sizes).
 struct BatchPlan {
   std::vector<EventDesc> events;
@@ -181,9 +206,7 @@ inline clue_status plan_batch(int D, int points_per_tile, const uint32_t* sizes,
   bp->team = !fixed && team_launch(off, static_cast<int64_t>(bp->events.size()));
   if (bp->team) bp->tuning.group_queries = 1;  // small boxes around each team's points
   bp->max_items = (off + 63) / 64 + tiles;
-  int bits = 0;
-  while ((int64_t(1) << bits) < tiles) ++bits;
-  bp->key_bits = bits;
+  bp->key_bits = tile_key_bits(tiles);
   return CLUE_OK;
 }
 
@@ -226,7 +249,7 @@ inline size_t tile_box_bytes(int64_t n, int64_t tiles, int D, int value_bytes) {
 inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) {
   std::memset(bytes, 0, sizeof(bytes));
   const int64_t n = w.n, NT = w.tiles;
-  const int64_t hist = radix_hist_elems(w.chunks);
+  const int64_t hist = sort_hist_elems(n, w.chunks, NT);
   const int64_t scan_elems =
       std::max({scan_temp_elems(n), scan_temp_elems(w.events), scan_temp_elems(NT)}) + 16;
   const int64_t stride = (n + 63) / 64 * 64;

@@ -17,17 +17,12 @@ void scan_exclusive(const int32_t* in, int32_t* out, int64_t n, int32_t* temp, i
 // radix_plan(key_bits).bits. Blocks take the chunks given (contiguous ranges in order
 // that cover [0, n)), or kRsTileKeys keys each (chunks NULL). The values are the keys'
 // places (0 to n - 1). The caller has counted the first pass's digits into hist
-// ([digit][block], then room for the totals: radix_hist_elems(n_blocks) ints). The
-// result is in (k0, v0) or (k1, v1); or, with last_values, the first last_count
-// values there and only the keys in k0 or k1.
-struct RadixPlan {
-  int bits;    // of a digit
-  int passes;
-};
-RadixPlan radix_plan(int key_bits);
+// ([digit][block], then room for the totals: radix_hist_elems ints), unless `counted` is
+// false. The result is in (k0, v0) or (k1, v1); or, with last_values, the first
+// last_count values there and only the keys in k0 or k1.
 void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int64_t n, int key_bits,
-                      int32_t* hist, const Chunk* chunks, int n_chunks, int32_t* last_values,
-                      int64_t last_count, bool* in_first, hipStream_t s);
+                      int32_t* hist, bool counted, const Chunk* chunks, int n_chunks,
+                      int32_t* last_values, int64_t last_count, bool* in_first, hipStream_t s);
 
 // ---- stages (clue_stages_impl.h, instantiated in clue_stages_f32.hip / _f64.hip) ----
 
@@ -81,6 +76,7 @@ struct BatchBuffersT {
   EventDesc* events;
   const int32_t* event_order;  // events largest first for the fused tile build; NULL: radix path
   Chunk* chunks;
+  int32_t sort_by_chunk;  // the tile sort's blocks are the chunks
   typename FloatBits<T>::Int* ext;  // [n_chunks][D][2] ordered-integer extremes
   int32_t ext_group;                // chunks per result of the extremes
   T* geo;                           // [E][3][D] mn, mx, side

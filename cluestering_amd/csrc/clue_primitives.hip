@@ -267,16 +267,9 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(
   }
 }
 
-RadixPlan radix_plan(int key_bits) {
-  RadixPlan p;
-  p.passes = key_bits <= 0 ? 1 : (key_bits + kRsMaxBits - 1) / kRsMaxBits;
-  p.bits = key_bits <= 0 ? 1 : (key_bits + p.passes - 1) / p.passes;
-  return p;
-}
-
 void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int64_t n, int key_bits,
-                      int32_t* hist, const Chunk* chunks, int n_chunks, int32_t* last_values,
-                      int64_t last_count, bool* in_first, hipStream_t s) {
+                      int32_t* hist, bool counted, const Chunk* chunks, int n_chunks,
+                      int32_t* last_values, int64_t last_count, bool* in_first, hipStream_t s) {
   *in_first = true;
   if (n <= 0) return;
   const RadixPlan plan = radix_plan(key_bits);
@@ -289,7 +282,7 @@ void radix_sort_pairs(uint32_t* k0, int32_t* v0, uint32_t* k1, int32_t* v1, int6
   for (int pass = 0; pass < plan.passes; ++pass) {
     const int shift = pass * plan.bits;
     const bool last = last_values && pass + 1 == plan.passes;
-    if (pass > 0)
+    if (pass > 0 || !counted)
       hipLaunchKernelGGL(k_rs_hist, dim3(nblocks), dim3(kBlock), 0, s, ka, n, chunks, shift,
                          plan.bits, hist);
     hipLaunchKernelGGL(k_rs_rows, dim3(static_cast<unsigned>(bins)), dim3(kBlock), 0, s, hist,

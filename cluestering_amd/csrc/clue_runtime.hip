@@ -290,6 +290,7 @@ clue_status bind_batch(void* const (&slot)[S_NUM], const BatchPlan& bp, const P*
   b.events = at<EventDesc>(slot, S_EVENTS);
   b.event_order = bp.event_order.empty() ? nullptr : at<int32_t>(slot, S_EORDER);
   b.chunks = at<Chunk>(slot, S_CHUNKS);
+  b.sort_by_chunk = sort_by_chunk(n, C) ? 1 : 0;
   b.ext = at<I>(slot, S_EXT);
   b.ext_group = bp.ext_group;
   b.geo = at<T>(slot, S_GEO);

@@ -201,25 +201,25 @@ __device__ __forceinline__ GeoT<T> event_geo(const T* geo, const RunParamsT<T>& 
 // (16,384 points in 2-D: 8.8 -> 6.2 us; 20,011 in 6-D: 17.6 -> 8.3; 2^20 in 2-D: 12.2 ->
 // 9.1).
 // ---------------------------------------------------------------------------
-constexpr int kKeysBlock = 1024;
-constexpr int kKeysWaves = kKeysBlock / kWave;
-static_assert(kPointChunk % kKeysBlock == 0, "whole rounds");
-
-template <class T>
-__global__ __launch_bounds__(kKeysBlock) void k_tile_keys(
+// Where the sort's blocks are not the chunks (small events, sort_by_chunk), nothing is
+// counted and a workgroup has 256 threads.
+template <class T, bool Count>
+__global__ __launch_bounds__(Count ? 1024 : 256) void k_tile_keys(
     CoordPtrs<T> c, const RunParamsT<T> rp, const Chunk* __restrict__ chunks,
     const EventDesc* __restrict__ events, int group,
     const typename FloatBits<T>::Int* __restrict__ ext, T* __restrict__ geo,
     uint32_t* __restrict__ keys, int digit_bits, int32_t* __restrict__ hist) {
   using I = typename FloatBits<T>::Int;
   constexpr I kHi = std::numeric_limits<I>::max(), kLo = std::numeric_limits<I>::min();
-  __shared__ int32_t cnt[kRsMaxBins];
+  constexpr int kKeysBlock = Count ? 1024 : 256;
+  constexpr int kKeysWaves = kKeysBlock / kWave;
+  __shared__ int32_t cnt[Count ? kRsMaxBins : 1];
   __shared__ I smin[kKeysWaves][kMaxDim], smax[kKeysWaves][kMaxDim];
   __shared__ T sgeo[3 * kMaxDim];
   const Chunk ch = chunks[blockIdx.x];
   const EventDesc ev = events[ch.event];
   const int D = rp.D;
-  const int bins = 1 << digit_bits;
+  const int bins = Count ? 1 << digit_bits : 0;
   for (int k = threadIdx.x; k < bins; k += kKeysBlock) cnt[k] = 0;
   const int first = static_cast<int>(blockIdx.x) - (ch.begin - ev.p_off) / kPointChunk;
   const int n_ext = ((ev.n + kPointChunk - 1) / kPointChunk + group - 1) / group;
@@ -268,24 +268,26 @@ __global__ __launch_bounds__(kKeysBlock) void k_tile_keys(
   g.mx = sgeo + D;
   g.side = sgeo + 2 * D;
   g.wrapped = rp.wrapped;
-  constexpr int kPer = kPointChunk / kKeysBlock;
-  int t[kPer] = {};
-  const int i0 = ch.begin + static_cast<int>(threadIdx.x);
-  for (int d = 0; d < D; ++d) {
-    T v[kPer];
+  constexpr int kPer = 2;
+  for (int i0 = ch.begin + static_cast<int>(threadIdx.x); i0 < ch.end; i0 += kPer * kKeysBlock) {
+    int t[kPer] = {};
+    for (int d = 0; d < D; ++d) {
+      T v[kPer];
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) v[u] = c.x[d][min(i0 + u * kKeysBlock, ch.end - 1)];
+      for (int u = 0; u < kPer; ++u) v[u] = c.x[d][min(i0 + u * kKeysBlock, ch.end - 1)];
 #pragma unroll
-    for (int u = 0; u < kPer; ++u) t[u] = t[u] * ev.nper + get_bin(g, v[u], d);
+      for (int u = 0; u < kPer; ++u) t[u] = t[u] * ev.nper + get_bin(g, v[u], d);
+    }
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int i = i0 + u * kKeysBlock;
+      if (i >= ch.end) break;
+      const uint32_t key = static_cast<uint32_t>(ev.t_base + t[u]);
+      keys[i] = key;
+      if constexpr (Count) atomicAdd(&cnt[key & (bins - 1)], 1);
+    }
   }
-#pragma unroll
-  for (int u = 0; u < kPer; ++u) {
-    const int i = i0 + u * kKeysBlock;
-    if (i >= ch.end) break;
-    const uint32_t key = static_cast<uint32_t>(ev.t_base + t[u]);
-    keys[i] = key;
-    atomicAdd(&cnt[key & (bins - 1)], 1);
-  }
+  if constexpr (!Count) return;
   __syncthreads();
   for (int k = threadIdx.x; k < bins; k += kKeysBlock)
     hist[static_cast<int64_t>(k) * gridDim.x + blockIdx.x] = cnt[k];
@@ -2854,32 +2856,35 @@ static __global__ __launch_bounds__(kBlock) void k_event_labels(
 }
 
 // The same after k_results: a seed's rank over the whole batch is the number of seed
-// bits before its own.
+// bits before its own. 2^parts_log2 workgroups share a chunk: as many as a full one has
+// rounds, or one where most are far from full.
 static __global__ __launch_bounds__(kBlock) void k_labels(
     const Chunk* __restrict__ chunks, const EventDesc* __restrict__ events,
     const int32_t* __restrict__ perm, const int32_t* __restrict__ link,
     const uint32_t* __restrict__ bits, const int32_t* __restrict__ before,
     int32_t* __restrict__ cluster, int32_t* __restrict__ seeds,
-    int32_t* __restrict__ event_of_cluster, int local_ids) {
+    int32_t* __restrict__ event_of_cluster, int local_ids, int parts_log2) {
   auto rank = [&](int i) {
     return before[i >> 5] + __popc(bits[i >> 5] & ((1u << (i & 31)) - 1u));
   };
-  const Chunk ch = chunks[blockIdx.x / (kPointChunk / kBlock)];
-  const int s = ch.begin + (blockIdx.x % (kPointChunk / kBlock)) * kBlock + threadIdx.x;
-  if (s >= ch.end) return;
+  const Chunk ch = chunks[blockIdx.x >> parts_log2];
   const EventDesc ev = events[ch.event];
-  int cur = s;
-  int nx = link[cur];
-  while (nx >= 0) {
-    cur = nx;
-    nx = link[cur];
-  }
-  const int i = perm[s];
-  const int c = (nx == -2) ? rank(perm[cur]) : -1;
-  cluster[i] = c >= 0 ? c - (local_ids ? rank(ev.p_off) : 0) : -1;
-  if (cur == s && nx == -2) {
-    seeds[c] = i;
-    if (event_of_cluster) event_of_cluster[c] = ev.index;
+  const int part = static_cast<int>(blockIdx.x) & ((1 << parts_log2) - 1);
+  for (int s = ch.begin + part * kBlock + static_cast<int>(threadIdx.x); s < ch.end;
+       s += kBlock << parts_log2) {
+    int cur = s;
+    int nx = link[cur];
+    while (nx >= 0) {
+      cur = nx;
+      nx = link[cur];
+    }
+    const int i = perm[s];
+    const int c = (nx == -2) ? rank(perm[cur]) : -1;
+    cluster[i] = c >= 0 ? c - (local_ids ? rank(ev.p_off) : 0) : -1;
+    if (cur == s && nx == -2) {
+      seeds[c] = i;
+      if (event_of_cluster) event_of_cluster[c] = ev.index;
+    }
   }
 }
 
@@ -3189,11 +3194,13 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
                      bb.chunks, bb.events, bb.ext_group, bb.ext);
   mark(kStageTiles);
   const RadixPlan digits = radix_plan(bb.key_bits);
-  hipLaunchKernelGGL(k_tile_keys<T>, dim3(bb.n_chunks), dim3(kKeysBlock), 0, s, cp, rp, bb.chunks,
-                     bb.events, bb.ext_group, bb.ext, bb.geo, bb.keys0, digits.bits, bb.rs_hist);
+  const bool by_chunk = bb.sort_by_chunk != 0;
+  hipLaunchKernelGGL((by_chunk ? k_tile_keys<T, true> : k_tile_keys<T, false>), dim3(bb.n_chunks),
+                     dim3(by_chunk ? 1024 : 256), 0, s, cp, rp, bb.chunks, bb.events, bb.ext_group,
+                     bb.ext, bb.geo, bb.keys0, digits.bits, bb.rs_hist);
   bool in_first = true;
-  radix_sort_pairs(bb.keys0, bb.vals0, bb.keys1, bb.vals1, n, bb.key_bits, bb.rs_hist, bb.chunks,
-                   bb.n_chunks, nullptr, 0, &in_first, s);
+  radix_sort_pairs(bb.keys0, bb.vals0, bb.keys1, bb.vals1, n, bb.key_bits, bb.rs_hist, by_chunk,
+                   by_chunk ? bb.chunks : nullptr, bb.n_chunks, nullptr, 0, &in_first, s);
   const uint32_t* skeys = in_first ? bb.keys0 : bb.keys1;
   const int32_t* sperm = in_first ? bb.vals0 : bb.vals1;
   GatherArgs<T> ga;
@@ -3272,9 +3279,11 @@ void launch_pipeline(const RunParamsT<T>& rp, const PointArraysT<T>& in, const B
       scan_exclusive(bb.rank, bb.rank, words, bb.scan_tmp, bb.n_seeds, s);
     }
     mark(kStageLabels);
-    hipLaunchKernelGGL(k_labels, dim3(bb.n_chunks * (kPointChunk / kBlock)), dim3(kBlock), 0, s,
-                       bb.chunks, bb.events, bb.sorted.perm, bb.snh, bits, bb.rank, out.cluster,
-                       bb.seeds, out.event_of_cluster, out.local_ids);
+    static_assert(kPointChunk == kBlock << 3, "eight rounds of a full chunk");
+    const int parts_log2 = bb.sort_by_chunk ? 3 : 0;
+    hipLaunchKernelGGL(k_labels, dim3(static_cast<unsigned>(bb.n_chunks) << parts_log2), dim3(kBlock),
+                       0, s, bb.chunks, bb.events, bb.sorted.perm, bb.snh, bits, bb.rank, out.cluster,
+                       bb.seeds, out.event_of_cluster, out.local_ids, parts_log2);
   }
   mark(kNumStages);
 }

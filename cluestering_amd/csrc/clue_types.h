@@ -33,8 +33,22 @@ constexpr int kRsMaxBits = 10;        // of a radix digit
 constexpr int kRsMaxBins = 1 << kRsMaxBits;
 static_assert(kPointChunk == kRsTileKeys, "a chunk is a block of the radix sort");
 inline int64_t scan_temp_elems(int64_t n) { return (n + kScanTileElems - 1) / kScanTileElems + 1; }
+// Digits of a radix sort by key_bits bits: as few passes as kRsMaxBits allows, of equal
+// widths.
+struct RadixPlan {
+  int bits;  // of a digit
+  int passes;
+};
+inline RadixPlan radix_plan(int key_bits) {
+  RadixPlan p;
+  p.passes = key_bits <= 0 ? 1 : (key_bits + kRsMaxBits - 1) / kRsMaxBits;
+  p.bits = key_bits <= 0 ? 1 : (key_bits + p.passes - 1) / p.passes;
+  return p;
+}
 // Digit counts per block, then the digits' totals.
-inline int64_t radix_hist_elems(int64_t blocks) { return kRsMaxBins * (blocks + 1); }
+inline int64_t radix_hist_elems(int64_t blocks, int digit_bits) {
+  return (blocks + 1) << digit_bits;
+}
 
 // Constants of the float exp (Cody-Waite reduction x = k ln2 + r with a 15-bit
 // ln2_hi, then the degree-6 minimax polynomial of e^r on [-ln2/2, ln2/2] whose

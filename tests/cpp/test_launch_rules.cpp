@@ -1,0 +1,57 @@
+// The rules by which the host sizes and shapes a launch, on the CPU (built with g++
+// under the address and undefined-behaviour sanitizers).
+#include <cstdio>
+#include <vector>
+
+#include "clue_host.h"
+
+static int g_fail = 0, g_pass = 0;
+#define CHECK(cond)                                              \
+  do {                                                           \
+    if (cond) {                                                  \
+      ++g_pass;                                                  \
+    } else {                                                     \
+      ++g_fail;                                                  \
+      std::printf("FAIL %s:%d: %s\n", __FILE__, __LINE__, #cond); \
+    }                                                            \
+  } while (0)
+
+using namespace clue_rt;
+
+// One event too large for the fused stages beside many small ones: the sort's digit
+// counts grow with the points, however many events they come in.
+static void test_sort_histogram() {
+  for (int D = 1; D <= 10; ++D)
+    for (uint32_t small : {1u, 10u, 64u, 256u, 700u, 2049u})
+      for (int count : {0, 1, 100, 5000, 100000}) {
+        std::vector<uint32_t> sizes(static_cast<size_t>(count) + 1, small);
+        sizes[0] = 140000;
+        BatchPlan bp;
+        std::string err;
+        CHECK(plan_batch(D, 0, sizes.data(), count + 1, nullptr, &bp, &err) == CLUE_OK);
+        CHECK(bp.event_order.empty());  // the radix path
+        WorkspaceShape w;
+        w.D = D;
+        w.n = bp.n_total;
+        w.events = static_cast<int64_t>(bp.events.size());
+        w.chunks = static_cast<int64_t>(bp.chunks.size());
+        w.tiles = bp.n_tiles_total;
+        w.max_items = bp.max_items;
+        size_t b[S_NUM];
+        workspace_requests(w, b);
+        CHECK(b[S_HIST] <= 4 * static_cast<size_t>(bp.n_total) + (64 << 10));
+        // Room for the counts of every block of the sort and the totals.
+        const int64_t blocks = sort_by_chunk(w.n, w.chunks) ? w.chunks : (w.n + 2047) / 2048;
+        const int bits = clue_dev::radix_plan(bp.key_bits).bits;
+        CHECK(b[S_HIST] >= sizeof(int32_t) * static_cast<size_t>((blocks + 1) << bits));
+      }
+  // A lone event's chunks are full: they are the blocks.
+  for (int64_t n : {1, 2047, 2048, 2049, 140000, 1 << 20})
+    CHECK(sort_by_chunk(n, (n + 2047) / 2048));
+}
+
+int main() {
+  test_sort_histogram();
+  std::printf("%d passed, %d failed\n", g_pass, g_fail);
+  return g_fail == 0 ? 0 : 1;
+}

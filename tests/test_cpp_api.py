@@ -53,6 +53,11 @@ def test_sqrt_sign_selection_is_correctly_rounded():
     _run("test_sqrt_select")
 
 
+def test_launch_rules_under_sanitizers():
+    """The host's rules for the shape and the workspace of a launch."""
+    _run("test_launch_rules")
+
+
 @pytest.mark.gpu
 def test_cpp_dropin_program():
     _run("test_clusterer", os.path.join(ROOT, "tests", "golden", "reference_data"))

@@ -559,3 +559,29 @@ def test_work_item_scans(gpu_ctx, oracle_mod, n):
                oracle_mod)
     finally:
         gpu_ctx.set_tuning()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("small,count", [(5, 2), (5, 3), (5, 3000), (300, 40), (2049, 9)])
+def test_large_event_among_small_ones(gpu_ctx, oracle_mod, small, count, dtype):
+    """An event of 1,521 tiles sends its batch down the radix path, whose sort takes the
+    events' chunks as blocks (2 and 9 small events) or, where most would be nearly empty,
+    2,048 points whatever their events."""
+    from cluestering_amd.device import Clusterer, PointsDevice
+    rng = np.random.default_rng(small + count)
+    sizes = np.full(count + 1, small, np.uint32)
+    sizes[count // 2] = 3000
+    n = int(sizes.sum())
+    c = rng.uniform(0, 30, (2, n)).astype(dtype)
+    w = rng.uniform(0.5, 1.5, n).astype(dtype)
+    kern = K.GaussianKernel(1.0, 1.0)
+    gpu, ref = _check(Case(c, w, 1.0, 1.5, 1.5, kernel=kern, sizes=sizes, points_per_tile=2, dtype=dtype,
+                           name=f"{count} x {small}"), gpu_ctx, oracle_mod)
+    assert gpu["n_clusters"] == ref.n_seeds
+    pts = PointsDevice.from_host(gpu_ctx, c, w, dtype=dtype)
+    algo = Clusterer(gpu_ctx, 1.0, 1.5, 1.5)
+    algo.points_per_tile = 2
+    eoc = gpu_ctx.empty(n, np.int32)
+    k = algo.make_clusters_batched(pts, sizes, None, kern, event_of_cluster=eoc)
+    event = np.repeat(np.arange(count + 1), sizes)
+    np.testing.assert_array_equal(eoc.to_host()[:k], event[np.nonzero(ref.is_seed)[0]])
