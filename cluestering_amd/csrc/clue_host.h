@@ -35,6 +35,17 @@ constexpr int kDefaultPointsPerTile = 128;
 constexpr int kTeamMaxPoints = 110000;
 constexpr int kTeamMaxPointsSmall = 49152;  // events of fewer than kTeamSmallEvent points
 constexpr int kTeamSmallEvent = 4096;
+// A team costs 5-13 ns of the chip whatever its item holds (512 threads to start, eight
+// waves' worth of set-up), which only a long walk pays back: the item slots must hold
+// kTeamItemPoints points on average. (Tiles of few points, by points_per_tile or by many
+// dimensions: 100,000 points at 4 per tile 798 us in 2-D and 944 in 3-D by teams, 472 and
+// 510 by waves; 50,000 in 8-D, 7 per slot, 758 and 582; 100,000 in 6-D, 18 per slot, 609
+// and 718; 3,000 events of 16 285 and 212.) A lone event of few points and as few items
+// still has CUs to spare: up to kTeamItemWork points times slots (8,000 points at one
+// per tile 165 us by teams and 281 by waves, 16,384 at one 293 and 368, 50,000 at 16
+// 348 and 353; 20,000 in 6-D at four, 3.2e8, 411 and 303).
+constexpr int kTeamItemPoints = 16;
+constexpr int64_t kTeamItemWork = 300000000;
 
 // Constants of exp(y * 2^-s) (clue_dev::ExpScaled): each constant of the float
 // exp scaled by a power of two, exact for |s| <= 8.
@@ -50,9 +61,11 @@ inline clue_dev::ExpScaled exp_scaled(int s) {
   return e;
 }
 
-inline bool team_launch(int64_t points, int64_t events) {
+// max_items: the launch's item slots.
+inline bool team_launch(int64_t points, int64_t events, int64_t max_items) {
   const bool small = events > 1 && points / events < kTeamSmallEvent;
-  return points <= (small ? kTeamMaxPointsSmall : kTeamMaxPoints);
+  if (points > (small ? kTeamMaxPointsSmall : kTeamMaxPoints)) return false;
+  return points >= kTeamItemPoints * max_items || (events == 1 && points * max_items <= kTeamItemWork);
 }
 
 // Capacity a grow-only device buffer holds after a request of `bytes`: unchanged
@@ -81,7 +94,7 @@ inline int tile_key_bits(int64_t tiles) {
 // points fill, 2,048 consecutive points whatever their events (the keys are the
 // batch's). A table of digit counts per chunk would then outgrow the points, and so
 // would the workgroups. One event of 140,000 points in 2-D beside 100,000 of 10: 5,127 us
-// and 393 MB of counts by chunks, 1,773 us and 0.6 MB by points; beside 20,000 of 256
+// and 414 MB of counts by chunks, 1,773 us and 1.1 MB by points; beside 20,000 of 256
 // 2,981 and 2,235 us, 4,000 of 256 1,114 and 1,021, 2,000 of 600 1,092 and 1,063; beside
 // 1,200 of 1,024, still by chunks, 1,295.
 inline bool sort_by_chunk(int64_t points, int64_t chunks) {
@@ -202,10 +215,10 @@ inline clue_status plan_batch(int D, int points_per_tile, const uint32_t* sizes,
   int64_t largest = 0;
   for (const EventDesc& ev : bp->events) largest = std::max<int64_t>(largest, ev.n);
   bp->ext_group = static_cast<int>(std::max<int64_t>(1, (largest + 512 * kChunk - 1) / (512 * kChunk)));
-  // A fixed tuning keeps one wave per item.
-  bp->team = !fixed && team_launch(off, static_cast<int64_t>(bp->events.size()));
-  if (bp->team) bp->tuning.group_queries = 1;  // small boxes around each team's points
   bp->max_items = (off + 63) / 64 + tiles;
+  // A fixed tuning keeps one wave per item.
+  bp->team = !fixed && team_launch(off, static_cast<int64_t>(bp->events.size()), bp->max_items);
+  if (bp->team) bp->tuning.group_queries = 1;  // small boxes around each team's points
   bp->key_bits = tile_key_bits(tiles);
   return CLUE_OK;
 }

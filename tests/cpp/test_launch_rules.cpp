@@ -50,7 +50,29 @@ static void test_sort_histogram() {
     CHECK(sort_by_chunk(n, (n + 2047) / 2048));
 }
 
+static bool team(int D, int per_tile, uint32_t n, int count = 1) {
+  std::vector<uint32_t> sizes(static_cast<size_t>(count), n);
+  BatchPlan bp;
+  std::string err;
+  CHECK(plan_batch(D, per_tile, sizes.data(), count, nullptr, &bp, &err) == CLUE_OK);
+  return bp.team;
+}
+
+// Teams of waves where an item's walk is long; one wave per item where the items are many
+// and hold few points.
+static void test_team_rule() {
+  for (int D = 1; D <= 7; ++D)
+    for (uint32_t n : {1u, 300u, 5003u, 20011u, 30000u, 65536u}) CHECK(team(D, 0, n));
+  CHECK(team(2, 0, 110000) && !team(2, 0, 110001));
+  CHECK(team(2, 1, 3000) && team(2, 1, 8000) && team(2, 16, 50000));
+  CHECK(!team(2, 1, 50000) && !team(2, 1, 100000) && !team(2, 4, 100000) && !team(3, 4, 100000));
+  CHECK(!team(6, 4, 20000) && !team(6, 8, 100000) && !team(8, 0, 50000));
+  CHECK(team(2, 0, 1000, 48) && team(2, 0, 400, 100) && team(3, 0, 4100, 26));
+  CHECK(!team(2, 0, 16, 3000) && !team(2, 0, 1, 40000) && !team(2, 0, 1000, 50));
+}
+
 int main() {
+  test_team_rule();
   test_sort_histogram();
   std::printf("%d passed, %d failed\n", g_pass, g_fail);
   return g_fail == 0 ? 0 : 1;
