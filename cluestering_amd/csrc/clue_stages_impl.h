@@ -1093,11 +1093,10 @@ __device__ __forceinline__ uint32_t query_cell(const GeoT<T>& g, const T (&xi)[D
   return key;
 }
 
-// What a coordinate adds to a bounding box. A NaN adds every value: the Chebyshev
-// distances leave a NaN difference out of their maximum, so the point may be near
-// any other in that dimension. (Under the other metrics it is near none, and a
-// candidate's box that holds it is only wider than it need be; their query boxes leave
-// it out.)
+// What a coordinate adds to a bounding box under the Chebyshev distances. They leave a
+// NaN difference out of their maximum, so a point with a NaN may be near any other in
+// that dimension, and it adds every value. (Under the other metrics it is near none, and
+// their boxes leave it out.)
 template <class T>
 __device__ __forceinline__ T box_low(T x) {
   return x == x ? x : -std::numeric_limits<T>::infinity();
@@ -1209,7 +1208,7 @@ __device__ __forceinline__ int64_t nh_first_block(int b, int t) {
 // density stage itself (k_density, from the same Hilbert order).
 template <int D, class T>
 __device__ __forceinline__ void write_nh_layout(int t, int b, int cnt, const int32_t* order,
-                                                int w, int n_waves,
+                                                int w, int n_waves, int nan_widens,
                                                 const T* __restrict__ sx, int64_t cs,
                                                 T* __restrict__ hx, int64_t hs,
                                                 int32_t* __restrict__ hidx, T* __restrict__ hbox) {
@@ -1235,8 +1234,15 @@ __device__ __forceinline__ void write_nh_layout(int t, int b, int cnt, const int
     T lo[D], hi[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      lo[d] = real ? box_low(x[d]) : std::numeric_limits<T>::infinity();
-      hi[d] = real ? box_high(x[d]) : -std::numeric_limits<T>::infinity();
+      lo[d] = real ? x[d] : std::numeric_limits<T>::infinity();
+      hi[d] = real ? x[d] : -std::numeric_limits<T>::infinity();
+    }
+    if (nan_widens) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        lo[d] = box_low(lo[d]);
+        hi[d] = box_high(hi[d]);
+      }
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -1262,16 +1268,17 @@ struct TileSetup {
   Item* items;
   const int32_t* ioff;
   int32_t max_items;
+  int32_t nan_widens;  // the metric is one of the Chebyshev distances (box_low)
 };
 template <int D, class T>
 __device__ __forceinline__ void tile_setup(const TileSetup& a, int t, int n_tiles, int b, int e,
                                            const T* __restrict__ sx, int64_t cs,
                                            T* __restrict__ tbox) {
   // The first points' loads go out before the search for the event.
-  const bool first_in = b + lane_id() < e;
   T x0[D];
 #pragma unroll
-  for (int d = 0; d < D; ++d) x0[d] = (tbox && first_in) ? sx[d * cs + b + lane_id()] : T(0);
+  for (int d = 0; d < D; ++d)
+    x0[d] = (tbox && b + lane_id() < e) ? sx[d * cs + b + lane_id()] : std::numeric_limits<T>::quiet_NaN();
   const int e_t = tile_event(a.events, a.n_events, t);
   const int first = first_item(a.ioff, b, t);
   const int slots = a.ioff ? (e - b + kWave - 1) / kWave
@@ -1286,12 +1293,10 @@ __device__ __forceinline__ void tile_setup(const TileSetup& a, int t, int n_tile
   }
   if (!tbox) return;
   T mn[D], mx[D];
-  bool nan[D];  // a NaN widens the box as in box_low
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    mn[d] = first_in ? x0[d] : std::numeric_limits<T>::infinity();
-    mx[d] = first_in ? x0[d] : -std::numeric_limits<T>::infinity();
-    nan[d] = x0[d] != x0[d];
+    mn[d] = fmin_t(std::numeric_limits<T>::infinity(), x0[d]);
+    mx[d] = fmax_t(-std::numeric_limits<T>::infinity(), x0[d]);
   }
 #pragma unroll 4
   for (int s = b + kWave + lane_id(); s < e; s += kWave)
@@ -1300,13 +1305,20 @@ __device__ __forceinline__ void tile_setup(const TileSetup& a, int t, int n_tile
       const T x = sx[d * cs + s];
       mn[d] = fmin_t(mn[d], x);
       mx[d] = fmax_t(mx[d], x);
-      nan[d] = nan[d] || x != x;
     }
+  if (a.nan_widens) {
+    for (int s = b + lane_id(); s < e; s += kWave)
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        const T x = sx[d * cs + s];
+        mn[d] = fmin_t(mn[d], box_low(x));
+        mx[d] = fmax_t(mx[d], box_high(x));
+      }
+  }
 #pragma unroll
   for (int d = 0; d < D; ++d) {
-    const bool any = ballot(nan[d]) != 0ull;
-    mn[d] = any ? -std::numeric_limits<T>::infinity() : wave_min_uniform(mn[d]);
-    mx[d] = any ? std::numeric_limits<T>::infinity() : wave_max_uniform(mx[d]);
+    mn[d] = wave_min_uniform(mn[d]);
+    mx[d] = wave_max_uniform(mx[d]);
   }
   if (lane_id() == 0) {
 #pragma unroll
@@ -1363,7 +1375,7 @@ __global__ __launch_bounds__(W * kWave) void k_query_order(
     if (mine) tile_setup<D>(setup, t, n_tiles, b, e, sx, cs, tbox);
     if (mine && e - b <= kWave) {  // one item: the query order is irrelevant
       if (b + lane < e) qfine[b + lane] = b + lane;
-      if (hx) write_nh_layout<D>(t, b, e - b, nullptr, 0, 1, sx, cs, hx, hs, hidx, hbox);
+      if (hx) write_nh_layout<D>(t, b, e - b, nullptr, 0, 1, setup.nan_widens, sx, cs, hx, hs, hidx, hbox);
     }
   }
   for (int k = 0; k < per; ++k) {
@@ -1427,7 +1439,7 @@ __global__ __launch_bounds__(W * kWave) void k_query_order(
       qfine[atomicAdd(&cnt[key_of(s)], 1)] = s;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");  // qfine of the tile
     __syncthreads();
-    if (hx) write_nh_layout<D>(t, b, e - b, qfine, w, W, sx, cs, hx, hs, hidx, hbox);
+    if (hx) write_nh_layout<D>(t, b, e - b, qfine, w, W, setup.nan_widens, sx, cs, hx, hs, hidx, hbox);
   }
 }
 
@@ -3085,12 +3097,19 @@ CLUE_NEIGHBOUR_EXTERN(9)
 CLUE_NEIGHBOUR_EXTERN(10)
 #undef CLUE_NEIGHBOUR_EXTERN
 
+template <class T>
+static TileSetup tile_setup_of(const NeighbourLaunch<T>& L) {
+  const BatchBuffersT<T>& b = *L.bb;
+  const bool chebyshev = L.rp->metric == M_CHEBYSHEV || L.rp->metric == M_WCHEBYSHEV;
+  return {b.events, b.n_events, b.items, b.icount, b.max_items, chebyshev ? 1 : 0};
+}
+
 constexpr int kOrderTilesAlone = 2048;  // 8 workgroups of 8 waves per CU
 
 template <int D, class T>
 static void launch_query_order_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
-  const TileSetup setup{b.events, b.n_events, b.items, b.icount, b.max_items};
+  const TileSetup setup = tile_setup_of(L);
   // Tiles per workgroup, whose sorts run one after the other. Few tiles leave CUs idle,
   // so each takes a workgroup of its own (5,003 points in 2-D: 13.4 us with eight
   // tiles, 7.2 with two, 5.7 with one; 16,384 points 13.2 -> 6.1, 20,011 in 6-D 12.2 ->
@@ -3117,7 +3136,7 @@ template <int D, class T>
 static void launch_tile_setup_d(const NeighbourLaunch<T>& L) {
   const BatchBuffersT<T>& b = *L.bb;
   const unsigned grid = static_cast<unsigned>((b.n_tiles_total + kWaves - 1) / kWaves);
-  const TileSetup setup{b.events, b.n_events, b.items, b.icount, b.max_items};
+  const TileSetup setup = tile_setup_of(L);
   hipLaunchKernelGGL((k_tile_setup<D, T>), dim3(grid), dim3(kBlock), 0, L.s, setup, b.toff,
                      b.n_tiles_total, b.sorted.x[0], L.cs, b.tbox, b.n_items);
 }
