@@ -106,7 +106,8 @@ class Tuning(C.Structure):
         ("block_waves", C.c_int32),
         ("nh_plain_scan", C.c_int32),
         ("persistent", C.c_int32),
-        ("reserved", C.c_int32 * 3),
+        ("team", C.c_int32),
+        ("reserved", C.c_int32 * 2),
     ]
 
 

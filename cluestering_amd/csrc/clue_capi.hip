@@ -562,6 +562,7 @@ clue_status clue_set_tuning(clue_ctx* ctx, const clue_tuning* tuning) {
     ctx->tuning.block_waves = tuning->block_waves ? tuning->block_waves : 4;
     ctx->tuning.nh_plain_scan = tuning->nh_plain_scan ? 1 : 0;
     ctx->tuning.persistent = tuning->persistent;
+    ctx->tuning.team = tuning->team ? 1 : 0;
   }
   return CLUE_OK;
 }
@@ -573,17 +574,25 @@ clue_status clue_get_tuning(clue_ctx* ctx, const clue_params* params, int32_t n,
     *out = ctx->tuning;
     return CLUE_OK;
   }
-  int64_t total = 0, events = 0;
+  int64_t total = 0, events = 0, tiles = 0;
+  const bool tiled = params->ndim >= 1 && params->ndim <= kMaxDim;  // else no run takes them
+  auto add = [&](int64_t points) {
+    int64_t nper = 0, nt = 0;
+    if (tiled)
+      event_tiles(points, params->ndim,
+                  params->points_per_tile > 0 ? params->points_per_tile : kDefaultPointsPerTile, &nper,
+                  &nt);
+    total += points;
+    tiles += nt;
+    ++events;
+  };
   if (sizes) {
-    for (int32_t e = 0; e < n_events; ++e) {
-      total += sizes[e];
-      events += sizes[e] > 0 ? 1 : 0;
-    }
-  } else {
-    total = n;
-    events = 1;
+    for (int32_t e = 0; e < n_events; ++e)
+      if (sizes[e] > 0) add(sizes[e]);
+  } else if (n > 0) {
+    add(n);
   }
-  *out = table_tuning(params->ndim, total, events);
+  *out = chosen_tuning(params->ndim, total, events, (total + 63) / 64 + tiles);
   return CLUE_OK;
 }
 

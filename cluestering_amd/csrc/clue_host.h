@@ -154,6 +154,14 @@ inline clue_tuning table_tuning(int ndim, int64_t n_total, int64_t n_events) {
   return out;
 }
 
+// The tuning of a run that none is fixed for: the table's, or teams of waves.
+inline clue_tuning chosen_tuning(int ndim, int64_t points, int64_t events, int64_t max_items) {
+  clue_tuning t = table_tuning(ndim, points, events);
+  t.team = team_launch(points, events, max_items) ? 1 : 0;
+  if (t.team) t.group_queries = 1;  // small boxes around each team's points
+  return t;
+}
+
 // Builds the batch descriptor: one EventDesc per non-empty event, its chunks,
 // tile bases, work-item bound and radix key width. `fixed` (may be NULL) replaces
 // the table's tuning. Returns CLUE_OK, or CLUE_ERR_CAPACITY with *err set when the
@@ -210,15 +218,16 @@ inline clue_status plan_batch(int D, int points_per_tile, const uint32_t* sizes,
       std::stable_sort(bp->event_order.begin(), bp->event_order.end(),
                        [&](int32_t a, int32_t b) { return bp->events[a].n > bp->events[b].n; });
   }
-  bp->tuning = fixed ? *fixed : table_tuning(D, off, static_cast<int64_t>(bp->events.size()));
   // At most 512 results per event: every workgroup of the key stage reads them all.
   int64_t largest = 0;
   for (const EventDesc& ev : bp->events) largest = std::max<int64_t>(largest, ev.n);
   bp->ext_group = static_cast<int>(std::max<int64_t>(1, (largest + 512 * kChunk - 1) / (512 * kChunk)));
   bp->max_items = (off + 63) / 64 + tiles;
-  // A fixed tuning keeps one wave per item.
-  bp->team = !fixed && team_launch(off, static_cast<int64_t>(bp->events.size()), bp->max_items);
-  if (bp->team) bp->tuning.group_queries = 1;  // small boxes around each team's points
+  const int64_t n_described = static_cast<int64_t>(bp->events.size());
+  bp->tuning = fixed ? *fixed : chosen_tuning(D, off, n_described, bp->max_items);
+  // A fixed tuning allows teams; the launch must still be small enough for them.
+  bp->team = bp->tuning.team && team_launch(off, n_described, bp->max_items);
+  if (bp->team) bp->tuning.group_queries = 1;
   bp->key_bits = tile_key_bits(tiles);
   return CLUE_OK;
 }

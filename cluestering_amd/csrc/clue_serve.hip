@@ -74,9 +74,8 @@ int64_t lane_bytes(const clue_params& p, const clue_srv::BatchShape& shape, cons
   bp.n_total = shape.points;
   bp.n_tiles_total = shape.tiles;
   bp.max_items = (shape.points + 63) / 64 + shape.tiles;
-  bp.tuning = table_tuning(p.ndim, shape.points, shape.events);
-  bp.team = team_launch(shape.points, shape.events, bp.max_items);
-  if (bp.team) bp.tuning.group_queries = 1;
+  bp.tuning = chosen_tuning(p.ndim, shape.points, shape.events, bp.max_items);
+  bp.team = bp.tuning.team != 0;
   bp.events.resize(static_cast<size_t>(shape.events));
   bp.chunks.resize(static_cast<size_t>(shape.chunks));
   clue_points pts{};

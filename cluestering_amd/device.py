@@ -69,12 +69,14 @@ class Context:
                    xcd_chunk_log2: Optional[int] = None,
                    block_waves: Optional[int] = None,
                    nh_plain_scan: Optional[bool] = None,
-                   persistent: Optional[int] = None) -> None:
+                   persistent: Optional[int] = None,
+                   team: Optional[bool] = None) -> None:
         """Fix the launch tuning of later runs (speed only; results never change).
         persistent: waves per CU that pull work items from device queues (0: one
-        wave per item). With no arguments the built-in table chooses again."""
+        wave per item). team: teams of waves per item in the launches small enough
+        for it (not given: none). With no arguments the built-in table chooses again."""
         if (group_queries is None and xcd_chunk_log2 is None and block_waves is None
-                and nh_plain_scan is None and persistent is None):
+                and nh_plain_scan is None and persistent is None and team is None):
             _capi.check(self._lib.clue_set_tuning(self.handle, None))
             return
         t = _capi.Tuning()
@@ -83,6 +85,7 @@ class Context:
         t.block_waves = 4 if block_waves is None else int(block_waves)
         t.nh_plain_scan = 1 if nh_plain_scan else 0
         t.persistent = 0 if persistent is None else int(persistent)
+        t.team = 1 if team else 0
         _capi.check(self._lib.clue_set_tuning(self.handle, C.byref(t)))
 
     def get_tuning(self, params: _capi.Params, sizes: Sequence[int]) -> dict:
@@ -94,7 +97,7 @@ class Context:
                                               len(sz), C.byref(t)))
         return {"group_queries": bool(t.group_queries), "xcd_chunk_log2": int(t.xcd_chunk_log2),
                 "block_waves": int(t.block_waves), "nh_plain_scan": bool(t.nh_plain_scan),
-                "persistent": int(t.persistent)}
+                "persistent": int(t.persistent), "team": bool(t.team)}
 
     def set_profiling(self, enabled: bool) -> None:
         _capi.check(self._lib.clue_set_profiling(self.handle, 1 if enabled else 0))

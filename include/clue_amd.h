@@ -256,9 +256,13 @@ typedef struct {
   int32_t persistent;     /* 0: one wave per work item, dispatched by the hardware; k > 0: k
                              persistent waves per CU pull (event, tile) work items from per-XCD
                              device queues (density and the block nearest-higher scan) */
-  int32_t reserved[3];
+  int32_t team;           /* 1: teams of waves per work item in the launches small enough for it, which
+                             group their queries and scan whole tiles whatever the fields above
+                             say; 0: one wave per work item in every launch */
+  int32_t reserved[2];
 } clue_tuning;
-/* Fixes the tuning of the context's later runs and plans; NULL returns to the table. */
+/* Fixes the tuning of the context's later runs and plans; NULL returns to the table.
+ * What clue_get_tuning gave for a batch keeps that batch's launch as it is. */
 clue_status clue_set_tuning(clue_ctx* ctx, const clue_tuning* tuning);
 /* The tuning a run of this batch would use (sizes: host, NULL = one event of n). */
 clue_status clue_get_tuning(clue_ctx* ctx, const clue_params* params, int32_t n,

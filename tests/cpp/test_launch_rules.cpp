@@ -1,6 +1,7 @@
 // The rules by which the host sizes and shapes a launch, on the CPU (built with g++
 // under the address and undefined-behaviour sanitizers).
 #include <cstdio>
+#include <cstring>
 #include <vector>
 
 #include "clue_host.h"
@@ -71,8 +72,27 @@ static void test_team_rule() {
   CHECK(!team(2, 0, 16, 3000) && !team(2, 0, 1, 40000) && !team(2, 0, 1000, 50));
 }
 
+// The tuning a batch is given, fixed, gives the same launch.
+static void test_chosen_tuning_keeps_the_launch() {
+  for (int D = 1; D <= 10; ++D)
+    for (uint32_t n : {1u, 300u, 5003u, 50000u, 110000u, 131072u, 1u << 20})
+      for (int count : {1, 2, 50})
+        for (int ppt : {0, 1, 16}) {
+          if (int64_t(n) * count > (1 << 21)) continue;
+          std::vector<uint32_t> sizes(static_cast<size_t>(count), n);
+          BatchPlan a, b;
+          std::string err;
+          CHECK(plan_batch(D, ppt, sizes.data(), count, nullptr, &a, &err) == CLUE_OK);
+          const clue_tuning t = a.tuning;
+          CHECK(plan_batch(D, ppt, sizes.data(), count, &t, &b, &err) == CLUE_OK);
+          CHECK(a.team == (t.team != 0) && b.team == a.team);
+          CHECK(std::memcmp(&b.tuning, &t, sizeof(t)) == 0);
+        }
+}
+
 int main() {
   test_team_rule();
+  test_chosen_tuning_keeps_the_launch();
   test_sort_histogram();
   std::printf("%d passed, %d failed\n", g_pass, g_fail);
   return g_fail == 0 ? 0 : 1;

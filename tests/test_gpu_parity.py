@@ -585,3 +585,23 @@ def test_large_event_among_small_ones(gpu_ctx, oracle_mod, small, count, dtype):
     k = algo.make_clusters_batched(pts, sizes, None, kern, event_of_cluster=eoc)
     event = np.repeat(np.arange(count + 1), sizes)
     np.testing.assert_array_equal(eoc.to_host()[:k], event[np.nonzero(ref.is_seed)[0]])
+
+
+@pytest.mark.parametrize("sizes", [[3000], [300, 0, 2000], [131072], [16] * 3000])
+def test_fixing_the_chosen_tuning_keeps_it(gpu_ctx, oracle_mod, sizes):
+    """get_tuning reports what a run would use, teams of waves among it, and fixing that
+    changes nothing."""
+    rng = np.random.default_rng(3)
+    n = int(sum(sizes))
+    case = Case(rng.uniform(0, 40, (2, n)), rng.uniform(0.5, 1.5, n), 1.0, 3.0, 1.5, sizes=sizes,
+                name=f"tuning of {len(sizes)} events")
+    params = case.clusterer(gpu_ctx).params(2)
+    chosen = gpu_ctx.get_tuning(params, sizes)
+    assert chosen["team"] == (n <= 49152 and len(sizes) < 3000)
+    gpu_ctx.set_tuning(**chosen)
+    try:
+        assert gpu_ctx.get_tuning(params, sizes) == chosen
+        _check(case, gpu_ctx, oracle_mod)
+    finally:
+        gpu_ctx.set_tuning()
+    assert gpu_ctx.get_tuning(params, sizes) == chosen
