@@ -1613,21 +1613,15 @@ __device__ __forceinline__ uint64_t read_lane(uint64_t v, int i) {
 // at a time, one per lane, so that their offsets and boxes arrive together.
 // ---------------------------------------------------------------------------
 template <int D>
-struct BoxUnion {
-  int lo[D], ext[D];
-  int tiles;  // 0: no active lane
-};
-template <int D>
 __device__ __forceinline__ BoxUnion<D> box_union(const int (&lo)[D], const int (&hi)[D]) {
   BoxUnion<D> u;
-  u.tiles = 1;
 #pragma unroll
   for (int d = 0; d < D; ++d) {
     u.lo[d] = wave_min_uniform(lo[d]);
     const int h = wave_max_uniform(hi[d]);
-    u.ext[d] = h - u.lo[d] + 1;
-    u.tiles = u.lo[d] > h ? 0 : u.tiles * u.ext[d];
+    u.ext[d] = u.lo[d] > h ? 0 : h - u.lo[d] + 1;
   }
+  first_tile_run(u);
   return u;
 }
 
@@ -1915,9 +1909,10 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
           each(std::false_type{});
       }
     };
-    const BoxUnion<D> u = box_union(lo, hi);
+    const BoxUnion<D> boxes = box_union(lo, hi);
     auto run = [&](auto mode_c) {
-      for (int base = 0; base < u.tiles; base += kWave) {
+      BoxUnion<D> u = boxes;
+      do for (int base = 0; base < u.tiles; base += kWave) {
         TileGroup<D> g;
         list_tiles(u, base, ev.nper, rp.wrapped, ev.t_base, toff, &g);
         uint64_t held = ballot(tile_in_reach<D, M>(g, qb, tbox, rp, thr_in));
@@ -1932,7 +1927,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_density(
                             : (in ? thr_in : T(-1));
           walk_tile(j0, j1, thr, mode_c);
         }
-      }
+      } while (next_tile_run(u));
     };
     // Both decisions are made once, outside the candidate loop:
     //  - in range: launch-wide, every exp argument within the radius is in range;
@@ -2165,8 +2160,8 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_nearest_higher(
   const bool cull = rp.cull != 0;
   const QueryBox<D, T> qb = query_box<D, M>(xi, si, active);
   const uint64_t kmin = wave_min_key_bound(key_i);
-  const BoxUnion<D> u = box_union(lo, hi);
-  for (int base = 0; base < u.tiles; base += kWave) {
+  BoxUnion<D> u = box_union(lo, hi);
+  do for (int base = 0; base < u.tiles; base += kWave) {
     TileGroup<D> g;
     list_tiles(u, base, ev.nper, rp.wrapped, ev.t_base, toff, &g);
     uint64_t held = ballot(g.j0 < g.j1);
@@ -2228,7 +2223,7 @@ __global__ __launch_bounds__(kMaxNeighbourBlock) void k_nearest_higher(
           accept(metric_value<D, M>(xi, si, sx, cs, k, ssig, rp), skey[k], key_in, k);
       }
     }
-  }
+  } while (next_tile_run(u));
   if (active) {
     snh[s] = nh;
     sdelta[s] = delta;

@@ -406,9 +406,9 @@ __global__ __launch_bounds__(kTeam * kWave) void k_density_team(
     return !(cull && out_of_reach<D, M>(qb, x, s, rp, thr_in));
   };
 
-  const BoxUnion<D> u = box_union(lo, hi);
+  BoxUnion<D> u = box_union(lo, hi);
   int turn = 0;  // chunks of the lists before the current one
-  for (int base = 0; base < u.tiles; base += kWave) {
+  do for (int base = 0; base < u.tiles; base += kWave) {
     TeamGroup<D> g;
     list_tiles(u, base, ev.nper, rp.wrapped, ev.t_base, toff, &g);
     g.number(tile_in_reach<D, M>(g, qb, tbox, rp, thr_in));
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(kTeam * kWave) void k_density_team(
       n = 0;
       __syncthreads();  // the list is free again
     }
-  }
+  } while (next_tile_run(u));
   if (wave != 0) return;
   const T rho = relay_take(relay, turn);
   if (me.active) {
@@ -614,13 +614,13 @@ __global__ __launch_bounds__(kTeam * kWave) void k_nearest_higher_team(
     g.in = in_own ? 1ull : 0ull;
     search(g);
   }
-  const BoxUnion<D> u = box_union(lo, hi);
-  for (int base = 0; base < u.tiles; base += kWave) {
+  BoxUnion<D> u = box_union(lo, hi);
+  do for (int base = 0; base < u.tiles; base += kWave) {
     list_tiles(u, base, ev.nper, rp.wrapped, ev.t_base, toff, &g);
     g.number(!(own_first && g.t == own) && tile_in_reach<D, M>(g, qb, tbox, rp, bmax));
     g.boxes(lo, hi);
     search(g);
-  }
+  } while (next_tile_run(u));
 
   if (wave != 0) {
     best_delta[wave][lane] = me.delta;

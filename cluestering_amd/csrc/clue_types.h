@@ -50,6 +50,67 @@ inline int64_t radix_hist_elems(int64_t blocks, int digit_bits) {
   return (blocks + 1) << digit_bits;
 }
 
+// The union of a wave's search boxes, in tiles: from lo on, ext of them per dimension. On
+// wrapped dimensions it can span almost twice the tiles there are, 2^D times as many
+// together. A launch has fewer than 2^26 tiles (2^32 threads at one wave each), so
+// from six dimensions on that can be more than 32 bits count. Such a union is visited in
+// runs, one per step of dimension 0 (in ten dimensions of 0 and 1), in the reference's
+// order; any other is one run. (constexpr: host and device. Up to five dimensions there
+// is nothing to keep between runs: the density stage has no scalar registers to spare
+// there, 2^20 points in 2-D took 690 us without and 704 with them.)
+constexpr int64_t kTileRunMax = INT32_MAX - 64;  // a wave counts a run's tiles by 64
+template <int D>
+struct BoxUnion {
+  static constexpr int kOuter = D < 6 ? 0 : D < 10 ? 1 : 2;
+  int lo[D], ext[D];
+  int tiles;                          // of a run; 0: no active lane
+  int last[kOuter > 0 ? kOuter : 1];  // lo of the outer dimensions in the last run
+  int first1;                         // lo[1] in the first run (two outer dimensions)
+};
+// tiles and the first run of the union given by lo and ext.
+template <int D>
+constexpr void first_tile_run(BoxUnion<D>& u, int64_t most = kTileRunMax) {
+  constexpr int K = BoxUnion<D>::kOuter;
+  if constexpr (K == 0) {
+    u.tiles = 1;
+    for (int d = 0; d < D; ++d) u.tiles *= u.ext[d];
+  } else {
+    int64_t inner = 1;
+    for (int d = D - 1; d >= K; --d) inner *= u.ext[d];
+    int64_t all = inner;
+    for (int d = 0; d < K; ++d) {
+      all *= u.ext[d];
+      u.last[d] = u.lo[d];
+    }
+    u.first1 = u.lo[K - 1];
+    if (all > most) {
+      for (int d = 0; d < K; ++d) {
+        u.last[d] += u.ext[d] - 1;
+        u.ext[d] = 1;
+      }
+      all = inner;
+    }
+    u.tiles = static_cast<int>(all);
+  }
+}
+// Goes on to the next run; false after the last.
+template <int D>
+constexpr bool next_tile_run(BoxUnion<D>& u) {
+  constexpr int K = BoxUnion<D>::kOuter;
+  if constexpr (K == 0) {
+    return false;
+  } else {
+    if (K == 2 && u.lo[K - 1] != u.last[K - 1]) {
+      ++u.lo[K - 1];
+      return true;
+    }
+    if (u.lo[0] == u.last[0]) return false;
+    ++u.lo[0];
+    if (K == 2) u.lo[K - 1] = u.first1;
+    return true;
+  }
+}
+
 // Constants of the float exp (Cody-Waite reduction x = k ln2 + r with a 15-bit
 // ln2_hi, then the degree-6 minimax polynomial of e^r on [-ln2/2, ln2/2] whose
 // constant and linear terms are 1), shared by the device code and the host code

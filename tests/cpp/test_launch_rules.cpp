@@ -90,7 +90,73 @@ static void test_chosen_tuning_keeps_the_launch() {
         }
 }
 
+// Every tile of a union once, dimension 0 outermost, in one run or (a small limit) several.
+template <int D>
+static void check_tile_order(const int (&first)[D], const int (&extents)[D], int64_t most) {
+  clue_dev::BoxUnion<D> u{};
+  int want[D] = {};
+  int64_t count = 0, all = 1;
+  for (int d = 0; d < D; ++d) {
+    u.lo[d] = first[d];
+    u.ext[d] = extents[d];
+    all *= extents[d];
+  }
+  bool same = true, more = true;
+  clue_dev::first_tile_run(u, most);
+  do {
+    for (int idx = 0; idx < u.tiles; ++idx, ++count) {
+      int q = idx;
+      same = same && more;
+      for (int d = D - 1; d >= 0; --d) {
+        same = same && u.lo[d] + (d == 0 ? q : q % u.ext[d]) == first[d] + want[d];
+        q /= u.ext[d];
+      }
+      int d = D - 1;
+      for (; d >= 0 && ++want[d] == extents[d]; --d) want[d] = 0;
+      more = d >= 0;
+    }
+  } while (clue_dev::next_tile_run(u));
+  CHECK(same && count == all);
+}
+
+// The widest union of nper tiles per dimension in D, all wrapped: counted in full.
+template <int D>
+static void check_widest(int nper, int64_t tiles) {
+  clue_dev::BoxUnion<D> u{};
+  for (int d = 0; d < D; ++d) u.ext[d] = 2 * nper - 1;
+  clue_dev::first_tile_run(u);
+  int64_t count = 0;
+  bool fits = true;
+  do {
+    fits = fits && u.tiles > 0 && u.tiles <= clue_dev::kTileRunMax;
+    count += u.tiles;
+  } while (clue_dev::next_tile_run(u));
+  CHECK(fits && count == tiles);
+}
+
+static void test_tile_runs() {
+  for (int64_t most : {int64_t(1), int64_t(5), int64_t(300), clue_dev::kTileRunMax}) {
+    check_tile_order<1>({4}, {7}, most);
+    check_tile_order<3>({1, 2, 3}, {5, 1, 6}, most);
+    check_tile_order<6>({1, 2, 3, 4, 5, 6}, {3, 1, 2, 4, 2, 3}, most);
+    check_tile_order<9>({0, 0, 1, 0, 0, 2, 0, 0, 3}, {2, 3, 1, 2, 2, 2, 1, 3, 2}, most);
+    check_tile_order<10>({5, 6, 0, 0, 0, 0, 0, 0, 0, 7}, {2, 3, 1, 2, 2, 2, 1, 3, 2, 2}, most);
+  }
+  // The most tiles per dimension of fewer than 2^26: 8191^2 up to 6^10.
+  check_widest<2>(8191, 268337161);
+  check_widest<5>(36, 1804229351);
+  check_widest<6>(20, 3518743761);
+  check_widest<7>(13, 6103515625);
+  check_widest<8>(9, 6975757441);
+  check_widest<9>(7, 10604499373);
+  check_widest<10>(6, 25937424601);
+  clue_dev::BoxUnion<10> none{};  // no active lane
+  clue_dev::first_tile_run(none);
+  CHECK(none.tiles == 0 && !clue_dev::next_tile_run(none));
+}
+
 int main() {
+  test_tile_runs();
   test_team_rule();
   test_chosen_tuning_keeps_the_launch();
   test_sort_histogram();
