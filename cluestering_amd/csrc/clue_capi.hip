@@ -154,6 +154,9 @@ clue_status run_batch(clue_ctx* ctx, const P* p, const Pts* pts, const uint32_t*
   if (st) return st;
   BatchBuffersT<T> bb;
   ResultArraysT<T> ra;
+  // From here on copies may read the host descriptors and the stage, also if the call
+  // ends with an error (the launch reports errors that earlier calls have left, too).
+  ctx->pending = true;
   st = prepare_batch(ctx->ws, bp, p, pts, res, &ctx->stage, ctx->stream, &bb, &ra);
   if (st) return st;
   ra.event_of_cluster = event_of_cluster;
@@ -167,7 +170,6 @@ clue_status run_batch(clue_ctx* ctx, const P* p, const Pts* pts, const uint32_t*
   launch_pipeline(rp, point_arrays(p, pts), bb, ra, ctx->stream,
                   ctx->profiling ? &hook : nullptr);
   CLUE_HIP(hipGetLastError());
-  ctx->pending = true;
   ctx->has_run = true;
   ctx->last_n = bp.n_total;
   ctx->last_seeds = bb.seeds;

@@ -81,3 +81,27 @@ def test_negative_metric_weight_out_of_box(gpu_ctx, oracle_mod, tuning, dtype):
     _check(Case(x, [1.0, 2.0, 4.0, 8.0], 0.5, 1.0, 0.5, metric=K.EuclideanMetric([1.0, -0.02]),
                 points_per_tile=1, dtype=dtype, name=f"negative weight {tuning}"), gpu_ctx, oracle_mod,
            tuning)
+
+
+def test_runs_after_an_error(gpu_ctx, oracle_mod):
+    """An error left by another call ends a launch early, with its copies and kernels under
+    way. The calls that follow wait for them before they write the descriptors again."""
+    rng = np.random.default_rng(8)
+    cases = []
+    for sizes in ([700] * 40, [9000, 3, 2500]):
+        n = sum(sizes)
+        cases.append(Case(rng.uniform(0, 30, (2, n)), rng.uniform(0.5, 1.5, n), 1.0, 3.0, 1.5, sizes=sizes,
+                          name=f"after an error, {len(sizes)} events"))
+    refs = [c.run_oracle(oracle_mod) for c in cases]
+    points = [c.points(gpu_ctx) for c in cases]
+    for k in (0, 1, 0, 1):
+        with pytest.raises(Exception):
+            gpu_ctx.empty(1 << 50, np.uint8)
+        try:
+            cases[1 - k].clusterer(gpu_ctx).make_clusters_batched(points[1 - k], cases[1 - k].sizes)
+        except Exception:
+            pass  # the error that was left
+        cases[k].clusterer(gpu_ctx).make_clusters_batched(points[k], cases[k].sizes)
+        out = points[k].results()
+        out["seeds"] = None
+        assert_same(out, refs[k], cases[k].name)
