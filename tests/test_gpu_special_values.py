@@ -105,3 +105,49 @@ def test_runs_after_an_error(gpu_ctx, oracle_mod):
         out = points[k].results()
         out["seeds"] = None
         assert_same(out, refs[k], cases[k].name)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("tuning", TUNINGS)
+@pytest.mark.parametrize("n", [40, 3000])
+def test_flat_sums_with_weights_beyond_numbers(gpu_ctx, n, tuning, dtype):
+    """Flat kernel, unit weights but for one infinite, one NaN and two whose sum overflows:
+    their neighbours' sums are infinite or NaN, every other point's is exact, though
+    the waves that met them take their sums again with selects."""
+    from cluestering_amd.device import Clusterer, PointsDevice
+    rng = np.random.default_rng(78)
+    xy = rng.uniform(0, np.sqrt(n) * 0.7, size=(2, n)).astype(dtype)
+    xy[:, :6] = [[-9.0, -8.5, 90.0, 90.5, 200.0, 200.5], np.zeros(6)]
+    w = np.ones(n, dtype)
+    w[1], w[3] = np.inf, np.nan
+    w[4] = w[5] = np.finfo(dtype).max * 0.75
+    if tuning is not None:
+        gpu_ctx.set_tuning(xcd_chunk_log2=4, block_waves=1, **tuning)
+    try:
+        p = PointsDevice.from_host(gpu_ctx, xy, w, dtype=dtype)
+        Clusterer(gpu_ctx, 1.0, 2.0).make_clusters(p, None, K.FlatKernel(0.5))
+    finally:
+        gpu_ctx.set_tuning()
+    rho = p.rho.to_host()
+    x, y = xy
+    near = np.sqrt((x[:, None] - x[None]) ** 2 + (y[:, None] - y[None]) ** 2) <= 1
+    want = 0.5 * near.sum(1) + 0.5   # the point itself counts 1
+    assert rho[0] == np.inf and rho[1] == np.inf and rho[4] == np.inf and rho[5] == np.inf
+    assert np.isnan(rho[2]) and np.isnan(rho[3])
+    np.testing.assert_array_equal(rho[6:], want[6:].astype(dtype))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("tuning", TUNINGS)
+@pytest.mark.parametrize("metric", [None, K.ManhattanMetric(), K.ChebyshevMetric()])
+def test_flat_sums_at_extreme_radii(gpu_ctx, oracle_mod, metric, tuning, dtype):
+    """Radii whose threshold times a power of two cannot stand for the comparison (too
+    small, too large, infinite), beside ones where it can."""
+    rng = np.random.default_rng(12)
+    n = 500
+    tiny, huge = (1e-10, 1e19) if dtype == np.float32 else (1e-19, 1e37)
+    for dc in (tiny, tiny * 100, huge, huge / 100, np.inf):
+        scale = 1.0 if np.isinf(dc) else dc
+        x = np.round(rng.uniform(0, 4, (2, n)), 1) * scale
+        _check(Case(x, rng.uniform(0.5, 1.5, n), dc, 3.0, dc, metric=metric, points_per_tile=50, dtype=dtype,
+                    name=f"radius {dc} {metric} {tuning}"), gpu_ctx, oracle_mod, tuning)
