@@ -245,7 +245,7 @@ struct WorkspaceShape {
   bool team = false;               // neighbour stages by teams of waves
   bool event_tiles = false;        // the fused per-event tile build (no radix-sort buffers)
   bool group_queries = false;
-  bool separate_dm_order = false;  // dm != dc and the plain nearest-higher scan
+  bool separate_dm_order = false;  // a second query order for dm (no run asks for one)
   bool nh_blocks = false;          // nearest-higher over the Hilbert block layout
   bool flat_kernel = false;
   bool has_sigma = false;
@@ -254,10 +254,9 @@ struct WorkspaceShape {
   bool own_nh = false;
   bool own_is_seed = false;
   bool sorted_boxes = false;       // density leaves out tiles by their bounding boxes
-  bool density_morton = false;     // density takes the Hilbert order of qfine
+  bool density_morton = false;     // density takes the Hilbert order of qfine (every grouped run)
 };
 
-// Bytes of every workspace slot for a batch of this shape (0: unused).
 // Bytes of the tiles' bounding boxes, 0 where the stages do without. Small tables are
 // always worth it; of the large ones those that hold fewer than 16 points per tile are
 // left out: in many dimensions, or with very small tiles, they would take more memory
@@ -268,6 +267,7 @@ inline size_t tile_box_bytes(int64_t n, int64_t tiles, int D, int value_bytes) {
   return bytes <= kTileBoxAlways || 16 * tiles <= n ? static_cast<size_t>(bytes) : 0;
 }
 
+// Bytes of every workspace slot for a batch of this shape (0: unused).
 inline void workspace_requests(const WorkspaceShape& w, size_t (&bytes)[S_NUM]) {
   std::memset(bytes, 0, sizeof(bytes));
   const int64_t n = w.n, NT = w.tiles;

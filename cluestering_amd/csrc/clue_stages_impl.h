@@ -107,9 +107,6 @@ struct MetricTraits {
 };
 
 // ---------------------------------------------------------------------------
-// Utility kernels.
-// ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
 // (a1) Per-event coordinate extremes (ComputeTiles.hpp:17-36). NaN coordinates
 // are skipped, as the reference's std::max/std::min fold skips them.
 // ---------------------------------------------------------------------------
@@ -3020,9 +3017,8 @@ static void launch_nh_blocks_dm(const NeighbourLaunch<T>& L) {
   go(k_nh_blocks<D, M, false, T>, L.grid);
 }
 
-// Nearest-higher over the block layout: the layout pass, then the scan. Its
-// waves take each tile's points in Hilbert order (qfine): the scan visits only the
-// blocks its lanes want, so grouping lanes by search-box class buys nothing here.
+// Nearest-higher over the block layout, which the query order and the density stage
+// have written.
 template <int D, class T>
 static void launch_nh_blocks_d(const NeighbourLaunch<T>& L) {
   switch (L.rp->metric) {

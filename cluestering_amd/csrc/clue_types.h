@@ -193,7 +193,7 @@ struct RunParamsT {
   T dm_sq_max;           // same for dm
   T seed_sq_max;         // same for seed_dc
   T in_scale;            // 2^k and 2^k times the value after the density radius' threshold, for
-  T in_limit;            // the flat kernel's sums (0: not representable)
+  T in_limit;            // the flat kernel's sums (0: selects instead)
   T kp0, kp1;            // kernel parameters (flat f | exp lambda, A | gauss sigma, A)
   T gauss_den;           // (2 * sigma) * sigma, as the reference evaluates it
   T gauss_inv_den;       // 1 / gauss_den when gauss_den is a power of two
